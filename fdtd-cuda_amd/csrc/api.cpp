@@ -1823,16 +1823,11 @@ int fdtd_get_slice(fdtd_sim *s, int comp, int axis, int index, float *out) {
         return FDTD_OK;
     }
     const float *f = comp < 3 ? s->E[s->p][comp] : s->H[s->p][comp - 3];
-    const size_t fl = sizeof(float);
+    // gathered on the device into the staging buffer, then one contiguous copy
+    const size_t plane = (size_t)n[axis == 0 ? 1 : 0] * n[axis == 2 ? 1 : 2] * sizeof(float);
+    HIPCHK(s, launch_slice(f, g, axis, index, s->dense, s->stream));
     HIPCHK(s, hipStreamSynchronize(s->stream));
-    if (axis == 0)   // rows j of NZ values, pitch sz
-        HIPCHK(s, hipMemcpy2D(out, g.NZ * fl, f + (size_t)index * g.sxy, g.sz * fl, g.NZ * fl, g.NY, hipMemcpyDeviceToHost));
-    else if (axis == 1)   // rows i of NZ values, pitch sxy
-        HIPCHK(s, hipMemcpy2D(out, g.NZ * fl, f + (size_t)index * g.sz, g.sxy * fl, g.NZ * fl, g.NX, hipMemcpyDeviceToHost));
-    else   // per i, NY single values with pitch sz
-        for (int i = 0; i < g.NX; i++)
-            HIPCHK(s, hipMemcpy2D(out + (size_t)i * g.NY, fl, f + (size_t)i * g.sxy + index, g.sz * fl, fl, g.NY,
-                                  hipMemcpyDeviceToHost));
+    HIPCHK(s, hipMemcpy(out, s->dense, plane, hipMemcpyDeviceToHost));
     return FDTD_OK;
 }
 

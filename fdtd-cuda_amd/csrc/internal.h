@@ -278,6 +278,8 @@ hipError_t launch_dft_mfma(const float *X, const void *Wf, double *acc, long mto
 hipError_t launch_flux_reduce(const double *acc, const FaceDev &fd, long mtot, long mE_pad, int F, double dA,
                               double *out, hipStream_t st);
 hipError_t launch_pack_field(const float *f, const Geom &g, float *dense, int to_dense, hipStream_t st);
+// The plane `index` along `axis` of a field into out, packed as fdtd_get_slice returns it.
+hipError_t launch_slice(const float *f, const Geom &g, int axis, int index, float *out, hipStream_t st);
 hipError_t launch_disp_sync_state(const DispDev &d, int from_field, hipStream_t st);
 // Hydrodynamic model: velocity update, then per component (x, y, z) continuity and E update.
 hipError_t launch_hydro(const DispDev &d, hipStream_t st);
