@@ -386,7 +386,8 @@ int plan_rows(fdtd_sim *s) {
     if (const char *v = std::getenv("FDTD_CCHUNK")) s->cchunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_SCHUNK")) s->schunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_XCD")) s->xcd = std::atoi(v) != 0;
-    if ((double)s->fsz * 4.0 >= 4294967296.0) return FDTD_OK;
+    // 32-bit byte offsets, the last word left for the lanes whose access is dropped
+    if ((double)s->fsz * 4.0 >= 4294967292.0 || (double)s->npsi * 4.0 >= 4294967292.0) return FDTD_OK;
     std::vector<uint32_t> img(kRowsAuxWords, 0u);
     auto put = [&](int q, float v) { std::memcpy(&img[q], &v, 4); };
     for (int a = 0; a < 3; a++) {
@@ -512,6 +513,14 @@ RowsArgs make_rows(fdtd_sim *s) {
     for (int c = 0; c < 3; c++) {
         r.Ein[c] = (const char *)(s->E[q][c] - fb); r.Hin[c] = (const char *)(s->H[q][c] - fb);
         r.Eout[c] = (char *)(s->E[1 - q][c] - fb); r.Hout[c] = (char *)(s->H[1 - q][c] - fb);
+    }
+    r.fbytes = (unsigned)(s->fsz * 4);
+    r.psi = (const char *)s->psi;
+    r.psi_bytes = (unsigned)(s->npsi * 4);
+    for (int a = 0; a < 6; a++) {
+        r.hin[a] = (unsigned)((s->psiH[s->pp][a] - s->psi) * 4);
+        r.hout[a] = (unsigned)((s->psiH[1 - s->pp][a] - s->psi) * 4);
+        r.eio[a] = (unsigned)((s->psiE[a] - s->psi) * 4);
     }
     r.aux = s->aux_d;
     r.Chh = (float)S.Chh; r.Che = (float)S.Che; r.Cee = (float)S.Cee; r.Ceh = (float)S.Ceh;
@@ -817,11 +826,17 @@ int fdtd_create(const fdtd_params *p, fdtd_sim **out) {
     const size_t hsz[6] = {hz_, hy_, hz_, hx_, hx_, hy_};
     const size_t esz[6] = {ez_, ey_, ez_, ex_, ey_, ex_};
     for (int a = 0; a < 6; a++) { s->hsz[a] = hsz[a]; s->esz[a] = esz[a]; }
+    // one allocation, so the row-blocked kernel reaches every array from one base
+    auto pad64 = [](size_t n) { return (n + 63) / 64 * 64; };
+    size_t npsi = 0;
+    for (int a = 0; a < 6; a++) npsi += 2 * pad64(hsz[a]) + pad64(esz[a]);
+    if ((rc = dalloc(s, &s->psi, npsi))) return fail(rc);
+    s->npsi = npsi;
+    npsi = 0;
+    auto take = [&](size_t n) { float *p = s->psi + npsi; npsi += pad64(n); return p; };
     for (int q = 0; q < 2; q++)
-        for (int a = 0; a < 6; a++)
-            if ((rc = dalloc(s, &s->psiH[q][a], hsz[a]))) return fail(rc);
-    for (int a = 0; a < 6; a++)
-        if ((rc = dalloc(s, &s->psiE[a], esz[a]))) return fail(rc);
+        for (int a = 0; a < 6; a++) s->psiH[q][a] = take(hsz[a]);
+    for (int a = 0; a < 6; a++) s->psiE[a] = take(esz[a]);
     // CPML tables: 1/(kappa d), recursion b and c/d, near slab then far slab
     for (int a = 0; a < 3; a++) {
         const fdtd::CpmlAxis &c = S.cp[a];

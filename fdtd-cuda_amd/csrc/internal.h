@@ -213,6 +213,11 @@ struct Pieces {
 struct RowsArgs {
     const char *Ein[3], *Hin[3];
     char *Eout[3], *Hout[3];
+    unsigned fbytes;                    // bytes of a field allocation
+    // forward psi: one allocation, byte offsets of the six psi_H arrays read
+    // and written by this step and of the psi_E arrays (updated in place)
+    const char *psi;
+    unsigned psi_bytes, hin[6], hout[6], eio[6];
     const unsigned *aux;
     float Chh, Che, Cee, Ceh;
     float ik0[2][2];
@@ -227,8 +232,10 @@ struct RowsArgs {
     int box[4][4];
     int nseg;
     int start[5];
+    int waves;                          // waves of a z column (rows_waves(NZ)), filled in by the launcher
     int tiles;                          // row tiles per block: 1, or 2-3 for the clean variant when tiles * W <= 16
 };
+constexpr int kRowsMaxWaves = 16;       // waves of a block: tiles * waves
 // Words of the table image and its layout (see kernels.hip).
 constexpr int kRowsAuxWords = 1548 + 48;
 constexpr int kRowsAuxAxis = 512, kRowsAuxMaxEdge = 64, kRowsAuxMaxLayers = 64;

@@ -639,6 +639,22 @@ __global__ __launch_bounds__(64 * TJ) void k_fused_step(StepDev s, int ichunk, i
     fused_body<TJ>(s, ichunk, nkt, pc, xcd_order(blockIdx.x, pc.start[pc.n]));
 }
 
+// ----------------------------------------------------------------- arguments in constant memory
+
+// Items are read through the constant address space: every block reads its
+// item at a uniform address, so the fields land in scalar registers exactly
+// as kernel arguments do.
+#define CONST_AS __attribute__((address_space(4)))
+template <typename T>
+__device__ __forceinline__ const T &batch_item(const T *items, unsigned idx) {
+    const CONST_AS T *c = (const CONST_AS T *)items;
+    return *(const T *)(c + idx);
+}
+__device__ __forceinline__ unsigned batch_map(const unsigned *map) {
+    const CONST_AS unsigned *c = (const CONST_AS unsigned *)map;
+    return c[blockIdx.x];
+}
+
 // ----------------------------------------------------------------- row-blocked step kernel
 
 __device__ inline float ldb(const char *b, unsigned o) { return *(const float *)(b + o); }
@@ -666,11 +682,31 @@ __device__ inline void lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Lambdas of the large kernels: inlined whatever the size of the caller (the
+// compiler stops inlining into a function of some thousand basic blocks, and
+// the register sets they work on would then live in scratch memory).
+#define INLINE_LAMBDA __attribute__((always_inline))
+
+// Raw buffer accesses: address = base + voffset (per lane) + soffset (scalar).
+// A lane whose voffset is kOob reads 0 and its store is dropped by the
+// hardware's range check, so accesses that only some lanes make need no branch
+// and the compiler's wait counts stay exact across them.  Behind a branch a
+// store counts as perhaps not issued, and a wait for loads issued before it
+// becomes a wait for the store's completion too: in the march of the
+// row-blocked kernel that put the completion of one plane's stores in front of
+// the next plane's arithmetic (clean box of a 281^3 grid alone 223 -> 215 us,
+// of a 121^3 grid and smaller a third less per plane).
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+constexpr unsigned kOob = 0xFFFFFFFCu;
+__device__ __forceinline__ rsrc_t make_rsrc(const void *base, unsigned bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
+}
+__device__ __forceinline__ float bld(rsrc_t r, unsigned voff, unsigned soff) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+}
 template <bool NT>
-__device__ inline void stn(char *b, unsigned o, float v) {
-    float *p = (float *)(b + o);
-    if (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
+__device__ __forceinline__ void bst(rsrc_t r, unsigned voff, unsigned soff, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)voff, (int)soff, NT ? 2 : 0);
 }
 
 // One full leapfrog step of the whole grid (TFSF excluded: k_tfsf_fix adds
@@ -712,7 +748,9 @@ __device__ inline void stn(char *b, unsigned o, float v) {
 // inside the clean box).
 //
 // The body takes the block's index within its simulation's cell set (L), so
-// batched launches run it over many simulations.
+// batched launches run it over many simulations.  The waves per column W and
+// the tiles T are launch arguments: they enter once per block, and one
+// instance serves every grid height.
 //
 // T row tiles per block: waves T*W; tile wg / W takes row tile jt = T*jb + tile
 // and the tiles march the same x chunk in step (one barrier per x step for
@@ -720,22 +758,28 @@ __device__ inline void stn(char *b, unsigned o, float v) {
 // ceil(waves / 4) free wave slots, so at four waves per SIMD a 5-wave block
 // holds two per CU (10 waves) while one 15-wave block (T = 3) holds 15.
 // Tiles past the last row tile of the box repeat its loads and store nothing.
-template <int W, int R, bool XG, bool YG, bool ADJ, int T = 1>
-__device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
-    static_assert(ADJ || !XG || !YG, "corner columns of the forward step run on the general kernel");
+// LDS of one block.
+template <int R, bool ADJ>
+struct RowsLds {
+    static constexpr int kTab = kAuxPsi + (ADJ ? 48 : 0);
+    float sK[2][2][kRowsMaxWaves][R + 1];   // last lane's hy, hx per wave and row (H at k-1 of the next wave)
+    float sE[2][2][kRowsMaxWaves][R + 1];   // first lane's ex, ey per wave and row (E at k+1 of the previous wave)
+    __align__(16) unsigned sT[kTab];
+};
+
+// Block L of the box x in [ia, ib), y in [ja, jbox): row-tile groups fastest, then z segments, then x chunks.
+template <int R, bool XG, bool YG, bool ADJ, bool ZS>
+__device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, int ja, int jbox, int ichunk, int L,
+                                           RowsLds<R, ADJ> &lds) {
     constexpr bool AS = ADJ && (XG || YG);   // adjoint on a side slab or corner column
-    static_assert(T >= 1 && W * T <= 16, "at most 16 waves per block");
-    __shared__ float sK[2][2][W * T][R + 1];   // last lane's hy, hx per wave and row (H at k-1 of the next wave)
-    __shared__ float sE[2][2][W * T][R + 1];   // first lane's ex, ey per wave and row (E at k+1 of the previous wave)
-    constexpr int kTab = kAuxPsi + (ADJ ? 48 : 36);
-    __shared__ __align__(16) unsigned sT[kTab];
+    const int W = ra.waves, T = ra.tiles;    // waves of a z column, row tiles of the block
+    auto &sK = lds.sK;
+    auto &sE = lds.sE;
+    auto &sT = lds.sT;
+    constexpr int kTab = RowsLds<R, ADJ>::kTab;
     const int NX = ra.NX, NY = ra.NY, NZ = ra.NZ;
     for (int q = threadIdx.y * 64 + threadIdx.x; q < kTab; q += 64 * W * T) sT[q] = ra.aux[q];
     const float *sTf = (const float *)sT;
-    int pc = 0;
-    while (pc + 1 < ra.npiece && L >= ra.start[pc + 1]) pc++;
-    L -= ra.start[pc];
-    const int ia = ra.box[pc][0], ib = ra.box[pc][1], ja = ra.box[pc][2], jbox = ra.box[pc][3];
     const int njt = (jbox - ja + R - 1) / R;
     const int njb = (njt + T - 1) / T;
     const int jtb = L % njb;
@@ -744,27 +788,27 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     const int ch = L / ra.nseg;
     // the wave index is uniform across a wave (blocks are 64 wide): keep it,
     // and the row tile and row offsets derived from it, in scalar registers
-    const int lane = threadIdx.x, wg = __builtin_amdgcn_readfirstlane((int)threadIdx.y), w = T == 1 ? wg : wg % W;
+    const int lane = threadIdx.x, wg = __builtin_amdgcn_readfirstlane((int)threadIdx.y), w = wg % W;
     const int t = w * 64 + lane;
-    const int jt0 = T == 1 ? jtb : jtb * T + wg / W;
+    const int jt0 = jtb * T + wg / W;
     const bool live = jt0 < njt;
     const int jt = live ? jt0 : njt - 1;
     const int k = seg * (64 * W - 2) - 1 + t;
     const int kc = min(k, NZ - 1);
     const bool kown = live && t > 0 && t < 64 * W - 1 && k < NZ;
-    const int i0 = ia + ch * ra.ichunk, i1 = min(i0 + ra.ichunk, ib);
+    const int i0 = ia + ch * ichunk, i1 = min(i0 + ichunk, ib);
     const int pp = ra.pp;
-    auto hlay = [&](int a, int x) { return x < ra.Nc[a] ? x : (x >= ra.F[a] ? ra.Nc[a] + x - ra.F[a] : -1); };
-    auto elay = [&](int a, int x) { return x <= ra.Nc[a] ? x : (x >= ra.F[a] ? ra.Nc[a] + 1 + x - ra.F[a] : -1); };
+    auto hlay = [&](int a, int x) INLINE_LAMBDA { return x < ra.Nc[a] ? x : (x >= ra.F[a] ? ra.Nc[a] + x - ra.F[a] : -1); };
+    auto elay = [&](int a, int x) INLINE_LAMBDA { return x <= ra.Nc[a] ? x : (x >= ra.F[a] ? ra.Nc[a] + 1 + x - ra.F[a] : -1); };
     // 1/(kappa d) of axis a (length n) at x, E positions if e
-    auto ik = [&](int a, bool e, int x, int n) {
+    auto ik = [&](int a, bool e, int x, int n) INLINE_LAMBDA {
         const int ew = (int)sT[kAuxEw + a];
         const int base = a * kAuxAxis + (e ? 0 : 128);
         const int q = x < ew ? base + x : (x >= n - ew ? base + 64 + x - (n - ew) : (e ? kAuxIkE0 : kAuxIkH0) + a);
         return sTf[q];
     };
-    auto coef = [&](int a, int which, int layer) { return sTf[a * kAuxAxis + 256 + which * 64 + layer]; };
-    auto psi = [&](int idx) { return *(gfloat *const *)&sT[kAuxPsi + 2 * idx]; };   // 0-5 set 0, 6-11 set 1, 12-17 psi_E
+    auto coef = [&](int a, int which, int layer) INLINE_LAMBDA { return sTf[a * kAuxAxis + 256 + which * 64 + layer]; };
+    auto psi = [&](int idx) INLINE_LAMBDA { return *(gfloat *const *)&sT[kAuxPsi + 2 * idx]; };   // 0-5 set 0, 6-11 set 1, 12-17 psi_E
     // adjoint: psi_E read from set pe (12 + 6 pe), written to the other
     const int ein = ADJ ? 12 + 6 * ra.pe : 12, eout = ADJ ? 18 - 6 * ra.pe : 12;
     const int hout = (1 - pp) * 6;
@@ -774,7 +818,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     const bool kA = k >= 0 && k < NZ - 1, kB = k >= 0 && k < NZ, kC = k > 0 && k < NZ - 1;
     const int kq = max(kc, 0);
     const int lzh = kA ? hlay(2, k) : -1, lze = kC ? elay(2, k) : -1;
-    const bool zh = __ballot(lzh >= 0) != 0, ze = __ballot(lze >= 0) != 0;
+    const bool zh = ZS && (!ADJ || __ballot(lzh >= 0) != 0), ze = ZS && (!ADJ || __ballot(lze >= 0) != 0);
     const float ikz_h = ik(2, false, kq, NZ), ikz_e = ik(2, true, kq, NZ);
     const float bzh = lzh >= 0 ? coef(2, 2, lzh) : 0.f, czh = lzh >= 0 ? coef(2, 3, lzh) : 0.f;
     const float bze = lze >= 0 ? coef(2, 0, lze) : 0.f, cze = lze >= 0 ? coef(2, 1, lze) : 0.f;
@@ -786,25 +830,35 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     unsigned ro[R + 2];
 #pragma unroll
     for (int r = 0; r < R + 2; r++) ro[r] = (unsigned)(min(jb + r, NY) + 1) * sz4 + (unsigned)(kc + 1) * 4u;
-    auto jA = [&](int r) { return !YG || (jb + r >= 0 && jb + r < NY - 1); };
-    auto jB = [&](int r) { return !YG || (jb + r >= 0 && jb + r < NY); };
-    auto jC = [&](int r) { return !YG || (jb + r > 0 && jb + r < NY - 1); };
-    auto jq = [&](int r) { return min(max(jb + r, 0), NY - 1); };
-    auto lyh = [&](int r) { return YG && jA(r) ? hlay(1, jb + r) : -1; };
-    auto lye = [&](int r) { return YG && jC(r) ? elay(1, jb + r) : -1; };
-    auto lxh = [&](int ip) { return XG && ip < NX - 1 ? hlay(0, ip) : -1; };
-    auto lxe = [&](int ip) { return XG && ip > 0 && ip < NX - 1 ? elay(0, ip) : -1; };
+    // field stores: rows 1..R of the lanes that own their cell
+    const unsigned fb = ra.fbytes;
+    const rsrc_t sEx = make_rsrc(ra.Eout[0], fb), sEy = make_rsrc(ra.Eout[1], fb), sEz = make_rsrc(ra.Eout[2], fb);
+    const rsrc_t sHx = make_rsrc(ra.Hout[0], fb), sHy = make_rsrc(ra.Hout[1], fb), sHz = make_rsrc(ra.Hout[2], fb);
+    unsigned so[R + 1];
+#pragma unroll
+    for (int r = 1; r <= R; r++) so[r] = kown && jb + r < jbox ? ro[r] : kOob;
+    // psi accesses of the forward step: lane part of the offset (the plane, row and layer are scalar)
+    const rsrc_t rp = make_rsrc(ra.psi, ra.psi_bytes);
+    const unsigned vzh = lzh >= 0 ? (unsigned)lzh * 4u : kOob, vze = lze >= 0 ? (unsigned)lze * 4u : kOob;
+    const unsigned vzhs = kown ? vzh : kOob, vzes = kown ? vze : kOob;
+    const unsigned vk = (unsigned)kq * 4u, vkA = kown && kA ? vk : kOob, vkC = kown && kC ? vk : kOob;
+    auto jA = [&](int r) INLINE_LAMBDA { return !YG || (jb + r >= 0 && jb + r < NY - 1); };
+    auto jB = [&](int r) INLINE_LAMBDA { return !YG || (jb + r >= 0 && jb + r < NY); };
+    auto jC = [&](int r) INLINE_LAMBDA { return !YG || (jb + r > 0 && jb + r < NY - 1); };
+    auto jq = [&](int r) INLINE_LAMBDA { return min(max(jb + r, 0), NY - 1); };
+    auto lyh = [&](int r) INLINE_LAMBDA { return YG && jA(r) ? hlay(1, jb + r) : -1; };
+    auto lye = [&](int r) INLINE_LAMBDA { return YG && jC(r) ? elay(1, jb + r) : -1; };
+    auto lxh = [&](int ip) INLINE_LAMBDA { return XG && ip < NX - 1 ? hlay(0, ip) : -1; };
+    auto lxe = [&](int ip) INLINE_LAMBDA { return XG && ip > 0 && ip < NX - 1 ? elay(0, ip) : -1; };
 
     const float Chh = ra.Chh, Che = ra.Che, Cee = ra.Cee, Ceh = ra.Ceh;
     // adjoint: the forward Ceh and Che (Q = cE Ehat, G = cH Hhat_tot) and their inverses
     const float cE = -Che, cH = -Ceh, icE = ADJ ? 1.f / cE : 0.f, icH = ADJ ? 1.f / cH : 0.f;
     const char *bEx = ra.Ein[0], *bEy = ra.Ein[1], *bEz = ra.Ein[2];
     const char *bHx = ra.Hin[0], *bHy = ra.Hin[1], *bHz = ra.Hin[2];
-    char *oEx = ra.Eout[0], *oEy = ra.Eout[1], *oEz = ra.Eout[2];
-    char *oHx = ra.Hout[0], *oHy = ra.Hout[1], *oHz = ra.Hout[2];
     const bool last_lane = lane == 63 && w < W - 1, first_lane = lane == 0 && w > 0;
 
-    auto e_up = [&](const float *x, const float *y, int b, float *xk, float *yk) {
+    auto e_up = [&](const float *x, const float *y, int b, float *xk, float *yk) INLINE_LAMBDA {
 #pragma unroll
         for (int r = 0; r <= R; r++) { xk[r] = from_upper_lane(x[r]); yk[r] = from_upper_lane(y[r]); }
         if (last_lane) {
@@ -813,7 +867,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
         }
     };
     // adjoint: the first lane (outside the z slabs) publishes its z weights
-    auto e_publish = [&](const float *x, const float *y, int b) {
+    auto e_publish = [&](const float *x, const float *y, int b) INLINE_LAMBDA {
         if (lane == 0) {
 #pragma unroll
             for (int r = 0; r <= R; r++) {
@@ -835,11 +889,10 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
         float hxy[R + 1], hzy[R + 1], exy[ADJ ? R + 2 : R], ezy[ADJ ? R + 2 : R];
         float hyx[R + 1], hzx[R + 1], eyx[ADJ ? R + 1 : R], ezx[ADJ ? R + 1 : R];
     };
-    auto load_psi = [&](int ip, PSet &P) {
-#pragma unroll
-        for (int r = 0; r <= R; r++) { P.hxz[r] = 0.f; P.hyz[r] = 0.f; P.exz[r] = 0.f; P.eyz[r] = 0.f; }
-        const bool iA = !XG || ip < NX - 1, iC = !XG || (ip > 0 && ip < NX - 1);
+    auto load_psi = [&](int ip, PSet &P) INLINE_LAMBDA {
         if (ADJ) {
+#pragma unroll
+            for (int r = 0; r <= R; r++) { P.hxz[r] = 0.f; P.hyz[r] = 0.f; P.exz[r] = 0.f; P.eyz[r] = 0.f; }
             // adjoint: psi_E of rows 0..R (z weights of the H half), psi_H of rows 1..R (E half).
             // Rows clamped into the grid: on a y slab or corner column a tile's halo row
             // can be j = -1 or j = NY (at planes 0 and NX-1 outside the arrays); their
@@ -893,54 +946,48 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
             }
             return;
         }
-        if (zh && iA && lzh >= 0) {
-            const gfloat *pa = psi(pp * 6 + 0), *pb = psi(pp * 6 + 2);
+        // every load issued, rows and layers clamped into the arrays (values unused where the term does not apply)
+        if constexpr (ZS) {
 #pragma unroll
-            for (int r = 0; r <= R; r++)
-                if (jA(r)) {
-                    const long q = ((long)ip * NY + jb + r) * Lzh + lzh;
-                    P.hxz[r] = pa[q];
-                    P.hyz[r] = pb[q];
-                }
-        }
-        if (ze && iA && lze >= 0) {
-            const gfloat *pa = psi(12 + 0), *pb = psi(12 + 2);
+            for (int r = 0; r <= R; r++) {
+                const unsigned o = ((unsigned)(ip * NY + jq(r)) * (unsigned)Lzh) * 4u;
+                P.hxz[r] = bld(rp, vzh, ra.hin[0] + o);
+                P.hyz[r] = bld(rp, vzh, ra.hin[2] + o);
+            }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
-                const long q = ((long)ip * NY + jb + r) * Lze + lze;
-                if (jC(r)) P.exz[r - 1] = pa[q];
-                if (iC && jA(r)) P.eyz[r - 1] = pb[q];
+                const unsigned o = ((unsigned)(ip * NY + jq(r)) * (unsigned)Lze) * 4u;
+                P.exz[r - 1] = bld(rp, vze, ra.eio[0] + o);
+                P.eyz[r - 1] = bld(rp, vze, ra.eio[2] + o);
             }
         }
         if (YG) {
-            const gfloat *h1 = psi(pp * 6 + 1), *h5 = psi(pp * 6 + 5), *e1 = psi(12 + 1), *e4 = psi(12 + 4);
 #pragma unroll
             for (int r = 0; r <= R; r++) {
-                const long q = ((long)ip * Lyh + max(lyh(r), 0)) * NZ + kq;
-                P.hxy[r] = h1[q];
-                P.hzy[r] = h5[q];
+                const unsigned o = ((unsigned)(ip * Lyh + max(lyh(r), 0)) * (unsigned)NZ) * 4u;
+                P.hxy[r] = bld(rp, vk, ra.hin[1] + o);
+                P.hzy[r] = bld(rp, vk, ra.hin[5] + o);
             }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
-                const long q = ((long)ip * Lye + max(lye(r), 0)) * NZ + kq;
-                P.exy[r - 1] = e1[q];
-                P.ezy[r - 1] = e4[q];
+                const unsigned o = ((unsigned)(ip * Lye + max(lye(r), 0)) * (unsigned)NZ) * 4u;
+                P.exy[r - 1] = bld(rp, vk, ra.eio[1] + o);
+                P.ezy[r - 1] = bld(rp, vk, ra.eio[4] + o);
             }
         }
         if (XG) {
-            const gfloat *h3 = psi(pp * 6 + 3), *h4 = psi(pp * 6 + 4), *e3 = psi(12 + 3), *e5 = psi(12 + 5);
             const int lh = max(lxh(ip), 0), le = max(lxe(ip), 0);
 #pragma unroll
             for (int r = 0; r <= R; r++) {
-                const long q = ((long)lh * NY + jq(r)) * NZ + kq;
-                P.hyx[r] = h3[q];
-                P.hzx[r] = h4[q];
+                const unsigned o = ((unsigned)(lh * NY + jq(r)) * (unsigned)NZ) * 4u;
+                P.hyx[r] = bld(rp, vk, ra.hin[3] + o);
+                P.hzx[r] = bld(rp, vk, ra.hin[4] + o);
             }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
-                const long q = ((long)le * NY + jq(r)) * NZ + kq;
-                P.eyx[r - 1] = e3[q];
-                P.ezx[r - 1] = e5[q];
+                const unsigned o = ((unsigned)(le * NY + jq(r)) * (unsigned)NZ) * 4u;
+                P.eyx[r - 1] = bld(rp, vk, ra.eio[3] + o);
+                P.ezx[r - 1] = bld(rp, vk, ra.eio[5] + o);
             }
         }
     };
@@ -950,7 +997,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     // H side (rows 1..R, from Hhat_tot): Wxz/Che = hx ik + c (psi/Che + hx),
     // Wyz/Che = hy ik - c (psi/Che - hy), psi_H <- b (psi +- Che h).  Zero
     // outside the component domains (k_adj_step's adj_v, adj_w).
-    auto zweights = [&](int ip, const float *x, const float *y, const PSet &P, bool wr, float *zx, float *zy) {
+    auto zweights = [&](int ip, const float *x, const float *y, const PSet &P, bool wr, float *zx, float *zy) INLINE_LAMBDA {
 #pragma unroll
         for (int r = 0; r <= R; r++) {
             // x and y parts of the ex and ey domains (always true on a clean box)
@@ -969,7 +1016,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
             zy[r] = dy ? ay : 0.f;
         }
     };
-    auto hweights = [&](int ip, const float *hx, const float *hy, const PSet &P, float *wx, float *wy) {
+    auto hweights = [&](int ip, const float *hx, const float *hy, const PSet &P, float *wx, float *wy) INLINE_LAMBDA {
 #pragma unroll
         for (int r = 1; r <= R; r++) {
             const bool dx = jA(r), dy = (!XG || ip < NX - 1) && jB(r);   // x and y parts of the hx, hy domains
@@ -992,7 +1039,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     // own cells write the psi adjoints).
     // y, V of rows 0..R+1 of plane ip: Vxy = Q ik + c (psi + Q), Vzy = Q ik - c (psi - Q)
     auto vyweights = [&](int ip, const float *ex, const float *ez, float exj, float ezj, const PSet &P, bool wr,
-                         float *vxy, float *vzy) {
+                         float *vxy, float *vzy) INLINE_LAMBDA {
 #pragma unroll
         for (int r = 0; r <= R + 1; r++) {
             const float Qx = cE * (r <= R ? ex[r] : exj), Qz = cE * (r <= R ? ez[r] : ezj);
@@ -1016,7 +1063,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     };
     // x, V of rows 0..R of plane ip: Vyx = Q ik - c (psi - Q), Vzx = Q ik + c (psi + Q)
     auto vxweights = [&](int ip, const float *ey, const float *ez, const float *pyx, const float *pzx, bool wr,
-                         float *vyx, float *vzx) {
+                         float *vyx, float *vzx) INLINE_LAMBDA {
         const bool iC = ip > 0 && ip < NX - 1;
         const float ikx = ik(0, true, min(max(ip, 0), NX - 1), NX);
         const int lx = lxe(ip);
@@ -1040,7 +1087,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
         }
     };
     // y, W of rows 0..R of plane ip: Wxy = G ik - c (psi - G), Wzy = G ik + c (psi + G)
-    auto wyweights = [&](int ip, const float *hx, const float *hz, const PSet &P, float *wxy, float *wzy) {
+    auto wyweights = [&](int ip, const float *hx, const float *hz, const PSet &P, float *wxy, float *wzy) INLINE_LAMBDA {
 #pragma unroll
         for (int r = 0; r <= R; r++) {
             const float Gx = cH * hx[r], Gz = cH * hz[r], iky = ik(1, false, jq(r), NY);
@@ -1062,7 +1109,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
         }
     };
     // x, W of rows 1..R of plane ip: Wyx = G ik + c (psi + G), Wzx = G ik - c (psi - G)
-    auto wxweights = [&](int ip, const float *hy, const float *hz, const PSet &P, bool wr, float *wyx, float *wzx) {
+    auto wxweights = [&](int ip, const float *hy, const float *hz, const PSet &P, bool wr, float *wyx, float *wzx) INLINE_LAMBDA {
         const bool iA = ip < NX - 1;
         const float ikx = ik(0, false, min(max(ip, 0), NX - 1), NX);
         const int lx = lxh(ip);
@@ -1098,14 +1145,13 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
                       const float *exk, const float *eyk, const float *ny, const float *nz, const float (*ho)[R + 1],
                       const PSet &P, bool wr, const float *zx, const float *zy, const float *vxy, const float *vzy,
                       const float *vyxc, const float *vzxc, const float *vyxn, const float *vzxn, float *hx, float *hy,
-                      float *hz) {
+                      float *hz) INLINE_LAMBDA {
         const bool iA = !XG || ip < NX - 1;
         const float ikx_h = XG ? ik(0, false, ip, NX) : ra.ik0[1][0];
         const int lx = lxh(ip);
 #pragma unroll
         for (int r = 0; r <= R; r++) {
             const int j = jb + r;
-            const bool own = wr && r > 0 && kown && j < jbox;
             const float iky_h = YG ? ik(1, false, jq(r), NY) : ra.ik0[1][1];
             const float xj = r < R ? ex[r + 1] : exj, zj = r < R ? ez[r + 1] : ezj;
             const float dEy_z = eyk[r] - ey[r], dEz_y = zj - ez[r];
@@ -1132,32 +1178,56 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
             }
             // per component the psi terms add in the reference's order:
             // hx +z -y, hy -z +x, hz -x +y (main.cu:834-1037)
-            if (!ADJ && zh && iA && jA(r) && lzh >= 0) {
-                const long q = ((long)ip * NY + j) * Lzh + lzh;
+            // (the recursions are formed on every lane and dropped where the lane, row or plane has no
+            // such term; the stores of the own cells carry no branch)
+            const bool srow = r > 0 && j < jbox;
+            if constexpr (!ADJ && ZS) {
+                const unsigned o = ((unsigned)(ip * NY + jq(r)) * (unsigned)Lzh) * 4u;
                 const float a = bzh * P.hxz[r] + czh * dEy_z;
                 const float b = bzh * P.hyz[r] + czh * dEx_z;
-                vx += Che * a;
-                vy -= Che * b;
-                if (own) { psi(hout + 0)[q] = a; psi(hout + 2)[q] = b; }
+                const bool u = iA && jA(r);
+                if (u && lzh >= 0) {
+                    vx += Che * a;
+                    vy -= Che * b;
+                }
+                if (wr && r > 0) {
+                    const unsigned v = u && srow ? vzhs : kOob;
+                    bst<false>(rp, v, ra.hout[0] + o, a);
+                    bst<false>(rp, v, ra.hout[2] + o, b);
+                }
             }
             const int ly = lyh(r);
             float pyz = 0.f;
-            if (!ADJ && YG && iA && ly >= 0 && kA) {
-                const long q = ((long)ip * Lyh + ly) * NZ + k;
-                const float by = coef(1, 2, ly), cyv = coef(1, 3, ly);
+            if constexpr (!ADJ && YG) {
+                const int lc = max(ly, 0);
+                const unsigned o = ((unsigned)(ip * Lyh + lc) * (unsigned)NZ) * 4u;
+                const float by = coef(1, 2, lc), cyv = coef(1, 3, lc);
                 const float a = by * P.hxy[r] + cyv * dEz_y;
                 pyz = by * P.hzy[r] + cyv * dEx_y;
-                vx -= Che * a;
-                if (own) { psi(hout + 1)[q] = a; psi(hout + 5)[q] = pyz; }
+                const bool u = iA && ly >= 0;
+                if (u && kA) vx -= Che * a;
+                if (wr && r > 0) {
+                    const unsigned v = u && srow ? vkA : kOob;
+                    bst<false>(rp, v, ra.hout[1] + o, a);
+                    bst<false>(rp, v, ra.hout[5] + o, pyz);
+                }
             }
-            if (!ADJ && XG && lx >= 0 && jA(r) && kA) {
-                const long q = ((long)lx * NY + j) * NZ + k;
-                const float bx = coef(0, 2, lx), cxv = coef(0, 3, lx);
+            if constexpr (!ADJ && XG) {
+                const int lc = max(lx, 0);
+                const unsigned o = ((unsigned)(lc * NY + jq(r)) * (unsigned)NZ) * 4u;
+                const float bx = coef(0, 2, lc), cxv = coef(0, 3, lc);
                 const float a = bx * P.hyx[r] + cxv * dEz_x;
                 const float b = bx * P.hzx[r] + cxv * dEy_x;
-                vy += Che * a;
-                vz -= Che * b;
-                if (own) { psi(hout + 3)[q] = a; psi(hout + 4)[q] = b; }
+                const bool u = lx >= 0 && jA(r);
+                if (u && kA) {
+                    vy += Che * a;
+                    vz -= Che * b;
+                }
+                if (wr && r > 0) {
+                    const unsigned v = u && srow ? vkA : kOob;
+                    bst<false>(rp, v, ra.hout[3] + o, a);
+                    bst<false>(rp, v, ra.hout[4] + o, b);
+                }
             }
             if (!ADJ && YG && iA && ly >= 0 && kA) vz += Che * pyz;
             hx[r] = jA(r) && kA ? vx : ho[0][r];
@@ -1176,14 +1246,14 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     struct HSet { float h[3][R + 1]; };
     float hyP[R + 1], hzP[R + 1];                         // H^{n+1/2} of plane i-1 (adjoint x slabs: Wyx, Wzx)
     float vyxC[R + 1], vzxC[R + 1];                       // adjoint x slabs: Vyx, Vzx of plane i
-    auto load_e = [&](int ip, ESet &e) {
+    auto load_e = [&](int ip, ESet &e) INLINE_LAMBDA {
         const unsigned pl = (unsigned)(ip + 1) * sxy4;
 #pragma unroll
         for (int r = 0; r <= R; r++) { e.x[r] = ldb(bEx, pl + ro[r]); e.y[r] = ldb(bEy, pl + ro[r]); e.z[r] = ldb(bEz, pl + ro[r]); }
         e.xj = ldb(bEx, pl + ro[R + 1]);
         e.zj = ldb(bEz, pl + ro[R + 1]);
     };
-    auto load_h = [&](int ip, HSet &h) {
+    auto load_h = [&](int ip, HSet &h) INLINE_LAMBDA {
         const unsigned pl = (unsigned)(ip + 1) * sxy4;
 #pragma unroll
         for (int r = 0; r <= R; r++) { h.h[0][r] = ldb(bHx, pl + ro[r]); h.h[1][r] = ldb(bHy, pl + ro[r]); h.h[2][r] = ldb(bHz, pl + ro[r]); }
@@ -1244,7 +1314,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
 
     // one x step: C = E of plane i, N = E of plane i+1, Fr <- E of plane i+2,
     // Hc = H of plane i, Hn <- H of plane i+1, Pc <- psi of plane i
-    auto step = [&](int i, ESet &C, ESet &N, ESet &Fr, HSet &Hc, HSet &Hn, PSet &Pc) {
+    auto step = [&](int i, ESet &C, ESet &N, ESet &Fr, HSet &Hc, HSet &Hn, PSet &Pc) INLINE_LAMBDA {
         const bool more = i + 1 < i1;
         const int buf = (i - i0) & 1;
         const unsigned pl = (unsigned)(i + 1) * sxy4;
@@ -1275,7 +1345,9 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
         const float *sy = ADJ ? wy : hy, *sx = ADJ ? wx : hx;
 #pragma unroll
         for (int r = 1; r <= R; r++) {
-            if (kown && jb + r < jbox) { stn<true>(oHx, pl + ro[r], hx[r]); stn<true>(oHy, pl + ro[r], hy[r]); stn<true>(oHz, pl + ro[r], hz[r]); }
+            bst<true>(sHx, so[r], pl, hx[r]);
+            bst<true>(sHy, so[r], pl, hy[r]);
+            bst<true>(sHz, so[r], pl, hz[r]);
             if (lane == 63) { sK[buf][0][wg][r] = sy[r]; sK[buf][1][wg][r] = sx[r]; }
         }
         e_publish(N.x, N.y, buf ^ 1);
@@ -1293,7 +1365,6 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
 #pragma unroll
         for (int r = 1; r <= R; r++) {
             const int j = jb + r;
-            const bool own = kown && j < jbox;
             const float iky_e = YG ? ik(1, true, jq(r), NY) : ra.ik0[0][1];
             const float dHz_y = hz[r] - hz[r - 1], dHy_z = hy[r] - hyk[r];
             const float dHx_z = hx[r] - hxk[r], dHz_x = hz[r] - hzP[r];
@@ -1319,29 +1390,42 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
             }
             const bool ux = iA && jC(r) && kC, uy = iC && jA(r) && kC, uz = iC && jC(r) && kA;
             // ex -z +y, ey +z -x, ez -y +x (main.cu:1172-1906)
-            if (!ADJ && ze && iA && lze >= 0) {
-                const long q = ((long)i * NY + j) * Lze + lze;
-                if (jC(r)) { const float a = bze * Pc.exz[r - 1] + cze * dHy_z; vx -= Ceh * a; if (own) psi(12 + 0)[q] = a; }
-                if (iC && jA(r)) { const float a = bze * Pc.eyz[r - 1] + cze * dHx_z; vy += Ceh * a; if (own) psi(12 + 2)[q] = a; }
+            const bool srow = j < jbox;
+            if constexpr (!ADJ && ZS) {
+                const unsigned o = ((unsigned)(i * NY + jq(r)) * (unsigned)Lze) * 4u;
+                const float a = bze * Pc.exz[r - 1] + cze * dHy_z, b = bze * Pc.eyz[r - 1] + cze * dHx_z;
+                const bool ua = iA && jC(r), ub = iC && jA(r);
+                if (ua && lze >= 0) vx -= Ceh * a;
+                if (ub && lze >= 0) vy += Ceh * b;
+                bst<false>(rp, ua && srow ? vzes : kOob, ra.eio[0] + o, a);
+                bst<false>(rp, ub && srow ? vzes : kOob, ra.eio[2] + o, b);
             }
             const int ly = lye(r);
-            if (!ADJ && YG && iA && ly >= 0) {
-                const long q = ((long)i * Lye + ly) * NZ + k;
-                const float by = coef(1, 0, ly), cyv = coef(1, 1, ly);
-                if (kC) { const float a = by * Pc.exy[r - 1] + cyv * dHz_y; vx += Ceh * a; if (own) psi(12 + 1)[q] = a; }
-                if (iC && kA) { const float a = by * Pc.ezy[r - 1] + cyv * dHx_y; vz -= Ceh * a; if (own) psi(12 + 4)[q] = a; }
+            if constexpr (!ADJ && YG) {
+                const int lc = max(ly, 0);
+                const unsigned o = ((unsigned)(i * Lye + lc) * (unsigned)NZ) * 4u;
+                const float by = coef(1, 0, lc), cyv = coef(1, 1, lc);
+                const float a = by * Pc.exy[r - 1] + cyv * dHz_y, b = by * Pc.ezy[r - 1] + cyv * dHx_y;
+                const bool ua = iA && ly >= 0, ub = iC && ly >= 0;
+                if (ua && kC) vx += Ceh * a;
+                if (ub && kA) vz -= Ceh * b;
+                bst<false>(rp, ua && srow ? vkC : kOob, ra.eio[1] + o, a);
+                bst<false>(rp, ub && srow ? vkA : kOob, ra.eio[4] + o, b);
             }
-            if (!ADJ && XG && lx >= 0) {
-                const long q = ((long)lx * NY + j) * NZ + k;
-                const float bx = coef(0, 0, lx), cxv = coef(0, 1, lx);
-                if (jA(r) && kC) { const float a = bx * Pc.eyx[r - 1] + cxv * dHz_x; vy -= Ceh * a; if (own) psi(12 + 3)[q] = a; }
-                if (jC(r) && kA) { const float a = bx * Pc.ezx[r - 1] + cxv * dHy_x; vz += Ceh * a; if (own) psi(12 + 5)[q] = a; }
+            if constexpr (!ADJ && XG) {
+                const int lc = max(lx, 0);
+                const unsigned o = ((unsigned)(lc * NY + jq(r)) * (unsigned)NZ) * 4u;
+                const float bx = coef(0, 0, lc), cxv = coef(0, 1, lc);
+                const float a = bx * Pc.eyx[r - 1] + cxv * dHz_x, b = bx * Pc.ezx[r - 1] + cxv * dHy_x;
+                const bool ua = lx >= 0 && jA(r), ub = lx >= 0 && jC(r);
+                if (ua && kC) vy -= Ceh * a;
+                if (ub && kA) vz += Ceh * b;
+                bst<false>(rp, ua && srow ? vkC : kOob, ra.eio[3] + o, a);
+                bst<false>(rp, ub && srow ? vkA : kOob, ra.eio[5] + o, b);
             }
-            if (own) {
-                stn<true>(oEx, pl + ro[r], ux ? vx : C.x[r]);
-                stn<true>(oEy, pl + ro[r], uy ? vy : C.y[r]);
-                stn<true>(oEz, pl + ro[r], uz ? vz : C.z[r]);
-            }
+            bst<true>(sEx, so[r], pl, ux ? vx : C.x[r]);
+            bst<true>(sEy, so[r], pl, uy ? vy : C.y[r]);
+            bst<true>(sEz, so[r], pl, uz ? vz : C.z[r]);
         }
         if constexpr (AS && XG) {
 #pragma unroll
@@ -1361,13 +1445,42 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     }
 }
 
-// Two rows per thread fit in 128 VGPRs (four waves per SIMD) on the clean
-// box.  The side-slab variants are not capped: their launches hold one block
-// per CU at most (a few hundred blocks), so a fourth wave per SIMD gains
-// nothing there, while the cap spilled the x-general variant to scratch.
-template <int W, int R, bool XG, bool YG, bool ADJ = false, int T = 1>
-__global__ __launch_bounds__(64 * W * T) __attribute__((amdgpu_waves_per_eu(R == 2 && !XG && !YG ? 4 : 1))) void k_step_rows(RowsArgs ra) {
-    rows_body<W, R, XG, YG, ADJ, T>(ra, ra.xcd ? xcd_order(blockIdx.x, ra.start[ra.npiece]) : (int)blockIdx.x);
+// Whether this wave holds lanes of the z slabs (uniform across the wave).
+template <int R>
+__device__ __forceinline__ bool rows_zwave(const RowsArgs &ra, int ja, int jbox, int L) {
+    const int W = ra.waves, T = ra.tiles;
+    const int njb = ((jbox - ja + R - 1) / R + T - 1) / T;
+    const int wg = __builtin_amdgcn_readfirstlane((int)threadIdx.y), w = wg % W;
+    const int k0 = (L / njb) % ra.nseg * (64 * W - 2) - 1 + 64 * w;   // lane 0
+    return k0 <= ra.Nc[2] || k0 + 63 >= ra.F[2];
+}
+
+// Waves without z-slab lanes run a march without the z-CPML loads and stores
+// (20 of some 60 memory instructions per plane); both marches hold the same
+// barriers.
+template <int R, bool XG, bool YG, bool ADJ>
+__device__ __forceinline__ void rows_piece(const RowsArgs &ra, int ia, int ib, int ja, int jbox, int ichunk, int L,
+                                           RowsLds<R, ADJ> &lds) {
+    if (ADJ || rows_zwave<R>(ra, ja, jbox, L)) rows_block<R, XG, YG, ADJ, true>(ra, ia, ib, ja, jbox, ichunk, L, lds);
+    else rows_block<R, XG, YG, ADJ, false>(ra, ia, ib, ja, jbox, ichunk, L, lds);
+}
+
+// A block of a launch over the pieces of one variant (ra.box, ra.start).
+template <int R, bool XG, bool YG, bool ADJ>
+__device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
+    __shared__ RowsLds<R, ADJ> lds;
+    int pc = 0;
+    while (pc + 1 < ra.npiece && L >= ra.start[pc + 1]) pc++;
+    rows_piece<R, XG, YG, ADJ>(ra, ra.box[pc][0], ra.box[pc][1], ra.box[pc][2], ra.box[pc][3], ra.ichunk,
+                                     L - ra.start[pc], lds);
+}
+
+// MW: the most waves a block of the launch may have, 16 (128 VGPRs) or 12
+// (168 VGPRs, for the variants that need more).  Two rows per thread fit in
+// 128 VGPRs on the clean box, so it always runs at four waves per SIMD.
+template <int MW, int R, bool XG, bool YG, bool ADJ = false>
+__global__ __launch_bounds__(64 * MW) __attribute__((amdgpu_waves_per_eu(R == 2 && !XG && !YG ? 4 : 1))) void k_step_rows(RowsArgs ra) {
+    rows_body<R, XG, YG, ADJ>(ra, ra.xcd ? xcd_order(blockIdx.x, ra.start[ra.npiece]) : (int)blockIdx.x);
 }
 
 // ----------------------------------------------------------------- split path kernels
@@ -2762,20 +2875,6 @@ hipError_t launch_fused_step(const StepDev &s, int tj, int ichunk, const int (*b
 
 // ----------------------------------------------------------------- batched launches
 
-// Items are read through the constant address space: every block reads its
-// item at a uniform address, so the fields land in scalar registers exactly
-// as kernel arguments do.
-#define CONST_AS __attribute__((address_space(4)))
-template <typename T>
-__device__ __forceinline__ const T &batch_item(const T *items, unsigned idx) {
-    const CONST_AS T *c = (const CONST_AS T *)items;
-    return *(const T *)(c + idx);
-}
-__device__ __forceinline__ unsigned batch_map(const unsigned *map) {
-    const CONST_AS unsigned *c = (const CONST_AS unsigned *)map;
-    return c[blockIdx.x];
-}
-
 template <int TJ>
 __global__ __launch_bounds__(64 * TJ) void k_fused_batch(const FusedItem *items, const unsigned *map) {
     const unsigned m = batch_map(map);
@@ -2783,10 +2882,10 @@ __global__ __launch_bounds__(64 * TJ) void k_fused_batch(const FusedItem *items,
     fused_body<TJ>(it.s, it.ichunk, it.nkt, it.pc, (int)(m & ((1u << kBatchLocalBits) - 1)));
 }
 
-template <int W, int R, bool XG, bool YG, int T>
-__global__ __launch_bounds__(64 * W * T) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 : 1))) void k_rows_batch(const RowsArgs *items, const unsigned *map) {
+template <int MW, int R, bool XG, bool YG>
+__global__ __launch_bounds__(64 * MW) __attribute__((amdgpu_waves_per_eu(R == 2 ? 4 : 1))) void k_rows_batch(const RowsArgs *items, const unsigned *map) {
     const unsigned m = batch_map(map);
-    rows_body<W, R, XG, YG, false, T>(batch_item(items, m >> kBatchLocalBits), (int)(m & ((1u << kBatchLocalBits) - 1)));
+    rows_body<R, XG, YG, false>(batch_item(items, m >> kBatchLocalBits), (int)(m & ((1u << kBatchLocalBits) - 1)));
 }
 
 // Local block L of a simulation's TFSF fix-up grid ((span + 63) / 64, span, 12) in x-fastest order.
@@ -2866,35 +2965,25 @@ hipError_t launch_fused_batch(const FusedItem *items, const unsigned *map, int n
     return hipGetLastError();
 }
 
-template <int W>
-static hipError_t launch_rows_batch_w(const RowsArgs *items, const unsigned *map, int nblocks, int R, int variant,
-                                      hipStream_t st) {
-    constexpr int T = W <= 5 ? 2 : 1;   // rows_batch_tiles(W)
-    const dim3 grid(nblocks), block(64, W * T);
-    if (R == 3 && variant == 0) hipLaunchKernelGGL((k_rows_batch<W, 3, false, false, T>), grid, block, 0, st, items, map);
-    else if (R == 2 && variant == 0) hipLaunchKernelGGL((k_rows_batch<W, 2, false, false, T>), grid, block, 0, st, items, map);
-    else if (R == 2 && variant == 1) hipLaunchKernelGGL((k_rows_batch<W, 2, true, false, T>), grid, block, 0, st, items, map);
-    else if (R == 2 && variant == 2) hipLaunchKernelGGL((k_rows_batch<W, 2, false, true, T>), grid, block, 0, st, items, map);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
 int rows_batch_tiles(int W) { return W <= 5 ? 2 : 1; }
 
 hipError_t launch_rows_batch(const RowsArgs *items, const unsigned *map, int nblocks, int W, int R, int variant,
                              hipStream_t st) {
     if (nblocks <= 0) return hipSuccess;
-    switch (W) {
-        case 2: return launch_rows_batch_w<2>(items, map, nblocks, R, variant, st);
-        case 3: return launch_rows_batch_w<3>(items, map, nblocks, R, variant, st);
-        case 4: return launch_rows_batch_w<4>(items, map, nblocks, R, variant, st);
-        case 5: return launch_rows_batch_w<5>(items, map, nblocks, R, variant, st);
-        case 6: return launch_rows_batch_w<6>(items, map, nblocks, R, variant, st);
-        case 8: return launch_rows_batch_w<8>(items, map, nblocks, R, variant, st);
-        case 12: return launch_rows_batch_w<12>(items, map, nblocks, R, variant, st);
-        case 16: return launch_rows_batch_w<16>(items, map, nblocks, R, variant, st);
+    const int nw = W * rows_batch_tiles(W);
+    const dim3 grid(nblocks), block(64, nw);
+    if (nw > kRowsMaxWaves || R < 2 || R > 3 || (R == 3 && variant != 0)) return hipErrorInvalidValue;
+    switch (variant) {
+        case 0:
+            if (R == 2) hipLaunchKernelGGL((k_rows_batch<16, 2, false, false>), grid, block, 0, st, items, map);
+            else if (nw <= 12) hipLaunchKernelGGL((k_rows_batch<12, 3, false, false>), grid, block, 0, st, items, map);
+            else hipLaunchKernelGGL((k_rows_batch<16, 3, false, false>), grid, block, 0, st, items, map);
+            break;
+        case 1: hipLaunchKernelGGL((k_rows_batch<16, 2, true, false>), grid, block, 0, st, items, map); break;
+        case 2: hipLaunchKernelGGL((k_rows_batch<16, 2, false, true>), grid, block, 0, st, items, map); break;
         default: return hipErrorInvalidValue;
     }
+    return hipGetLastError();
 }
 
 hipError_t launch_tfsf_fix_batch(const FusedItem *items, const unsigned *map, int nblocks, hipStream_t st) {
@@ -2933,60 +3022,12 @@ hipError_t launch_batch_advance(int *dyn, int dt, int dslot, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <int W, bool XG, bool YG, bool ADJ>
-static hipError_t launch_rows_w(const RowsArgs &ra, int R, dim3 grid, hipStream_t st) {
-    if (ra.tiles == 2) {
-        if constexpr (W * 2 <= 16 && !(XG && YG)) {
-            switch (R) {
-                case 2: hipLaunchKernelGGL((k_step_rows<W, 2, XG, YG, ADJ, 2>), grid, dim3(64, 2 * W), 0, st, ra); break;
-                case 3:
-                    if constexpr (!XG && !YG && !ADJ) {
-                        hipLaunchKernelGGL((k_step_rows<W, 3, false, false, false, 2>), grid, dim3(64, 2 * W), 0, st, ra);
-                        break;
-                    }
-                    return hipErrorInvalidValue;
-                default: return hipErrorInvalidValue;
-            }
-            return hipGetLastError();
-        }
-        return hipErrorInvalidValue;
-    }
-    if (ra.tiles == 3) {
-        if constexpr (W * 3 <= 16 && !XG && !YG && !ADJ) {
-            switch (R) {
-                case 2: hipLaunchKernelGGL((k_step_rows<W, 2, false, false, false, 3>), grid, dim3(64, 3 * W), 0, st, ra); break;
-                case 3: hipLaunchKernelGGL((k_step_rows<W, 3, false, false, false, 3>), grid, dim3(64, 3 * W), 0, st, ra); break;
-                default: return hipErrorInvalidValue;
-            }
-            return hipGetLastError();
-        }
-        return hipErrorInvalidValue;
-    }
-    switch (R) {
-        case 2: hipLaunchKernelGGL((k_step_rows<W, 2, XG, YG, ADJ>), grid, dim3(64, W), 0, st, ra); break;
-        case 3:
-            if constexpr (!(XG && YG) && (!ADJ || (!XG && !YG))) {
-                hipLaunchKernelGGL((k_step_rows<W, 3, XG, YG, ADJ>), grid, dim3(64, W), 0, st, ra);
-                break;
-            }
-            return hipErrorInvalidValue;
-        default: return hipErrorInvalidValue;
-    }
+template <int R, bool XG, bool YG, bool ADJ = false>
+static hipError_t launch_rows_g(const RowsArgs &ra, dim3 grid, hipStream_t st) {
+    const int nw = ra.waves * ra.tiles;
+    if (nw <= 12) hipLaunchKernelGGL((k_step_rows<12, R, XG, YG, ADJ>), grid, dim3(64, nw), 0, st, ra);
+    else hipLaunchKernelGGL((k_step_rows<16, R, XG, YG, ADJ>), grid, dim3(64, nw), 0, st, ra);
     return hipGetLastError();
-}
-
-template <bool XG, bool YG, bool ADJ = false>
-static hipError_t launch_rows_g(const RowsArgs &ra, int R, int W, dim3 grid, hipStream_t st) {
-    switch (W) {
-        case 2: return launch_rows_w<2, XG, YG, ADJ>(ra, R, grid, st);
-        case 3: return launch_rows_w<3, XG, YG, ADJ>(ra, R, grid, st);
-        case 4: return launch_rows_w<4, XG, YG, ADJ>(ra, R, grid, st);
-        case 5: return launch_rows_w<5, XG, YG, ADJ>(ra, R, grid, st);
-        case 6: return launch_rows_w<6, XG, YG, ADJ>(ra, R, grid, st);
-        case 8: return launch_rows_w<8, XG, YG, ADJ>(ra, R, grid, st);
-        case 12: return launch_rows_w<12, XG, YG, ADJ>(ra, R, grid, st);
-        default: return launch_rows_w<16, XG, YG, ADJ>(ra, R, grid, st);
-    }
 }
 
 int rows_waves(int NZ) {
@@ -3007,6 +3048,7 @@ long rows_prepare(RowsArgs &ra, int R, int variant) {
     const bool xg = variant == 1 || variant == 4 || variant == 6, yg = variant == 2 || variant == 5 || variant == 6;
     if (variant == 6 && ra.tiles != 1) return -1;   // the corner variant is built for one row tile
     const int T = ra.tiles;
+    ra.waves = W;
     ra.nseg = (ra.NZ + 1 + 64 * W - 3) / (64 * W - 2);
     long total = 0;
     for (int q = 0; q < ra.npiece; q++) {
@@ -3025,16 +3067,15 @@ long rows_prepare(RowsArgs &ra, int R, int variant) {
 hipError_t launch_step_rows(RowsArgs ra, int R, int variant, hipStream_t st) {
     const long total = rows_prepare(ra, R, variant);
     if (total < 0) return hipErrorInvalidValue;
-    const int W = rows_waves(ra.NZ);
     const dim3 grid((unsigned)total);
     switch (variant) {
-        case 0: return launch_rows_g<false, false>(ra, R, W, grid, st);
-        case 1: return launch_rows_g<true, false>(ra, R, W, grid, st);
-        case 2: return launch_rows_g<false, true>(ra, R, W, grid, st);
-        case 3: return launch_rows_g<false, false, true>(ra, R, W, grid, st);
-        case 4: return launch_rows_g<true, false, true>(ra, R, W, grid, st);
-        case 5: return launch_rows_g<false, true, true>(ra, R, W, grid, st);
-        default: return launch_rows_g<true, true, true>(ra, R, W, grid, st);
+        case 0: return R == 2 ? launch_rows_g<2, false, false>(ra, grid, st) : launch_rows_g<3, false, false>(ra, grid, st);
+        case 1: return R == 2 ? launch_rows_g<2, true, false>(ra, grid, st) : launch_rows_g<3, true, false>(ra, grid, st);
+        case 2: return R == 2 ? launch_rows_g<2, false, true>(ra, grid, st) : launch_rows_g<3, false, true>(ra, grid, st);
+        case 3: return R == 2 ? launch_rows_g<2, false, false, true>(ra, grid, st) : launch_rows_g<3, false, false, true>(ra, grid, st);
+        case 4: return launch_rows_g<2, true, false, true>(ra, grid, st);
+        case 5: return launch_rows_g<2, false, true, true>(ra, grid, st);
+        default: return launch_rows_g<2, true, true, true>(ra, grid, st);
     }
 }
 

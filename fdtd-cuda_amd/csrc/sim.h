@@ -24,6 +24,8 @@ struct fdtd_sim {
     // fields: [parity][component]
     float *E[2][3] = {}, *H[2][3] = {};
     int p = 0;                      // current field parity
+    float *psi = nullptr;           // the allocation of every psi array (npsi floats)
+    size_t npsi = 0;
     float *psiH[2][6] = {}, *psiE[6] = {};
     int pp = 0;                     // current psi_H parity
     // CPML tables (float)
