@@ -369,6 +369,28 @@ hipEvent_t next_event(fdtd_sim *s, int which) {
 }
 
 
+// x chunk of the one-launch update.  A block marches chunk + 2 planes' worth of
+// time (the plane before its chunk is recomputed, and the march fills up), and
+// the launch takes as many rounds of resident blocks as its block count needs:
+// the chunk with the smallest rounds * (chunk + 2) is taken.  It goes from one
+// plane where every block is resident at once to 12 where many rounds run
+// (measured us per step, chunks 1, 2, 4, 8, 12, 16: 37^3 22, 26, 34, 47, -, 53;
+// 85^3 37, 34, 39, 55, -, 67; 125 x 173 x 204 -, 102, 89, 92, -, -; 281^3 648,
+// 477, 400, 373, 370, 375).
+int one_launch_chunk(const fdtd_sim *s, int tiles) {
+    const int nw = rows_waves(s->g.NZ) * tiles;
+    const long slots = 256L * std::max(1, 4 / ((nw + 3) / 4));   // blocks resident at four waves per SIMD
+    const long rows = (s->g.NY + 2 * tiles - 1) / (2 * tiles);
+    int best = 1;
+    long cost = -1;
+    for (int c : {1, 2, 3, 4, 6, 8, 12}) {
+        const long blocks = rows * ((s->g.NX + c - 1) / c);
+        const long t = (blocks + slots - 1) / slots * (c + 2);
+        if (cost < 0 || t < cost) { cost = t; best = c; }
+    }
+    return best;
+}
+
 // The row-blocked kernel (k_step_rows) runs the whole grid with TFSF left
 // out; k_tfsf_fix then adds it, which needs the TFSF cells and their
 // neighbours free of CPML and with 1/(kappa d) at its interior value.  The
@@ -502,6 +524,17 @@ int plan_rows(fdtd_sim *s) {
             return set_err(s, FDTD_ERR_DEVICE, "side streams or events could not be created");
     }
     s->use_rows = s->has_clean;
+    // One launch for the whole update up to 12 M cells, unless a knob of the stream schedule
+    // asks for that (FDTD_ONE_LAUNCH=0: the schedule with its defaults); two rows per thread
+    // only.  Measured us per step, one launch against the streams: 22 and 91 at 0.05 M cells,
+    // 35 and 90 at 0.6 M, 89 and 121 at 4.4 M, 374 and 369 at 22 M, 929 and 907 at 68 M
+    // (there the post-update launch overlaps the next step's side pieces).
+    s->one_launch = s->rows == 2 && (long)s->g.NX * s->g.NY * s->g.NZ <= 12000000L;
+    if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = s->one_launch && std::atoi(v) != 0;
+    for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
+                          "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
+        if (std::getenv(k)) s->one_launch = false;
+    s->one_chunk = one_launch_chunk(s, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1);
     return FDTD_OK;
 }
 
@@ -757,6 +790,42 @@ int launch_rows_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Di
     return FDTD_OK;
 }
 
+// The whole field update in one launch on the solver stream, then the
+// post-update launch.
+int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const DispDev *dd, bool samp, bool *disp_done,
+                      bool *samp_done, hipEvent_t ev0, hipEvent_t ev1) {
+    StepAll a{};
+    a.r = make_rows(s);
+    a.line = l;
+    a.r.tiles = s->tiles * rows_waves(s->g.NZ) <= 16 ? s->tiles : 1;
+    // the costlier pieces first, so the launch ends on the cheap ones; equal chunks within a piece
+    auto add = [&](int kind, int chunk, const int (*b)[4], int n) {
+        for (int q = 0; q < n; q++) {
+            const int len = b[q][1] - b[q][0], parts = (len + chunk - 1) / chunk;
+            a.kind[a.n] = kind;
+            a.ich[a.n] = (len + parts - 1) / parts;
+            std::memcpy(a.box[a.n], b[q], sizeof(a.box[0]));
+            a.n++;
+        }
+    };
+    const int side = std::min(s->one_chunk, 8);
+    add(3, side, s->cbox4, s->ncorner);
+    add(1, side, s->xbox, s->nxbox);
+    add(2, side, s->ybox, s->nybox);
+    add(0, s->one_chunk, &s->cbox, 1);
+    if (ev0) HIPCHK(s, hipEventRecord(ev0, s->stream));
+    HIPCHK(s, launch_step_all(a, s->stream));
+    if (ev1) HIPCHK(s, hipEventRecord(ev1, s->stream));
+    // the box and the sample ride with the TFSF fix-up where their cells are apart from it
+    const bool merge_disp = dd && !s->S.hydro && disp_in_clean(s);
+    const bool merge_samp = samp && d.sample_row && (s->nbox <= 0 || disp_in_clean(s)) && sample_in_clean(s);
+    if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, merge_disp ? dd : nullptr, merge_samp, s->stream));
+    else HIPCHK(s, launch_tfsf_fix(d, s->stream));
+    *disp_done = merge_disp;
+    *samp_done = merge_samp;
+    return FDTD_OK;
+}
+
 }  // namespace fdtd_host
 
 
@@ -950,7 +1019,13 @@ int fdtd_get_info(const fdtd_sim *s, fdtd_grid_info *g) {
         g->tile[3] = s->tiles * W <= 16 ? s->tiles : 1;
         g->tile[4] = s->stiles * W <= 16 ? s->stiles : 1;
         g->tile[5] = s->ctj;
-        g->tile[6] = s->stream2 ? (s->stream3 ? 3 : 1) : 0;
+        g->tile[6] = s->stream2 && !s->one_launch ? (s->stream3 ? 3 : 1) : 0;
+        if (s->one_launch) {
+            g->tile[1] = s->one_chunk;
+            g->tile[2] = std::min(s->one_chunk, 8);
+            g->tile[4] = g->tile[3];
+            g->tile[5] = 0;
+        }
     } else {
         g->tile[0] = s->tj;
         g->tile[1] = s->ichunk;
@@ -1695,8 +1770,9 @@ int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
             d.tfsf_on = 0;
             if (samp) d.sample_row = s->X + (size_t)s->slot * s->mtot;
             if (step_timing && !only_clean) HIPCHK(s, hipEventRecord(ev0, s->stream));
-            int rc2 = launch_rows_update(s, d, l, s->nbox ? &dd : nullptr, samp, &disp_done, &samp_done,
-                                         only_clean ? ev0 : nullptr, only_clean ? ev1 : nullptr);
+            int rc2 = (s->one_launch ? launch_one_update : launch_rows_update)(
+                s, d, l, s->nbox ? &dd : nullptr, samp, &disp_done, &samp_done, only_clean ? ev0 : nullptr,
+                only_clean ? ev1 : nullptr);
             if (rc2) return rc2;
             if (step_timing && !only_clean) HIPCHK(s, hipEventRecord(ev1, s->stream));
         } else {

@@ -252,6 +252,23 @@ int rows_waves(int NZ);
 // the corner columns (x and y general), two rows, one row tile.
 hipError_t launch_step_rows(RowsArgs ra, int R, int variant, hipStream_t st);
 
+// The field update of a step in one launch (k_step_all): the pieces of the
+// grid on the row-blocked kernel with two rows per thread, and the 1D line.
+// kind[q]: bit 0 x general, bit 1 y general (0 clean box, 1 x slab, 2 y slab,
+// 3 corner column).  r: common arguments (tiles for every piece; its boxes and
+// chunk are not used).  start is filled in by the launcher.
+constexpr int kStepAllPieces = 9;
+struct StepAll {
+    RowsArgs r;
+    LineDev line;
+    int n;
+    int kind[kStepAllPieces], ich[kStepAllPieces], box[kStepAllPieces][4];
+    int start[kStepAllPieces + 1];
+};
+hipError_t launch_step_all(StepAll a, hipStream_t st);
+// Blocks of one piece (two rows per thread, r.tiles row tiles per block).
+long rows_pieces_blocks(const RowsArgs &r, const int box[4], int ichunk);
+
 // box[q] = {ia, ib, ja, jb}; one to four disjoint boxes.
 hipError_t launch_fused_step(const StepDev &s, int tj, int ichunk, const int (*box)[4], int nbox, hipStream_t st);
 hipError_t launch_split_h(const StepDev &s, hipStream_t st);

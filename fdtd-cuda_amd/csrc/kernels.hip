@@ -695,7 +695,7 @@ __device__ inline void lds_sync() {
 // becomes a wait for the store's completion too: in the march of the
 // row-blocked kernel that put the completion of one plane's stores in front of
 // the next plane's arithmetic (clean box of a 281^3 grid alone 223 -> 215 us,
-// of a 121^3 grid and smaller a third less per plane).
+// a whole 37^3 grid in x chunks of 16 planes 57 -> 45 us).
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr unsigned kOob = 0xFFFFFFFCu;
 __device__ __forceinline__ rsrc_t make_rsrc(const void *base, unsigned bytes) {
@@ -2054,13 +2054,13 @@ __global__ void k_disp_sync(DispDev d, int from_field) {
 
 // One block: h_inc (main.cu:2328-2336), e_inc (main.cu:2280-2326) into the
 // other buffer, first-order Mur ends and the additive source (main.cu:2831-2859).
-__device__ __forceinline__ void line_body(const LineDev &l, int t) {
+__device__ __forceinline__ void line_body(const LineDev &l, int t, int tid, int nthreads) {
     const int L = l.L;
-    for (int i = threadIdx.x; i < L - 1; i += blockDim.x) l.h[i] = l.h[i] - l.ch * (l.e_old[i + 1] - l.e_old[i]);
+    for (int i = tid; i < L - 1; i += nthreads) l.h[i] = l.h[i] - l.ch * (l.e_old[i + 1] - l.e_old[i]);
     __syncthreads();
-    for (int i = threadIdx.x + 1; i < L - 1; i += blockDim.x) l.e_new[i] = l.e_old[i] - l.ce * (l.h[i] - l.h[i - 1]);
+    for (int i = tid + 1; i < L - 1; i += nthreads) l.e_new[i] = l.e_old[i] - l.ce * (l.h[i] - l.h[i - 1]);
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         const double e1 = l.mur[0], e2 = l.mur[1];
         l.e_new[0] = e1 + l.mur_coef * (l.e_new[1] - l.e_old[0]);
         l.e_new[L - 1] = e2 + l.mur_coef * (l.e_new[L - 2] - l.e_old[L - 1]);
@@ -2080,7 +2080,37 @@ __device__ __forceinline__ void line_body(const LineDev &l, int t) {
     }
 }
 
-__global__ __launch_bounds__(1024) void k_line(LineDev l) { line_body(l, l.t); }
+__global__ __launch_bounds__(1024) void k_line(LineDev l) { line_body(l, l.t, threadIdx.x, blockDim.x); }
+
+// The whole field update of a step in one launch: block 0 is the 1D line, the
+// others the pieces of the grid (corner columns, x slabs, y slabs, clean box),
+// each piece with its own x chunk.  Small grids are bound by the march (2-3 us
+// per plane whatever the grid) and by the packets between launches: on one
+// stream, with chunks of 1 to 4 planes, the step of a 37^3 grid takes 22 us
+// against 91 us with the pieces on four streams in chunks of 16, of 85^3 34
+// against 90, of 125 x 173 x 204 88 against 122.  Large grids are bound by
+// memory: at 281^3 the launch moves 1.56 GB (1.25 GB it cannot do without) in
+// 315 us, 4.9 TB/s, what a large copy reaches on this card.
+__global__ __launch_bounds__(64 * kRowsMaxWaves) void k_step_all(StepAll) {
+    // the arguments in place (their only copy; a by-value struct indexed by piece would be copied to scratch)
+    const StepAll &a = batch_item((const StepAll *)(const CONST_AS StepAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
+    __shared__ RowsLds<2, false> lds;
+    if (blockIdx.x == 0) {
+        line_body(a.line, a.line.t, threadIdx.y * 64 + threadIdx.x, 64 * a.r.waves * a.r.tiles);
+        return;
+    }
+    const int b = (int)blockIdx.x - 1;
+    int q = 0;
+    while (q + 1 < a.n && b >= a.start[q + 1]) q++;
+    const int ia = a.box[q][0], ib = a.box[q][1], ja = a.box[q][2], jb = a.box[q][3], ich = a.ich[q];
+    const int L = a.r.xcd ? xcd_order(b - a.start[q], a.start[q + 1] - a.start[q]) : b - a.start[q];
+    switch (a.kind[q]) {
+        case 0: rows_piece<2, false, false, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 1: rows_piece<2, true, false, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 2: rows_piece<2, false, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        default: rows_piece<2, true, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+    }
+}
 
 // ----------------------------------------------------------------- DFT contraction
 
@@ -2904,7 +2934,7 @@ __global__ __launch_bounds__(256) void k_tfsf_fix_batch(const FusedItem *items, 
 
 __global__ __launch_bounds__(1024) void k_line_batch(const LineDev *items, const int *dyn, int step_off) {
     const CONST_AS int *d = (const CONST_AS int *)dyn;
-    line_body(batch_item(items, blockIdx.x), d[0] + step_off);
+    line_body(batch_item(items, blockIdx.x), d[0] + step_off, threadIdx.x, blockDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_disp_batch(const DispDev *items, const unsigned *map) {
@@ -3077,6 +3107,34 @@ hipError_t launch_step_rows(RowsArgs ra, int R, int variant, hipStream_t st) {
         case 5: return launch_rows_g<2, false, true, true>(ra, grid, st);
         default: return launch_rows_g<2, true, true, true>(ra, grid, st);
     }
+}
+
+hipError_t launch_step_all(StepAll a, hipStream_t st) {
+    const int W = rows_waves(a.r.NZ);
+    if (a.n < 1 || a.n > kStepAllPieces || a.r.tiles < 1 || a.r.tiles * W > kRowsMaxWaves) return hipErrorInvalidValue;
+    a.r.waves = W;
+    a.r.nseg = (a.r.NZ + 1 + 64 * W - 3) / (64 * W - 2);
+    long total = 0;
+    for (int q = 0; q < a.n; q++) {
+        const int *b = a.box[q];
+        const bool xg = a.kind[q] & 1, yg = a.kind[q] & 2;
+        if (a.kind[q] < 0 || a.kind[q] > 3 || a.ich[q] < 1 || b[0] < 0 || b[1] > a.r.NX || b[0] >= b[1] || b[2] < 0 ||
+            b[3] > a.r.NY || b[2] >= b[3])
+            return hipErrorInvalidValue;
+        if ((!xg && (b[0] < 1 || b[1] > a.r.NX - 1)) || (!yg && (b[2] < 1 || b[3] > a.r.NY - 1))) return hipErrorInvalidValue;
+        a.start[q] = (int)total;
+        total += rows_pieces_blocks(a.r, b, a.ich[q]);
+    }
+    if (total + 1 > 0x7fffffff) return hipErrorInvalidValue;
+    a.start[a.n] = (int)total;
+    hipLaunchKernelGGL(k_step_all, dim3((unsigned)(total + 1)), dim3(64, W * a.r.tiles), 0, st, a);
+    return hipGetLastError();
+}
+
+long rows_pieces_blocks(const RowsArgs &r, const int box[4], int ichunk) {
+    const int W = rows_waves(r.NZ), T = r.tiles;
+    const long nseg = (r.NZ + 1 + 64 * W - 3) / (64 * W - 2);
+    return (long)(((box[3] - box[2] + 1) / 2 + T - 1) / T) * nseg * ((box[1] - box[0] + ichunk - 1) / ichunk);
 }
 
 hipError_t launch_adj_step(const AdjDev &a, int tj, int ichunk, const int (*box)[4], int nbox, hipStream_t st) {

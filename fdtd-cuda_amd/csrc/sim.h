@@ -101,6 +101,8 @@ struct fdtd_sim {
     float ik0[2][2] = {};           // interior 1/(kappa d): [E, H][x, y]
     unsigned *aux_d = nullptr;      // table image of the row-blocked kernel
     std::vector<uint32_t> aux_img;  // host copy of it
+    bool one_launch = false;        // field update of fdtd_step in one launch (k_step_all), not on streams
+    int one_chunk = 1;              // its x chunk
     bool concurrent = true;         // side slabs on a second stream beside the clean box (FDTD_CONCURRENT=0 to serialise)
     hipStream_t stream2 = nullptr;
     // ev_line: the 1D line's completion in a step; the transposed step reuses it

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 # the middle wave of three holds k = 63 .. 126; the far slab starts at NZ - 1 - 6
 @pytest.mark.parametrize("nz,first_far", [(119, 125), (120, 126), (121, 127), (176, 182), (184, 190), (50, 56)])
 def test_far_slab_at_a_wave_edge(nz, first_far):
-    p = small_params(fdtd_amd, n=20)
+    p = small_params(fdtd_amd, n=20, sphere=0)
     p.NCELLZ = nz
     fields = []
     for split in (False, True):
