@@ -205,7 +205,7 @@ void adj_release(fdtd_sim *s) {
     dfree(s, s->adj.corr);
     dfree(s, s->adj.aux_d);
     s->adj.ready = false;
-    s->adj.rows = s->adj.rows_slabs = false;
+    s->adj.rows = s->adj.rows_slabs = s->adj.one_launch = false;
 }
 
 // Builds the dispersive box from the masks and uploads ids; state zeroed.
@@ -369,7 +369,7 @@ hipEvent_t next_event(fdtd_sim *s, int which) {
 }
 
 
-// x chunk of the one-launch update.  A block marches chunk + 2 planes' worth of
+// x chunk of a march.  A block marches chunk + 2 planes' worth of
 // time (the plane before its chunk is recomputed, and the march fills up), and
 // the launch takes as many rounds of resident blocks as its block count needs:
 // the chunk with the smallest rounds * (chunk + 2) is taken.  It goes from one
@@ -377,18 +377,52 @@ hipEvent_t next_event(fdtd_sim *s, int which) {
 // (measured us per step, chunks 1, 2, 4, 8, 12, 16: 37^3 22, 26, 34, 47, -, 53;
 // 85^3 37, 34, 39, 55, -, 67; 125 x 173 x 204 -, 102, 89, 92, -, -; 281^3 648,
 // 477, 400, 373, 370, 375).
-int one_launch_chunk(const fdtd_sim *s, int tiles) {
-    const int nw = rows_waves(s->g.NZ) * tiles;
-    const long slots = 256L * std::max(1, 4 / ((nw + 3) / 4));   // blocks resident at four waves per SIMD
-    const long rows = (s->g.NY + 2 * tiles - 1) / (2 * tiles);
+// columns: blocks per x chunk; slots: blocks resident at once.
+int march_chunk(long columns, int NX, long slots, int most) {
     int best = 1;
     long cost = -1;
-    for (int c : {1, 2, 3, 4, 6, 8, 12}) {
-        const long blocks = rows * ((s->g.NX + c - 1) / c);
+    for (int c : {1, 2, 3, 4, 6, 8, 12, 16, 32}) {
+        if (c > most) break;
+        const long blocks = columns * ((NX + c - 1) / c);
         const long t = (blocks + slots - 1) / slots * (c + 2);
         if (cost < 0 || t < cost) { cost = t; best = c; }
     }
     return best;
+}
+// per_simd: waves per SIMD that the kernel's registers allow.
+int one_launch_chunk(const fdtd_sim *s, int tiles, int per_simd) {
+    const int nw = rows_waves(s->g.NZ) * tiles;
+    const long slots = 256L * std::max(1, per_simd / ((nw + 3) / 4));
+    return march_chunk((s->g.NY + 2 * tiles - 1) / (2 * tiles), s->g.NX, slots, 12);
+}
+
+// x chunk of the general kernels over the whole grid (tj - 1 own rows per block,
+// zt own cells per wave; their registers allow four waves per SIMD).  A block
+// of 8 rows marches a plane in about 6 us: the transposed step of a 69^3 grid
+// takes 216 us in chunks of 32 planes, 38 us by this rule.
+int general_chunk(const fdtd_sim *s, int zt) {
+    const long columns = (long)((s->g.NY + s->tj - 2) / (s->tj - 1)) * ((s->g.NZ + zt - 1) / zt);
+    return march_chunk(columns, s->g.NX, 256L * std::max(1, 4 / ((s->tj + 3) / 4)), 32);
+}
+
+// The pieces of a one-launch step, the costlier ones first, so the launch ends
+// on the cheap ones; equal chunks within a piece.
+template <typename A>
+void add_pieces(const fdtd_sim *s, A &a, int chunk) {
+    auto add = [&](int kind, int c, const int (*b)[4], int n) {
+        for (int q = 0; q < n; q++) {
+            const int len = b[q][1] - b[q][0], parts = (len + c - 1) / c;
+            a.kind[a.n] = kind;
+            a.ich[a.n] = (len + parts - 1) / parts;
+            std::memcpy(a.box[a.n], b[q], sizeof(a.box[0]));
+            a.n++;
+        }
+    };
+    const int side = std::min(chunk, 8);
+    add(3, side, s->cbox4, s->ncorner);
+    add(1, side, s->xbox, s->nxbox);
+    add(2, side, s->ybox, s->nybox);
+    add(0, chunk, &s->cbox, 1);
 }
 
 // The row-blocked kernel (k_step_rows) runs the whole grid with TFSF left
@@ -534,7 +568,7 @@ int plan_rows(fdtd_sim *s) {
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
                           "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
         if (std::getenv(k)) s->one_launch = false;
-    s->one_chunk = one_launch_chunk(s, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1);
+    s->one_chunk = one_launch_chunk(s, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1, 4);
     return FDTD_OK;
 }
 
@@ -798,21 +832,7 @@ int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Dis
     a.r = make_rows(s);
     a.line = l;
     a.r.tiles = s->tiles * rows_waves(s->g.NZ) <= 16 ? s->tiles : 1;
-    // the costlier pieces first, so the launch ends on the cheap ones; equal chunks within a piece
-    auto add = [&](int kind, int chunk, const int (*b)[4], int n) {
-        for (int q = 0; q < n; q++) {
-            const int len = b[q][1] - b[q][0], parts = (len + chunk - 1) / chunk;
-            a.kind[a.n] = kind;
-            a.ich[a.n] = (len + parts - 1) / parts;
-            std::memcpy(a.box[a.n], b[q], sizeof(a.box[0]));
-            a.n++;
-        }
-    };
-    const int side = std::min(s->one_chunk, 8);
-    add(3, side, s->cbox4, s->ncorner);
-    add(1, side, s->xbox, s->nxbox);
-    add(2, side, s->ybox, s->nybox);
-    add(0, s->one_chunk, &s->cbox, 1);
+    add_pieces(s, a, s->one_chunk);
     if (ev0) HIPCHK(s, hipEventRecord(ev0, s->stream));
     HIPCHK(s, launch_step_all(a, s->stream));
     if (ev1) HIPCHK(s, hipEventRecord(ev1, s->stream));
@@ -1028,7 +1048,7 @@ int fdtd_get_info(const fdtd_sim *s, fdtd_grid_info *g) {
         }
     } else {
         g->tile[0] = s->tj;
-        g->tile[1] = s->ichunk;
+        g->tile[1] = s->ichunk ? s->ichunk : general_chunk(s, 63);
     }
     return FDTD_OK;
 }
@@ -1180,7 +1200,7 @@ int adj_alloc(fdtd_sim *s) {
     // needs the row path, wave-edge lanes outside the z slabs of E (their
     // published z weights carry no psi), and the dispersive box grown by two
     // cells inside the clean box and free of z CPML (launch_adj_box_fix)
-    s->adj.rows = false;
+    s->adj.rows = s->adj.one_launch = false;
     if (const char *v = std::getenv("FDTD_ADJ_SCHUNK")) s->adj_schunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_ADJ_RCHUNK")) s->adj_rchunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_ADJ_SCHED")) s->adj_sched = std::min(3, std::max(0, std::atoi(v)));
@@ -1229,6 +1249,13 @@ int adj_alloc(fdtd_sim *s) {
             // the general transposed kernel)
             const char *sl = std::getenv("FDTD_ADJ_SLABS");
             s->adj.rows_slabs = !(sl && std::string(sl) == "general");
+            // every piece in one launch where fdtd_step runs that way too, unless a knob of the
+            // transposed step's schedule or tiles is set
+            s->adj.one_launch = s->one_launch && rows_waves(NZ) * rows_tiles(NZ) <= kAdjAllMaxWaves;
+            for (const char *k : {"FDTD_ADJ_SLABS", "FDTD_ADJ_SCHUNK", "FDTD_ADJ_RCHUNK", "FDTD_ADJ_SCHED", "FDTD_ADJ_TILES",
+                                  "FDTD_ADJ_ROWS", "FDTD_ADJ_CTJ", "FDTD_ADJ_CICH", "FDTD_ADJ_CORNER_ROWS", "FDTD_ADJ_CRCHUNK",
+                                  "FDTD_ADJ_CCHUNK", "FDTD_ADJ_STILES", "FDTD_ADJ_FUSE_INJECT", "FDTD_ADJ_EARLY", "FDTD_ADJ_STJ"})
+                if (std::getenv(k)) s->adj.one_launch = false;
             // amounts of the dispersive-cell correction (schedule 3)
             if (s->nbox > 0) {
                 const long nc = (long)(s->box_n[0] + 2) * (s->box_n[1] + 2) * (s->box_n[2] + 2);
@@ -1301,6 +1328,25 @@ int fdtd_adjoint(fdtd_sim *s, int nsteps, int ckpt, const int r0[3], int nf, con
 
 namespace {
 
+// Row-blocked arguments of a transposed step (the coefficients swapped, the adjoint's psi).
+RowsArgs adj_rows_args(fdtd_sim *s, int pa, int pe, int ph) {
+    const Setup &S = s->S;
+    RowsArgs r = make_rows(s);
+    const long fb = s->fbase;
+    for (int c = 0; c < 3; c++) {
+        r.Ein[c] = (const char *)(s->adj.E[pa][c] - fb); r.Hin[c] = (const char *)(s->adj.H[pa][c] - fb);
+        r.Eout[c] = (char *)(s->adj.E[1 - pa][c] - fb); r.Hout[c] = (char *)(s->adj.H[1 - pa][c] - fb);
+    }
+    r.aux = s->adj.aux_d;
+    r.Chh = 1.0f;
+    r.Che = (float)-S.Ceh;
+    r.Cee = (float)S.Cee;
+    r.Ceh = (float)-S.Che;
+    r.pp = ph;
+    r.pe = pe;
+    return r;
+}
+
 // One transposed step: adjoint level pa -> 1 - pa, psi_E pe, psi_H ph.  On
 // the row path the clean box runs on the row-blocked kernel (variant 3) with
 // the dispersive-cell correction after it, the x and y slabs and the corner
@@ -1333,7 +1379,22 @@ int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, cons
     if (!s->adj.rows) {
         const int full[1][4] = {{0, s->g.NX, 0, s->g.NY}};
         HIPCHK(s, launch_adj_disp(ad, s->stream));
-        HIPCHK(s, launch_adj_step(av, s->tj, s->ichunk, full, 1, s->stream));
+        HIPCHK(s, launch_adj_step(av, s->tj, s->ichunk ? s->ichunk : general_chunk(s, 62), full, 1, s->stream));
+        return FDTD_OK;
+    }
+    if (s->adj.one_launch) {
+        AdjAll a{};
+        a.r = adj_rows_args(s, pa, pe, ph);
+        a.r.tiles = rows_tiles(s->g.NZ);
+        a.ad = ad;
+        add_pieces(s, a, one_launch_chunk(s, a.r.tiles, 3));
+        HIPCHK(s, launch_adj_all(a, s->stream));
+        AdjInject none{};
+        const AdjInject &inj = s->nbox > 0 && next.on ? next : none;
+        if (s->nbox) {
+            HIPCHK(s, launch_adj_box_fix(av, inj, s->stream));
+            *injected = inj.on != 0;
+        }
         return FDTD_OK;
     }
     const bool fork = s->stream2 != nullptr;
@@ -1367,19 +1428,7 @@ int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, cons
         if (sched == 3) HIPCHK(s, launch_adj_box_corr(av, s->adj.corr, s->stream4));
         if (sched >= 2) HIPCHK(s, hipEventRecord(s->ev_line, s->stream4));
     }
-    RowsArgs r = make_rows(s);
-    const long fb = s->fbase;
-    for (int c = 0; c < 3; c++) {
-        r.Ein[c] = (const char *)(s->adj.E[pa][c] - fb); r.Hin[c] = (const char *)(s->adj.H[pa][c] - fb);
-        r.Eout[c] = (char *)(s->adj.E[1 - pa][c] - fb); r.Hout[c] = (char *)(s->adj.H[1 - pa][c] - fb);
-    }
-    r.aux = s->adj.aux_d;
-    r.Chh = 1.0f;
-    r.Che = (float)-S.Ceh;
-    r.Cee = (float)S.Cee;
-    r.Ceh = (float)-S.Che;
-    r.pp = ph;
-    r.pe = pe;
+    RowsArgs r = adj_rows_args(s, pa, pe, ph);
     // x and y slabs on the row-blocked transposed variants (two rows, one row
     // tile, short x chunks so the thin slabs fill the device), or all four
     // slabs on the general transposed kernel
@@ -1779,7 +1828,7 @@ int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
             HIPCHK(s, launch_line(l, s->stream));
             const int full[1][4] = {{0, s->g.NX, 0, s->g.NY}};
             if (step_timing) HIPCHK(s, hipEventRecord(ev0, s->stream));
-            HIPCHK(s, launch_fused_step(d, s->tj, s->ichunk, full, 1, s->stream));
+            HIPCHK(s, launch_fused_step(d, s->tj, s->ichunk ? s->ichunk : general_chunk(s, 63), full, 1, s->stream));
             if (step_timing) HIPCHK(s, hipEventRecord(ev1, s->stream));
         }
         if (step_timing) s->ev_used++;

@@ -355,6 +355,19 @@ long rows_prepare(RowsArgs &ra, int R, int variant);
 long fused_batch_blocks(const Geom &g, int tj, int ichunk, Pieces *pc, int *nkt);
 long fused_pieces(const Geom &g, int tj, int ichunk, const int (*box)[4], int nbox, Pieces *pc, int *nkt);
 
+// The transposed step of every piece and the transposed dispersive update in
+// one launch (kinds as StepAll; r as for variant 3 of launch_step_rows; at most
+// kAdjAllMaxWaves waves per block).  nd and start are filled in by the launcher.
+constexpr int kAdjAllMaxWaves = 12;
+struct AdjAll {
+    RowsArgs r;
+    AdjDispDev ad;
+    int nd, n;
+    int kind[kStepAllPieces], ich[kStepAllPieces], box[kStepAllPieces][4];
+    int start[kStepAllPieces + 1];
+};
+hipError_t launch_adj_all(AdjAll a, hipStream_t st);
+
 // Adjoint: inject dJ/dE^{n+1}(r0), transposed dispersive update, fused transposed step.
 hipError_t launch_adj_inject(float *const E[3], long p0, float ax, float ay, float az, hipStream_t st);
 hipError_t launch_adj_disp(const AdjDispDev &a, hipStream_t st);

@@ -2800,10 +2800,9 @@ __global__ void k_adj_box_add(AdjDev a, AdjInject inj, const float *corr) {
 // given the adjoint of (E^{n+1}, E^n, P^{n+1}, J^{n+1}) returns that of
 // (E^n, E^{n-1}, P^n, J^n), the curl weight Q = a0 Ehat_tot for k_adj_step,
 // and accumulates dJ/drho = Ehat_tot dE'/drho + sum_q Jhat_tot (p3 E' + p4 E + p5 E1).
-__global__ void k_adj_disp(AdjDispDev A) {
+__device__ __forceinline__ void adj_disp_body(const AdjDispDev &A, long idx) {
     const DispDev &d = A.d;
     const long nb = (long)d.n[0] * d.n[1] * d.n[2];
-    const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= nb) return;
     const int bk = (int)(idx % d.n[2]);
     const int bj = (int)((idx / d.n[2]) % d.n[1]);
@@ -2861,6 +2860,34 @@ __global__ void k_adj_disp(AdjDispDev A) {
         }
     }
     if (A.grad && d.rho) A.grad[idx] += gsum;
+}
+
+__global__ void k_adj_disp(AdjDispDev A) { adj_disp_body(A, (long)blockIdx.x * blockDim.x + threadIdx.x); }
+
+// The transposed step of the whole grid in one launch, as k_step_all: the first
+// nd blocks run the transposed dispersive update (it reads the input level, and
+// no piece reads what it writes), the others the pieces.  The dispersive-cell
+// correction follows in a launch of its own.  120 steps forward and back on an
+// 81^3 grid take 10.0 ms with both directions in one launch each, 24.7 ms with
+// their pieces on four streams (121^3 14.9 and 26.0, 221^3 46.2 and 48.9); this
+// launch takes 32 us on the 81^3 grid, bound by the march.
+__global__ __launch_bounds__(64 * 12) void k_adj_all(AdjAll) {
+    const AdjAll &a = batch_item((const AdjAll *)(const CONST_AS AdjAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
+    __shared__ RowsLds<2, true> lds;
+    const int b = (int)blockIdx.x - a.nd;
+    if (b < 0) {
+        adj_disp_body(a.ad, (long)blockIdx.x * (64 * a.r.waves * a.r.tiles) + threadIdx.y * 64 + threadIdx.x);
+        return;
+    }
+    int q = 0;
+    while (q + 1 < a.n && b >= a.start[q + 1]) q++;
+    const int ia = a.box[q][0], ib = a.box[q][1], ja = a.box[q][2], jb = a.box[q][3], ich = a.ich[q], L = b - a.start[q];
+    switch (a.kind[q]) {
+        case 0: rows_piece<2, false, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 1: rows_piece<2, true, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 2: rows_piece<2, false, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        default: rows_piece<2, true, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+    }
 }
 
 __global__ void k_adj_inject(float *ex, float *ey, float *ez, long p0, float ax, float ay, float az) {
@@ -3109,9 +3136,11 @@ hipError_t launch_step_rows(RowsArgs ra, int R, int variant, hipStream_t st) {
     }
 }
 
-hipError_t launch_step_all(StepAll a, hipStream_t st) {
+// Checks the pieces of a one-launch step and fills in the rest; returns the blocks of all pieces or -1.
+template <typename A>
+static long pieces_prepare(A &a, int max_waves) {
     const int W = rows_waves(a.r.NZ);
-    if (a.n < 1 || a.n > kStepAllPieces || a.r.tiles < 1 || a.r.tiles * W > kRowsMaxWaves) return hipErrorInvalidValue;
+    if (a.n < 1 || a.n > kStepAllPieces || a.r.tiles < 1 || a.r.tiles * W > max_waves) return -1;
     a.r.waves = W;
     a.r.nseg = (a.r.NZ + 1 + 64 * W - 3) / (64 * W - 2);
     long total = 0;
@@ -3120,14 +3149,32 @@ hipError_t launch_step_all(StepAll a, hipStream_t st) {
         const bool xg = a.kind[q] & 1, yg = a.kind[q] & 2;
         if (a.kind[q] < 0 || a.kind[q] > 3 || a.ich[q] < 1 || b[0] < 0 || b[1] > a.r.NX || b[0] >= b[1] || b[2] < 0 ||
             b[3] > a.r.NY || b[2] >= b[3])
-            return hipErrorInvalidValue;
-        if ((!xg && (b[0] < 1 || b[1] > a.r.NX - 1)) || (!yg && (b[2] < 1 || b[3] > a.r.NY - 1))) return hipErrorInvalidValue;
+            return -1;
+        if ((!xg && (b[0] < 1 || b[1] > a.r.NX - 1)) || (!yg && (b[2] < 1 || b[3] > a.r.NY - 1))) return -1;
         a.start[q] = (int)total;
         total += rows_pieces_blocks(a.r, b, a.ich[q]);
     }
-    if (total + 1 > 0x7fffffff) return hipErrorInvalidValue;
+    if (total > 0x7fffff00) return -1;
     a.start[a.n] = (int)total;
-    hipLaunchKernelGGL(k_step_all, dim3((unsigned)(total + 1)), dim3(64, W * a.r.tiles), 0, st, a);
+    return total;
+}
+
+hipError_t launch_step_all(StepAll a, hipStream_t st) {
+    const long total = pieces_prepare(a, kRowsMaxWaves);
+    if (total < 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_step_all, dim3((unsigned)(total + 1)), dim3(64, a.r.waves * a.r.tiles), 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_adj_all(AdjAll a, hipStream_t st) {
+    static_assert(sizeof(AdjAll) <= 4096, "kernel arguments");
+    const long total = pieces_prepare(a, kAdjAllMaxWaves);
+    if (total < 0) return hipErrorInvalidValue;
+    const int nt = 64 * a.r.waves * a.r.tiles;
+    const long nb = (long)a.ad.d.n[0] * a.ad.d.n[1] * a.ad.d.n[2];
+    a.nd = (int)((nb + nt - 1) / nt);
+    if (total + a.nd > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_adj_all, dim3((unsigned)(total + a.nd)), dim3(64, a.r.waves * a.r.tiles), 0, st, a);
     return hipGetLastError();
 }
 

@@ -76,6 +76,7 @@ struct fdtd_sim {
         double *grad = nullptr;
         bool rows = false;          // transposed step on the clean box by the row-blocked kernel
         bool rows_slabs = false;    // and on the x and y slabs by its slab variants
+        bool one_launch = false;    // all of them in one launch (k_adj_all)
         float *corr = nullptr;      // amounts of the dispersive-cell correction (6 per cell of the box grown by one)
         unsigned *aux_d = nullptr;  // its table image (adjoint psi pointers)
     } adj;
@@ -90,7 +91,7 @@ struct fdtd_sim {
     // kernels set to 1 on a NaN or Inf (status_d: its device address)
     unsigned *status_h = nullptr, *status_d = nullptr;
     long probe_cell = 0;            // ex probe of the line kernel (main.cu:2728: NX/2, NY/2, NZ/2 - NZ/4)
-    int tj = 8, ichunk = 32;
+    int tj = 8, ichunk = 0;         // general kernel over the whole grid (FDTD_TJ, FDTD_ICHUNK; x chunk 0: by general_chunk)
     int ctj = 4;                    // tile rows of the general kernel on the corner columns (FDTD_CTJ: 4, 8, 16)
     // fused step: row-blocked kernel over the whole grid + TFSF fix-up, or the general kernel alone
     bool use_rows = false;

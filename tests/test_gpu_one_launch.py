@@ -34,3 +34,50 @@ def test_one_launch_gives_the_streams_bits(n, ncpml, sphere, nonlocal_, monkeypa
         out.append([s.get_field(c) for c in range(6)] + [s.flux()["raw"], *s.get_line()])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n,ncpml,block,r0", [((20, 22, 24), 5, (5, 4, 3), "clean"), ((26, 20, 40), 6, (4, 6, 5), "x slab"),
+                                              ((24, 33, 110), 5, (7, 5, 6), "corner"), ((22, 20, 38), 6, (3, 3, 3), "clean")])
+def test_transposed_step_in_one_launch_gives_the_streams_bits(n, ncpml, block, r0, monkeypatch):
+    """k_adj_all (and the last grid, whose wave edge lies in the far z slab: the
+    general transposed kernel) against the transposed step on streams."""
+    p = small_params(fdtd_amd, ncpml=ncpml, sphere=0)
+    p.NCELLX, p.NCELLY, p.NCELLZ = n
+    p.inc_phi = 90.0
+    rng = np.random.default_rng(n[2])
+    rho = rng.uniform(0.1, 0.9, size=block).astype(np.float32)
+    out = []
+    for one in ("1", "0"):
+        monkeypatch.setenv("FDTD_ONE_LAUNCH", one)
+        s = fdtd_amd.Simulation(p)
+        c = [e // 2 for e in s.shape]
+        lo = [a - b // 2 for a, b in zip(c, block)]
+        s.set_design(lo, rho)
+        r = np.random.default_rng(1)
+        for q in range(3):
+            s.set_field(q, (r.standard_normal(s.shape) * 0.1).astype(np.float32))
+        at = {"clean": (c[0], c[1], lo[2] + block[2] + 1), "x slab": (2, c[1], c[2]), "corner": (2, 3, c[2])}[r0]
+        J, g = s.adjoint(50, at, [4e14, 5e14], checkpoint=20)
+        out.append([np.array(J), g] + [s.get_field(q) for q in range(6)])
+    assert np.abs(out[0][1]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [(24, 24, 24), (33, 21, 70), (90, 70, 64)])
+def test_general_kernel_chunks_by_rule(n, monkeypatch):
+    """The general kernel with the x chunk its rule takes against chunks of 32 planes."""
+    monkeypatch.setenv("FDTD_PATH", "general")
+    p = small_params(fdtd_amd)
+    p.NCELLX, p.NCELLY, p.NCELLZ = n
+    out = []
+    for ic in (None, "32"):
+        if ic:
+            monkeypatch.setenv("FDTD_ICHUNK", ic)
+        s = fdtd_amd.Simulation(p)
+        assert s.get_info().fused_path == 0
+        s.step(200)
+        out.append([s.get_field(c) for c in range(6)])
+    for c in range(6):
+        scale = max(np.abs(f).max() for f in (out[1][:3] if c < 3 else out[1][3:]))
+        assert np.abs(out[0][c] - out[1][c]).max() <= 1e-5 * scale, c
