@@ -108,6 +108,7 @@ DispDev make_disp(fdtd_sim *s, int parity) {
     DispDev d{};
     d.g = s->g;
     for (int a = 0; a < 3; a++) { d.lo[a] = s->box_lo[a]; d.n[a] = s->box_n[a]; d.ik_e[a] = s->ik_e[a]; }
+    d.per = S.P.periodic_xy ? 1 : 0;
     for (int c = 0; c < 3; c++) {
         d.id[c] = s->disp_id[c];
         for (int q = 0; q < 8; q++) d.st[c][q] = s->disp_st[c][q];
@@ -810,7 +811,7 @@ int launch_rows_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Di
     }
     const bool merge_samp = tf_early && samp && d.sample_row && (s->nbox <= 0 || disp_early) && sample_in_clean(s);
     if (tf_early) {
-        if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, merge_disp ? dd : nullptr, merge_samp, s->stream));
+        if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, true, merge_disp ? dd : nullptr, merge_samp, s->stream));
         else HIPCHK(s, launch_tfsf_fix(d, s->stream));
         *disp_done = *disp_done || merge_disp;
         *samp_done = merge_samp;
@@ -839,7 +840,7 @@ int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Dis
     // the box and the sample ride with the TFSF fix-up where their cells are apart from it
     const bool merge_disp = dd && !s->S.hydro && disp_in_clean(s);
     const bool merge_samp = samp && d.sample_row && (s->nbox <= 0 || disp_in_clean(s)) && sample_in_clean(s);
-    if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, merge_disp ? dd : nullptr, merge_samp, s->stream));
+    if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, true, merge_disp ? dd : nullptr, merge_samp, s->stream));
     else HIPCHK(s, launch_tfsf_fix(d, s->stream));
     *disp_done = merge_disp;
     *samp_done = merge_samp;
@@ -1359,7 +1360,6 @@ RowsArgs adj_rows_args(fdtd_sim *s, int pa, int pe, int ph) {
 // it is on (the caller turns it on only where the objective cell lies in the
 // clean box, which no side launch writes); *injected reports whether it was.
 int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, const AdjInject &next, bool *injected) {
-    const Setup &S = s->S;
     AdjDev av{};
     const StepDev sd = make_step(s, false);
     av.g = sd.g; av.c = sd.c;
@@ -1714,7 +1714,7 @@ static StepDev inplace_step(fdtd_sim *s, bool tfsf) {
 int fdtd_update_h(fdtd_sim *s) {
     if (!s) return FDTD_ERR_INVALID;
     const StepDev d = inplace_step(s, false);
-    HIPCHK(s, s->S.P.periodic_xy ? launch_periodic_h(d, s->stream) : launch_split_h(d, s->stream));
+    HIPCHK(s, s->S.P.periodic_xy ? launch_periodic_h(d, nullptr, s->stream) : launch_split_h(d, s->stream));
     return FDTD_OK;
 }
 
@@ -1741,13 +1741,19 @@ int fdtd_update_e(fdtd_sim *s) {
     return FDTD_OK;
 }
 
-int fdtd_dft_accumulate(fdtd_sim *s) {
-    if (!s) return FDTD_ERR_INVALID;
-    int rc = FDTD_OK;
+// The point monitor's sample of the current E, at the end of an in-place step.
+static int record_monitor(fdtd_sim *s) {
     if (s->mon && s->t - s->mon_t0 < s->mon_cap) {
         const float *E1[3] = {s->E[s->p][0], s->E[s->p][1], s->E[s->p][2]};
         HIPCHK(s, launch_probe(E1, s->mon_p, s->mon + 3 * (size_t)(s->t - s->mon_t0), s->stream));
     }
+    return FDTD_OK;
+}
+
+int fdtd_dft_accumulate(fdtd_sim *s) {
+    if (!s) return FDTD_ERR_INVALID;
+    int rc = FDTD_OK;
+    if (int rm = record_monitor(s)) return rm;
     if (sampling_step(s)) {
         StepDev d = make_step(s, false);
         for (int c = 0; c < 3; c++) { d.Ein[c] = s->E[s->p][c]; d.Hin[c] = s->H[s->p][c]; }
@@ -1759,19 +1765,26 @@ int fdtd_dft_accumulate(fdtd_sim *s) {
     return rc;
 }
 
-// One periodic step (Periodic_XY): line, E ghosts + H with the source
-// plane, H ghosts + E with the source plane, dispersive box, monitors; the
-// reference's order (main.cu:2724-2934) with its corrections folded into the
-// updates.  Fields update in place.
+// One periodic step (Periodic_XY): H with the source plane and the line, E
+// with the source plane, dispersive box and monitors; the reference's order
+// (main.cu:2724-2934) with its corrections folded into the updates.  Fields
+// update in place.  The layer's cells lie strictly between the two monitor
+// planes, so the sample shares the box's launch.
 static int periodic_step(fdtd_sim *s) {
     const LineDev l = make_line(s);
-    HIPCHK(s, launch_line(l, s->stream));
-    const StepDev d = inplace_step(s, true);
-    HIPCHK(s, launch_periodic_h(d, s->stream));
+    StepDev d = inplace_step(s, true);
+    HIPCHK(s, launch_periodic_h(d, &l, s->stream));
     HIPCHK(s, launch_periodic_e(d, s->stream));
     s->le ^= 1;
-    if (s->nbox) HIPCHK(s, launch_dispersive(make_disp(s, s->p), s->stream));
-    return fdtd_dft_accumulate(s);
+    const bool samp = sampling_step(s);
+    if (samp) d.sample_row = s->X + (size_t)s->slot * s->mtot;
+    DispDev dd{};
+    if (s->nbox) dd = make_disp(s, s->p);
+    HIPCHK(s, launch_post(d, false, s->nbox ? &dd : nullptr, samp, s->stream));
+    if (int rc = record_monitor(s)) return rc;
+    const int rc = samp ? after_sample(s) : FDTD_OK;
+    s->t++;
+    return rc;
 }
 
 int fdtd_step(fdtd_sim *s, int nsteps) {

@@ -106,6 +106,7 @@ struct DispDev {
     // state per component, box-dense SoA: 0 E^n, 1 E^{n-1}, then per pole q
     // (0 Drude, 1-2 CP) P~^n at 2+2q and J~^n = P~^n - P~^{n-1} at 3+2q, P~ = P/eps0
     float *st[3][8];
+    int per;                        // periodic x, y: H at i-1 and j-1 across the edges
     const float *H[3];              // H^{n+1/2}
     float *E[3];                    // output field (E^{n+1} written at dispersive cells)
     const float *ik_e[3];
@@ -272,10 +273,10 @@ long rows_pieces_blocks(const RowsArgs &r, const int box[4], int ichunk);
 // box[q] = {ia, ib, ja, jb}; one to four disjoint boxes.
 hipError_t launch_fused_step(const StepDev &s, int tj, int ichunk, const int (*box)[4], int nbox, hipStream_t st);
 hipError_t launch_split_h(const StepDev &s, hipStream_t st);
-// Periodic x, y: E ghost wrap + H update (with the near z plane of the TFSF
-// when s.tfsf_on), H ghost wrap + E update, and the plane corrections alone
-// for the split path.  In place: Ein == Eout, Hin == Hout.
-hipError_t launch_periodic_h(const StepDev &s, hipStream_t st);
+// Periodic x, y: H update (with the near z plane of the TFSF when s.tfsf_on,
+// and the 1D line when given), E update, and the plane corrections alone for
+// the split path.  In place: Ein == Eout, Hin == Hout.
+hipError_t launch_periodic_h(const StepDev &s, const LineDev *line, hipStream_t st);
 hipError_t launch_periodic_e(const StepDev &s, hipStream_t st);
 hipError_t launch_periodic_tfsf(const StepDev &s, hipStream_t st);
 hipError_t launch_split_e(const StepDev &s, hipStream_t st);
@@ -284,10 +285,10 @@ hipError_t launch_tfsf_split(const StepDev &s, hipStream_t st);
 hipError_t launch_tfsf_fix(const StepDev &s, hipStream_t st);
 hipError_t launch_line(const LineDev &l, hipStream_t st);
 hipError_t launch_dispersive(const DispDev &d, hipStream_t st);
-// launch_tfsf_fix, launch_dispersive (Drude + CP, when d is given) and, with
+// launch_tfsf_fix (with tfsf), launch_dispersive (Drude + CP, when d is given) and, with
 // sample, the DFT sample of s.Eout / s.Hout into s.sample_row, in one launch;
 // only for cell sets that are pairwise disjoint.
-hipError_t launch_post(const StepDev &s, const DispDev *d, bool sample, hipStream_t st);
+hipError_t launch_post(const StepDev &s, bool tfsf, const DispDev *d, bool sample, hipStream_t st);
 hipError_t launch_dft_sample_split(const StepDev &s, hipStream_t st);
 hipError_t launch_twiddle(double *W, const int *t_slot_host, int K, int nvalid, int F, const double *freq,
                           double dt, hipStream_t st);

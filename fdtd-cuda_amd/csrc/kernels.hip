@@ -1483,14 +1483,57 @@ __global__ __launch_bounds__(64 * MW) __attribute__((amdgpu_waves_per_eu(R == 2 
     rows_body<R, XG, YG, ADJ>(ra, ra.xcd ? xcd_order(blockIdx.x, ra.start[ra.npiece]) : (int)blockIdx.x);
 }
 
+// ----------------------------------------------------------------- 1D incident line
+
+// One block: h_inc (main.cu:2328-2336), e_inc (main.cu:2280-2326) into the
+// other buffer, first-order Mur ends and the additive source (main.cu:2831-2859).
+__device__ __forceinline__ void line_body(const LineDev &l, int t, int tid, int nthreads) {
+    const int L = l.L;
+    for (int i = tid; i < L - 1; i += nthreads) l.h[i] = l.h[i] - l.ch * (l.e_old[i + 1] - l.e_old[i]);
+    __syncthreads();
+    for (int i = tid + 1; i < L - 1; i += nthreads) l.e_new[i] = l.e_old[i] - l.ce * (l.h[i] - l.h[i - 1]);
+    __syncthreads();
+    if (tid == 0) {
+        const double e1 = l.mur[0], e2 = l.mur[1];
+        l.e_new[0] = e1 + l.mur_coef * (l.e_new[1] - l.e_old[0]);
+        l.e_new[L - 1] = e2 + l.mur_coef * (l.e_new[L - 2] - l.e_old[L - 1]);
+        l.mur[0] = l.e_new[1];
+        l.mur[1] = l.e_new[L - 2];
+        double pulse;
+        if (l.static_field) {
+            pulse = (t < 1000) ? l.amp * t / 1000.0 : l.amp;  // main.cu:2852-2857
+        } else {
+            // powf on a float-converted argument, as the reference (main.cu:2848)
+            const float b = (float)(((double)t - l.delay) / l.width);
+            const float b2 = b * b;
+            pulse = l.amp * exp(-(double)b2 / 2.0) * sin(l.w0dt * (double)t);
+        }
+        l.e_new[l.src] += pulse;
+        if (l.probe && l.status && !__builtin_isfinite(*l.probe)) *l.status = 1u;
+    }
+}
+
 // ----------------------------------------------------------------- split path kernels
 
-__global__ void k_split_h(StepDev s) {
+// Cell of a thread of the whole-grid kernels: 256 consecutive cells (k fastest)
+// of the y-z plane blockIdx.y per block, so no wave is a partly filled piece of
+// one row.  A launch is bound by the latency of its two rounds of waves: 97^3
+// cells 18.0 -> 16.1 us (split path), 75 x 64 x 225 cells 15.9 -> 13.2 us
+// (periodic; its two ghost-layer launches of 3 and 4 us and the line's 4 us are
+// gone besides), against blocks of 64 cells of a row.
+__device__ __forceinline__ bool plane_cell(const Geom &g, int &i, int &j, int &k) {
+    const int idx = (int)(blockIdx.x * 256 + threadIdx.x);
+    i = (int)blockIdx.y;
+    j = idx / g.NZ;
+    k = idx - j * g.NZ;
+    return j < g.NY;
+}
+static dim3 plane_grid(const Geom &g) { return dim3((unsigned)(((long)g.NY * g.NZ + 255) / 256), g.NX); }
+
+__global__ __launch_bounds__(256) void k_split_h(StepDev s) {
     const Geom &g = s.g;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    const int i = blockIdx.z;
-    if (k >= g.NZ) return;
+    int i, j, k;
+    if (!plane_cell(g, i, j, k)) return;
     const long p = gidx(g, i, j, k);
     ENbr e;
     e.ex = s.Ein[0][p]; e.ey = s.Ein[1][p]; e.ez = s.Ein[2][p];
@@ -1502,12 +1545,10 @@ __global__ void k_split_h(StepDev s) {
     s.Hout[0][p] = hx; s.Hout[1][p] = hy; s.Hout[2][p] = hz;
 }
 
-__global__ void k_split_e(StepDev s) {
+__global__ __launch_bounds__(256) void k_split_e(StepDev s) {
     const Geom &g = s.g;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;
-    const int i = blockIdx.z;
-    if (k >= g.NZ) return;
+    int i, j, k;
+    if (!plane_cell(g, i, j, k)) return;
     const long p = gidx(g, i, j, k);
     HNbr h;
     h.hx = s.Hin[0][p]; h.hy = s.Hin[1][p]; h.hz = s.Hin[2][p];
@@ -1523,57 +1564,26 @@ __global__ void k_split_e(StepDev s) {
 //
 // x and y wrap around (the i == NCELLX-1 / j == NCELLY-1 and i == 0 / j == 0
 // branches of UPDATE_h* and UPDATE_e*, main.cu:781-1044, 1067-1912, real
-// build): every column is updated, the neighbours across the x and y edges
-// are read from the ghost layers, which k_wrap_e / k_wrap_h fill with the
-// opposite face before each half step, so the stencils need no wrap logic;
-// CPML along z only.  With tfsf_on the near z plane of the TFSF box adds the
-// incident wave (CORRECT_Z near face, main.cu:638-697; Periodic_XY skips the
-// far face, main.cu:698): H at k0-1 after its update, E^n at k0 before.
-// Updates run in place (E and H of the current level), as the split path.
+// build): every column is updated, and the neighbours across the x and y edges
+// are read from the opposite face (the ghost layers are not used); CPML along
+// z only.  With tfsf_on the near z plane of the TFSF box adds the incident wave
+// (CORRECT_Z near face, main.cu:638-697; Periodic_XY skips the far face,
+// main.cu:698): H at k0-1 after its update, E^n at k0 before.  Updates run in
+// place (E and H of the current level), as the split path.
+__device__ __forceinline__ long up_wrapped(int x, int n, long pitch) { return x + 1 < n ? pitch : -(long)(n - 1) * pitch; }
+__device__ __forceinline__ long down_wrapped(int x, int n, long pitch) { return x > 0 ? -pitch : (long)(n - 1) * pitch; }
 
-// E ghosts for the H update: plane x = NX <- x = 0 (rows 0..NY-1), then row
-// y = NY <- y = 0 for x = 0..NX (the corner follows from the ghost plane).
-__global__ void k_wrap_e(float *ex, float *ey, float *ez, Geom g) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int u = blockIdx.y;
-    if (k >= g.NZ) return;
-    float *f[3] = {ex, ey, ez};
-    if (blockIdx.z == 0) {
-        if (u >= g.NY) return;
-        const long d = gidx(g, g.NX, u, k), src = gidx(g, 0, u, k);
-        for (int c = 0; c < 3; c++) f[c][d] = f[c][src];
-    } else {
-        if (u > g.NX) return;
-        const long d = gidx(g, u, g.NY, k), src = gidx(g, u == g.NX ? 0 : u, 0, k);
-        for (int c = 0; c < 3; c++) f[c][d] = f[c][src];
-    }
-}
-
-// H ghosts for the E update: plane x = -1 <- x = NX-1, row y = -1 <- y = NY-1
-// for x = -1..NX-1.
-__global__ void k_wrap_h(float *hx, float *hy, float *hz, Geom g) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int u = blockIdx.y;
-    if (k >= g.NZ) return;
-    float *f[3] = {hx, hy, hz};
-    if (blockIdx.z == 0) {
-        if (u >= g.NY) return;
-        const long d = gidx(g, -1, u, k), src = gidx(g, g.NX - 1, u, k);
-        for (int c = 0; c < 3; c++) f[c][d] = f[c][src];
-    } else {
-        if (u > g.NX) return;
-        const int i = u - 1;
-        const long d = gidx(g, i, -1, k), src = gidx(g, i < 0 ? g.NX - 1 : i, g.NY - 1, k);
-        for (int c = 0; c < 3; c++) f[c][d] = f[c][src];
-    }
-}
-
-__global__ void k_per_h(StepDev s) {
+// The last plane of blocks runs the 1D line when it is given (line.e_new set):
+// the H update reads e_inc^n, which the line kernel does not write.
+__global__ __launch_bounds__(256) void k_per_h(StepDev s, LineDev line) {
     const Geom &g = s.g;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y, i = blockIdx.z;
-    if (k >= g.NZ) return;
-    const long p = gidx(g, i, j, k);
+    if ((int)blockIdx.y == g.NX) {
+        if (blockIdx.x == 0) line_body(line, line.t, threadIdx.x, 256);
+        return;
+    }
+    int i, j, k;
+    if (!plane_cell(g, i, j, k)) return;
+    const long p = gidx(g, i, j, k), pj = p + up_wrapped(j, g.NY, g.sz), pi = p + up_wrapped(i, g.NX, g.sxy);
     const CpmlDev &cz = s.cp[2];
     const float Chh = s.c.Chh, Che = s.c.Che;
     const float ikx = s.cp[0].ik_h[i], iky = s.cp[1].ik_h[j];
@@ -1582,29 +1592,28 @@ __global__ void k_per_h(StepDev s) {
         const int lz = h_layer(cz, k), Lz = 2 * cz.Nc;
         const float ikz = cz.ik_h[k];
         // hx (main.cu:781-865)
-        const float dEy = ey[p + 1] - ey[p], dEzj = ez[p + g.sz] - ez[p];
+        const float dEy = ey[p + 1] - ey[p], dEzj = ez[pj] - ez[p];
         float h = Chh * s.Hin[0][p] + Che * (dEy * ikz - dEzj * iky);
         if (lz >= 0) h += Che * psi_step(s.psiH_in.p[0], s.psiH_out.p[0], zslab(g, Lz, i, j, lz), cz.bh[lz], cz.ch[lz], dEy, true);
         if (s.tfsf_on) h += tfsf_term_ct<false, 0, 2>(s.tf, i, j, k);
         s.Hout[0][p] = h;
         // hy (main.cu:877-948)
-        const float dEzi = ez[p + g.sxy] - ez[p], dEx = ex[p + 1] - ex[p];
+        const float dEzi = ez[pi] - ez[p], dEx = ex[p + 1] - ex[p];
         h = Chh * s.Hin[1][p] + Che * (dEzi * ikx - dEx * ikz);
         if (lz >= 0) h -= Che * psi_step(s.psiH_in.p[2], s.psiH_out.p[2], zslab(g, Lz, i, j, lz), cz.bh[lz], cz.ch[lz], dEx, true);
         if (s.tfsf_on) h += tfsf_term_ct<false, 1, 2>(s.tf, i, j, k);
         s.Hout[1][p] = h;
     }
     // hz (main.cu:962-1044), every k
-    const float dExj = ex[p + g.sz] - ex[p], dEyi = ey[p + g.sxy] - ey[p];
+    const float dExj = ex[pj] - ex[p], dEyi = ey[pi] - ey[p];
     s.Hout[2][p] = Chh * s.Hin[2][p] + Che * (dExj * iky - dEyi * ikx);
 }
 
-__global__ void k_per_e(StepDev s) {
+__global__ __launch_bounds__(256) void k_per_e(StepDev s) {
     const Geom &g = s.g;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y, i = blockIdx.z;
-    if (k >= g.NZ - 1) return;
-    const long p = gidx(g, i, j, k);
+    int i, j, k;
+    if (!plane_cell(g, i, j, k) || k >= g.NZ - 1) return;
+    const long p = gidx(g, i, j, k), pj = p + down_wrapped(j, g.NY, g.sz), pi = p + down_wrapped(i, g.NX, g.sxy);
     const CpmlDev &cz = s.cp[2];
     const float Cee = s.c.Cee, Ceh = s.c.Ceh;
     const float ikx = s.cp[0].ik_e[i], iky = s.cp[1].ik_e[j];
@@ -1615,20 +1624,20 @@ __global__ void k_per_e(StepDev s) {
         // ex (main.cu:1067-1170)
         float eo = s.Ein[0][p];
         if (s.tfsf_on) eo += tfsf_term_ct<true, 0, 2>(s.tf, i, j, k);
-        const float dHzj = hz[p] - hz[p - g.sz], dHy = hy[p] - hy[p - 1];
+        const float dHzj = hz[p] - hz[pj], dHy = hy[p] - hy[p - 1];
         float e = Cee * eo + Ceh * (dHzj * iky - dHy * ikz);
         if (lz >= 0) e -= Ceh * psi_step(s.psiE.p[0], s.psiE.p[0], zslab(g, Lz, i, j, lz), cz.be[lz], cz.ce[lz], dHy, true);
         s.Eout[0][p] = e;
         // ey (main.cu:1359-1475)
         eo = s.Ein[1][p];
         if (s.tfsf_on) eo += tfsf_term_ct<true, 1, 2>(s.tf, i, j, k);
-        const float dHx = hx[p] - hx[p - 1], dHzi = hz[p] - hz[p - g.sxy];
+        const float dHx = hx[p] - hx[p - 1], dHzi = hz[p] - hz[pi];
         e = Cee * eo + Ceh * (dHx * ikz - dHzi * ikx);
         if (lz >= 0) e += Ceh * psi_step(s.psiE.p[2], s.psiE.p[2], zslab(g, Lz, i, j, lz), cz.be[lz], cz.ce[lz], dHx, true);
         s.Eout[1][p] = e;
     }
     // ez (main.cu:1663-1766), k < NZ-1
-    const float dHyi = hy[p] - hy[p - g.sxy], dHxj = hx[p] - hx[p - g.sz];
+    const float dHyi = hy[p] - hy[pi], dHxj = hx[p] - hx[pj];
     s.Eout[2][p] = Cee * s.Ein[2][p] + Ceh * (dHyi * ikx - dHxj * iky);
 }
 
@@ -1646,23 +1655,33 @@ __global__ void k_per_tfsf(StepDev s) {
     s.Eout[1][pe] += tfsf_term_ct<true, 1, 2>(s.tf, i, j, k0);
 }
 
-// CORRECT_X/Y/Z in place over the bounding box of the TFSF planes.
-__global__ void k_tfsf_split(StepDev s) {
+// CORRECT_X/Y/Z in place: per normal axis the planes t0-1, t0 and t1 over
+// [t0-1, t1] of the other two, a cell on planes of several axes taken by the
+// lowest one.  Only the planes' cells are visited (the box they bound has
+// some 20 times as many; a 97^3 grid 13.4 -> 5.5 us).
+__global__ __launch_bounds__(256) void k_tfsf_split(StepDev s, int nbx, int span) {
     const TfsfDev &t = s.tf;
-    const int k = t.t0[2] - 1 + blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = t.t0[1] - 1 + blockIdx.y;
-    const int i = t.t0[0] - 1 + blockIdx.z;
-    if (k > t.t1[2]) return;
-    const bool onx = i == t.t0[0] - 1 || i == t.t0[0] || i == t.t1[0];
-    const bool ony = j == t.t0[1] - 1 || j == t.t0[1] || j == t.t1[1];
-    const bool onz = k == t.t0[2] - 1 || k == t.t0[2] || k == t.t1[2];
-    if (!(onx || ony || onz)) return;
+    const int L = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (L >= nbx * span * 9) return;
+    const int u0 = (L / nbx) % span, v0 = L % nbx * 64 + lane, pq = L / (nbx * span), a = pq / 3, q = pq % 3;
+    const int b0 = a == 0 ? 1 : 0, b1 = a == 2 ? 1 : 2;   // other axes, b1 fastest in memory
+    const int u = pick3(b0, t.t0[0], t.t0[1], t.t0[2]) - 1 + u0, v = pick3(b1, t.t0[0], t.t0[1], t.t0[2]) - 1 + v0;
+    if (u > pick3(b0, t.t1[0], t.t1[1], t.t1[2]) || v > pick3(b1, t.t1[0], t.t1[1], t.t1[2])) return;
+    const int t0a = pick3(a, t.t0[0], t.t0[1], t.t0[2]), t1a = pick3(a, t.t1[0], t.t1[1], t.t1[2]);
+    const int xa = q == 0 ? t0a - 1 : (q == 1 ? t0a : t1a);
+    const int i = a == 0 ? xa : u, j = a == 1 ? xa : (a == 0 ? u : v), k = a == 2 ? xa : v;
+    auto on = [&](int ax, int x) {
+        const int lo = pick3(ax, t.t0[0], t.t0[1], t.t0[2]), hi = pick3(ax, t.t1[0], t.t1[1], t.t1[2]);
+        return x == lo - 1 || x == lo || x == hi;
+    };
+    if ((a >= 1 && on(0, i)) || (a >= 2 && on(1, j))) return;
     const long p = gidx(s.g, i, j, k);
+    const float dh[3] = {tfsf_h_ct<0>(t, i, j, k), tfsf_h_ct<1>(t, i, j, k), tfsf_h_ct<2>(t, i, j, k)};
+    const float de[3] = {tfsf_e_ct<0>(t, i, j, k), tfsf_e_ct<1>(t, i, j, k), tfsf_e_ct<2>(t, i, j, k)};
+#pragma unroll
     for (int c = 0; c < 3; c++) {
-        float dh = tfsf_h(t, c, i, j, k);
-        if (dh != 0.f) s.Hout[c][p] += dh;
-        float de = tfsf_e(t, c, i, j, k);
-        if (de != 0.f) s.Eout[c][p] += de;
+        if (dh[c] != 0.f) s.Hout[c][p] += dh[c];
+        if (de[c] != 0.f) s.Eout[c][p] += de[c];
     }
 }
 
@@ -1761,13 +1780,15 @@ __device__ __forceinline__ void disp_body(const DispDev &d, long idx) {
     const int i = d.lo[0] + bi, j = d.lo[1] + bj, k = d.lo[2] + bk;
     const Geom &g = d.g;
     const long p = gidx(g, i, j, k);
+    // H at j-1 and i-1 (periodic runs: across the edge)
+    const long pj = p + (d.per ? down_wrapped(j, g.NY, g.sz) : -g.sz), pi = p + (d.per ? down_wrapped(i, g.NX, g.sxy) : -g.sxy);
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         if (!d.id[c][idx]) continue;
         float curl;
-        if (c == 0) curl = (d.H[2][p] - d.H[2][p - g.sz]) * d.ik_e[1][j] - (d.H[1][p] - d.H[1][p - 1]) * d.ik_e[2][k];
-        else if (c == 1) curl = (d.H[0][p] - d.H[0][p - 1]) * d.ik_e[2][k] - (d.H[2][p] - d.H[2][p - g.sxy]) * d.ik_e[0][i];
-        else curl = (d.H[1][p] - d.H[1][p - g.sxy]) * d.ik_e[0][i] - (d.H[0][p] - d.H[0][p - g.sz]) * d.ik_e[1][j];
+        if (c == 0) curl = (d.H[2][p] - d.H[2][pj]) * d.ik_e[1][j] - (d.H[1][p] - d.H[1][p - 1]) * d.ik_e[2][k];
+        else if (c == 1) curl = (d.H[0][p] - d.H[0][p - 1]) * d.ik_e[2][k] - (d.H[2][p] - d.H[2][pi]) * d.ik_e[0][i];
+        else curl = (d.H[1][p] - d.H[1][pi]) * d.ik_e[0][i] - (d.H[0][p] - d.H[0][pj]) * d.ik_e[1][j];
         float *const *st = d.st[c];
         const float en = st[0][idx], en1 = st[1][idx];
         float P[3], J[3];
@@ -2050,35 +2071,7 @@ __global__ void k_disp_sync(DispDev d, int from_field) {
     }
 }
 
-// ----------------------------------------------------------------- 1D incident line
-
-// One block: h_inc (main.cu:2328-2336), e_inc (main.cu:2280-2326) into the
-// other buffer, first-order Mur ends and the additive source (main.cu:2831-2859).
-__device__ __forceinline__ void line_body(const LineDev &l, int t, int tid, int nthreads) {
-    const int L = l.L;
-    for (int i = tid; i < L - 1; i += nthreads) l.h[i] = l.h[i] - l.ch * (l.e_old[i + 1] - l.e_old[i]);
-    __syncthreads();
-    for (int i = tid + 1; i < L - 1; i += nthreads) l.e_new[i] = l.e_old[i] - l.ce * (l.h[i] - l.h[i - 1]);
-    __syncthreads();
-    if (tid == 0) {
-        const double e1 = l.mur[0], e2 = l.mur[1];
-        l.e_new[0] = e1 + l.mur_coef * (l.e_new[1] - l.e_old[0]);
-        l.e_new[L - 1] = e2 + l.mur_coef * (l.e_new[L - 2] - l.e_old[L - 1]);
-        l.mur[0] = l.e_new[1];
-        l.mur[1] = l.e_new[L - 2];
-        double pulse;
-        if (l.static_field) {
-            pulse = (t < 1000) ? l.amp * t / 1000.0 : l.amp;  // main.cu:2852-2857
-        } else {
-            // powf on a float-converted argument, as the reference (main.cu:2848)
-            const float b = (float)(((double)t - l.delay) / l.width);
-            const float b2 = b * b;
-            pulse = l.amp * exp(-(double)b2 / 2.0) * sin(l.w0dt * (double)t);
-        }
-        l.e_new[l.src] += pulse;
-        if (l.probe && l.status && !__builtin_isfinite(*l.probe)) *l.status = 1u;
-    }
-}
+// ----------------------------------------------------------------- 1D line alone, one-launch step
 
 __global__ __launch_bounds__(1024) void k_line(LineDev l) { line_body(l, l.t, threadIdx.x, blockDim.x); }
 
@@ -3253,23 +3246,16 @@ hipError_t launch_probe(const float *const E[3], long p0, float *out, hipStream_
     return hipGetLastError();
 }
 
-hipError_t launch_periodic_h(const StepDev &s, hipStream_t st) {
-    const Geom &g = s.g;
-    const dim3 wg((g.NZ + 63) / 64, g.NX + 1 > g.NY ? g.NX + 1 : g.NY, 2), block(64);
-    hipLaunchKernelGGL(k_wrap_e, wg, block, 0, st, const_cast<float *>(s.Ein[0]), const_cast<float *>(s.Ein[1]),
-                       const_cast<float *>(s.Ein[2]), g);
-    const dim3 grid((g.NZ + 63) / 64, g.NY, g.NX);
-    hipLaunchKernelGGL(k_per_h, grid, block, 0, st, s);
+hipError_t launch_periodic_h(const StepDev &s, const LineDev *line, hipStream_t st) {
+    const LineDev none{};
+    dim3 grid = plane_grid(s.g);
+    if (line) grid.y++;
+    hipLaunchKernelGGL(k_per_h, grid, dim3(256), 0, st, s, line ? *line : none);
     return hipGetLastError();
 }
 
 hipError_t launch_periodic_e(const StepDev &s, hipStream_t st) {
-    const Geom &g = s.g;
-    const dim3 wg((g.NZ + 63) / 64, g.NX + 1 > g.NY ? g.NX + 1 : g.NY, 2), block(64);
-    hipLaunchKernelGGL(k_wrap_h, wg, block, 0, st, const_cast<float *>(s.Hin[0]), const_cast<float *>(s.Hin[1]),
-                       const_cast<float *>(s.Hin[2]), g);
-    const dim3 grid((g.NZ + 63) / 64, g.NY, g.NX);
-    hipLaunchKernelGGL(k_per_e, grid, block, 0, st, s);
+    hipLaunchKernelGGL(k_per_e, plane_grid(s.g), dim3(256), 0, st, s);
     return hipGetLastError();
 }
 
@@ -3280,22 +3266,21 @@ hipError_t launch_periodic_tfsf(const StepDev &s, hipStream_t st) {
 }
 
 hipError_t launch_split_h(const StepDev &s, hipStream_t st) {
-    dim3 grid((s.g.NZ + 63) / 64, s.g.NY, s.g.NX), block(64);
-    hipLaunchKernelGGL(k_split_h, grid, block, 0, st, s);
+    hipLaunchKernelGGL(k_split_h, plane_grid(s.g), dim3(256), 0, st, s);
     return hipGetLastError();
 }
 
 hipError_t launch_split_e(const StepDev &s, hipStream_t st) {
-    dim3 grid((s.g.NZ + 63) / 64, s.g.NY, s.g.NX), block(64);
-    hipLaunchKernelGGL(k_split_e, grid, block, 0, st, s);
+    hipLaunchKernelGGL(k_split_e, plane_grid(s.g), dim3(256), 0, st, s);
     return hipGetLastError();
 }
 
 hipError_t launch_tfsf_split(const StepDev &s, hipStream_t st) {
     const TfsfDev &t = s.tf;
-    const int nk = t.t1[2] - t.t0[2] + 2, nj = t.t1[1] - t.t0[1] + 2, ni = t.t1[0] - t.t0[0] + 2;
-    dim3 grid((nk + 63) / 64, nj, ni), block(64);
-    hipLaunchKernelGGL(k_tfsf_split, grid, block, 0, st, s);
+    int span = 0;
+    for (int a = 0; a < 3; a++) span = max(span, t.t1[a] - t.t0[a] + 2);
+    const int nbx = (span + 63) / 64;
+    hipLaunchKernelGGL(k_tfsf_split, dim3((unsigned)(((long)nbx * span * 9 + 3) / 4)), dim3(256), 0, st, s, nbx, span);
     return hipGetLastError();
 }
 
@@ -3308,15 +3293,16 @@ hipError_t launch_tfsf_fix(const StepDev &s, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_post(const StepDev &s, const DispDev *d, bool sample, hipStream_t st) {
+hipError_t launch_post(const StepDev &s, bool tfsf, const DispDev *d, bool sample, hipStream_t st) {
     static_assert(sizeof(StepDev) + sizeof(DispDev) + 32 <= 4096, "kernel arguments");
     const TfsfDev &t = s.tf;
     int span = 0;
     for (int a = 0; a < 3; a++) span = max(span, t.t1[a] - t.t0[a] + 3);
     const int nbx = (span + 63) / 64;
     const long nb = d ? (long)d->n[0] * d->n[1] * d->n[2] : 0;
-    const long nd = (nb + 255) / 256, nt = ((long)nbx * span * 12 + 3) / 4, ns = sample ? (s.fd.mE + 255) / 256 : 0;
+    const long nd = (nb + 255) / 256, nt = tfsf ? ((long)nbx * span * 12 + 3) / 4 : 0, ns = sample ? (s.fd.mE + 255) / 256 : 0;
     if (nd + nt + ns > 0x7fffffff) return hipErrorInvalidValue;
+    if (nd + nt + ns == 0) return hipSuccess;
     const DispDev none{};
     hipLaunchKernelGGL(k_post, dim3((unsigned)(nd + nt + ns)), dim3(256), 0, st, s, d ? *d : none, (int)nd, nbx, span,
                        (int)nt, (int)ns);
