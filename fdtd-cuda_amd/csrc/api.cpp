@@ -2105,8 +2105,23 @@ int fdtd_reflectance(fdtd_sim *s, double *R, double *T, double *ref_r, double *r
     std::vector<double> raw(12 * (size_t)F);
     if (int rc = fdtd_flux(s, nullptr, nullptr, nullptr, raw.data())) return rc;
     // the incident wave at the source plane, sampled like the monitors: the same
-    // FP64 line replayed on the host for the steps run so far
-    const std::vector<std::complex<double>> inc = fdtd::line_dft(S, s->t);
+    // FP64 line run again for the steps so far, on the device in the staging
+    // buffer where the line fits one block's LDS and the steps the buffer
+    std::vector<std::complex<double>> inc(F, 0.0);
+    const long need = line_dft_scratch(S.L, s->t, S.P.dft_stride, F);
+    if (S.P.StaticField == 1 || s->t == 0) {
+        // no samples
+    } else if (need > 0 && (size_t)need * 2 <= (size_t)S.N[0] * S.N[1] * S.N[2]) {
+        double *out = nullptr;
+        HIPCHK(s, launch_line_dft(make_line(s), S.m0, s->t, S.P.dft_stride, F, s->freq_d, S.dt, (double *)s->dense, &out,
+                                  s->stream));
+        std::vector<double> v(2 * (size_t)F);
+        HIPCHK(s, hipStreamSynchronize(s->stream));
+        HIPCHK(s, hipMemcpy(v.data(), out, v.size() * sizeof(double), hipMemcpyDeviceToHost));
+        for (int m = 0; m < F; m++) inc[m] = {v[m], v[F + m]};
+    } else {
+        inc = fdtd::line_dft(S, s->t);
+    }
     const double area = S.N[0] * S.P.dx * S.N[1] * S.P.dy;
     for (int m = 0; m < F; m++) {
         const double a2 = std::norm(S.Einc[m]);

@@ -284,6 +284,11 @@ hipError_t launch_tfsf_split(const StepDev &s, hipStream_t st);
 // TFSF terms added after a fused step run with tfsf_on = 0 (H faces, E faces, curl of dH).
 hipError_t launch_tfsf_fix(const StepDev &s, hipStream_t st);
 hipError_t launch_line(const LineDev &l, hipStream_t st);
+// DFT of e_inc[m0] over the first `steps` steps of the line (re then im, F
+// each, at *out in the scratch of line_dft_scratch doubles; -1: line too long).
+long line_dft_scratch(int L, int steps, int stride, int F);
+hipError_t launch_line_dft(const LineDev &l, int m0, int steps, int stride, int F, const double *freq, double dt,
+                           double *scratch, double **out, hipStream_t st);
 hipError_t launch_dispersive(const DispDev &d, hipStream_t st);
 // launch_tfsf_fix (with tfsf), launch_dispersive (Drude + CP, when d is given) and, with
 // sample, the DFT sample of s.Eout / s.Hout into s.sample_row, in one launch;

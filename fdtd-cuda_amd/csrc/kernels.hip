@@ -1485,6 +1485,15 @@ __global__ __launch_bounds__(64 * MW) __attribute__((amdgpu_waves_per_eu(R == 2 
 
 // ----------------------------------------------------------------- 1D incident line
 
+// The source's amplitude at step t.
+__device__ inline double line_pulse(const LineDev &l, int t) {
+    if (l.static_field) return (t < 1000) ? l.amp * t / 1000.0 : l.amp;  // main.cu:2852-2857
+    // powf on a float-converted argument, as the reference (main.cu:2848)
+    const float b = (float)(((double)t - l.delay) / l.width);
+    const float b2 = b * b;
+    return l.amp * exp(-(double)b2 / 2.0) * sin(l.w0dt * (double)t);
+}
+
 // One block: h_inc (main.cu:2328-2336), e_inc (main.cu:2280-2326) into the
 // other buffer, first-order Mur ends and the additive source (main.cu:2831-2859).
 __device__ __forceinline__ void line_body(const LineDev &l, int t, int tid, int nthreads) {
@@ -1499,16 +1508,7 @@ __device__ __forceinline__ void line_body(const LineDev &l, int t, int tid, int 
         l.e_new[L - 1] = e2 + l.mur_coef * (l.e_new[L - 2] - l.e_old[L - 1]);
         l.mur[0] = l.e_new[1];
         l.mur[1] = l.e_new[L - 2];
-        double pulse;
-        if (l.static_field) {
-            pulse = (t < 1000) ? l.amp * t / 1000.0 : l.amp;  // main.cu:2852-2857
-        } else {
-            // powf on a float-converted argument, as the reference (main.cu:2848)
-            const float b = (float)(((double)t - l.delay) / l.width);
-            const float b2 = b * b;
-            pulse = l.amp * exp(-(double)b2 / 2.0) * sin(l.w0dt * (double)t);
-        }
-        l.e_new[l.src] += pulse;
+        l.e_new[l.src] += line_pulse(l, t);
         if (l.probe && l.status && !__builtin_isfinite(*l.probe)) *l.status = 1u;
     }
 }
@@ -2069,6 +2069,68 @@ __global__ void k_disp_sync(DispDev d, int from_field) {
         if (from_field) d.st[c][0][idx] = d.E[c][p];
         else d.E[c][p] = d.st[c][0][idx];
     }
+}
+
+// The incident wave at the source plane over the first `steps` steps, for the
+// spectra that are divided by it: the line run again from rest in the LDS of
+// one block (e in [0, L), h in [L, 2L)), two barriers a step, then its DFT at
+// the monitors' samples.  Bound by the barriers (0.6 us a step); the host
+// took 3 us a step for the same recurrences (L = 1200).  The pulse of every
+// step is formed beforehand by a launch over the steps.
+__global__ __launch_bounds__(256) void k_line_pulses(LineDev l, int steps, double *pulse) {
+    const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+    if (t < steps) pulse[t] = line_pulse(l, t);
+}
+constexpr int kReplayMaxLine = 4096;     // 64 KB of LDS
+__global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int stride, int m0, const double *pulse, double *hist) {
+    extern __shared__ double lds[];
+    const int L = l.L, tid = threadIdx.x, nt = blockDim.x;
+    double *e = lds, *h = lds + L;
+    for (int i = tid; i < 2 * L; i += nt) lds[i] = 0.0;
+    double mur = 0.0, next = steps > 0 ? pulse[0] : 0.0;   // e^n one cell in from this thread's end (threads 0 and 1)
+    __syncthreads();
+    for (int t = 0; t < steps; t++) {
+        const double p = next;
+        next = pulse[min(t + 1, steps - 1)];
+        for (int i = tid; i < L - 1; i += nt) h[i] -= l.ch * (e[i + 1] - e[i]);
+        // the ends need the old end value and the new value one cell in
+        const int end = tid == 0 ? 0 : L - 1, in = tid == 0 ? 1 : L - 2;
+        const double eo = tid < 2 ? e[end] : 0.0, ei = tid < 2 ? e[in] : 0.0;
+        __syncthreads();
+        for (int i = tid + 1; i < L - 1; i += nt) {
+            double v = e[i] - l.ce * (h[i] - h[i - 1]);
+            if (i == l.src) v += p;
+            e[i] = v;
+            if (i == m0 && t % stride == 0) hist[t / stride] = v;
+        }
+        if (tid < 2) {
+            const double en = ei - l.ce * (h[in] - h[in - 1]);
+            e[end] = mur + l.mur_coef * (en - eo);
+            mur = en;
+        }
+        __syncthreads();
+    }
+}
+// out[f], out[F + f] = sum over the samples of hist[s] exp(i 2 pi f (s stride + 1) dt)
+__global__ __launch_bounds__(256) void k_line_dft(const double *hist, int n, int stride, const double *freq, double dt, int F,
+                                                  double *out) {
+    __shared__ double red[2][256];
+    const int f = (int)blockIdx.x, tid = threadIdx.x;
+    double re = 0.0, im = 0.0;
+    for (int s = tid; s < n; s += 256) {
+        double sn, cs;
+        sincos(2.0 * kPI * freq[f] * ((double)s * stride + 1.0) * dt, &sn, &cs);
+        re += hist[s] * cs;
+        im += hist[s] * sn;
+    }
+    red[0][tid] = re;
+    red[1][tid] = im;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (tid < w) { red[0][tid] += red[0][tid + w]; red[1][tid] += red[1][tid + w]; }
+        __syncthreads();
+    }
+    if (tid == 0) { out[f] = red[0][0]; out[F + f] = red[1][0]; }
 }
 
 // ----------------------------------------------------------------- 1D line alone, one-launch step
@@ -3410,5 +3472,23 @@ hipError_t launch_pack_field(const float *f, const Geom &g, float *dense, int to
 hipError_t launch_slice(const float *f, const Geom &g, int axis, int index, float *out, hipStream_t st) {
     const int nu = axis == 0 ? g.NY : g.NX, nv = axis == 2 ? g.NY : g.NZ;
     hipLaunchKernelGGL(k_slice, dim3((nv + 255) / 256, nu), dim3(256), 0, st, f, g, axis, index, nu, nv, out);
+    return hipGetLastError();
+}
+
+long line_dft_scratch(int L, int steps, int stride, int F) {
+    if (L > kReplayMaxLine || L < 4) return -1;
+    return (long)steps + (steps + stride - 1) / stride + 2L * F;
+}
+
+hipError_t launch_line_dft(const LineDev &l, int m0, int steps, int stride, int F, const double *freq, double dt,
+                           double *scratch, double **out, hipStream_t st) {
+    if (line_dft_scratch(l.L, steps, stride, F) < 0 || steps < 1 || stride < 1) return hipErrorInvalidValue;
+    const int n = (steps + stride - 1) / stride;
+    double *pulse = scratch, *hist = pulse + steps, *o = hist + n;
+    const int nt = min(1024, ((l.L + 1) / 2 + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_line_pulses, dim3((steps + 255) / 256), dim3(256), 0, st, l, steps, pulse);
+    hipLaunchKernelGGL(k_line_replay, dim3(1), dim3(nt), 2 * l.L * sizeof(double), st, l, steps, stride, m0, pulse, hist);
+    hipLaunchKernelGGL(k_line_dft, dim3(F), dim3(256), 0, st, hist, n, stride, freq, dt, F, o);
+    *out = o;
     return hipGetLastError();
 }
