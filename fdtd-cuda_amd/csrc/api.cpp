@@ -825,15 +825,20 @@ int launch_rows_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Di
     return FDTD_OK;
 }
 
+StepAll make_step_all(fdtd_sim *s, const LineDev &l, int tiles, int chunk) {
+    StepAll a{};
+    a.r = make_rows(s);
+    a.line = l;
+    a.r.tiles = tiles;
+    add_pieces(s, a, chunk);
+    return a;
+}
+
 // The whole field update in one launch on the solver stream, then the
 // post-update launch.
 int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const DispDev *dd, bool samp, bool *disp_done,
                       bool *samp_done, hipEvent_t ev0, hipEvent_t ev1) {
-    StepAll a{};
-    a.r = make_rows(s);
-    a.line = l;
-    a.r.tiles = s->tiles * rows_waves(s->g.NZ) <= 16 ? s->tiles : 1;
-    add_pieces(s, a, s->one_chunk);
+    const StepAll a = make_step_all(s, l, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1, s->one_chunk);
     if (ev0) HIPCHK(s, hipEventRecord(ev0, s->stream));
     HIPCHK(s, launch_step_all(a, s->stream));
     if (ev1) HIPCHK(s, hipEventRecord(ev1, s->stream));

@@ -3,7 +3,9 @@
 // the reference runs one simulation per process (main.cu:2724-2934); each
 // batched step is that loop body for every simulation at once.
 //
-// Per step every kernel runs ONCE for all simulations that use it: the 1D
+// Per step every kernel runs ONCE for all simulations that use it.  Where all
+// of them have the row path, the lines and the whole field update are one
+// launch (k_step_batch).  Else: the 1D
 // lines (one block each); the field update of fdtd_step's fast path (the
 // row-blocked kernel on clean boxes and side slabs, one launch per variant,
 // block height and rows per thread; the general kernel on corner columns, or
@@ -33,9 +35,9 @@ namespace {
 
 // One batched launch of a step: its kernel, shape and block map.
 struct Launch {
-    enum Type { Rows = 0, Fused = 1, Tfsf = 2, Disp = 3, Sample = 4 };
+    enum Type { Rows = 0, Fused = 1, Tfsf = 2, Disp = 3, Sample = 4, All = 5 };
     int type = 0;
-    int a = 0, b = 0, c = 0;             // Rows: W, R, variant; Fused: tile rows
+    int a = 0, b = 0, c = 0;             // Rows: W, R, variant; Fused: tile rows; All: waves per block
     std::vector<unsigned> map;
     unsigned *d = nullptr;
     bool same(const Launch &o) const { return type == o.type && a == o.a && b == o.b && c == o.c && map == o.map; }
@@ -55,6 +57,11 @@ struct fdtd_batch {
     FusedItem *fused[2] = {};
     RowsArgs *rows[2][3] = {};
     LineDev *line[2] = {};
+    StepAll *all[2] = {};
+    // every simulation's whole field update in one launch per step (k_step_batch),
+    // on one stream, with x chunk one_chunk; else the launches per variant below
+    bool one = false;
+    int one_chunk = 1;
     DispDev *disp[2] = {};
     SampleItem *samp[2] = {};
     int *dyn = nullptr;                     // {t of the next step, ring row of the next sample}
@@ -322,6 +329,12 @@ void add_blocks(Launch &l, int sim, long n) {
     for (long L = 0; L < n; L++) l.map.push_back(((unsigned)sim << kBatchLocalBits) | (unsigned)L);
 }
 
+// Waves per block of the one-launch step for W waves a column: 12 where the
+// columns of several row tiles fill that (and for 5 waves, two tiles in 12), else
+// one column; and its row tiles.
+int one_waves(int W) { return W <= 6 ? 12 : W; }
+int one_tiles(int W) { return one_waves(W) / W; }
+
 // Uploads every per-simulation argument for both parities and rebuilds the
 // launch list; a changed list invalidates the captured graph.
 int upload_items(fdtd_batch *b) {
@@ -331,6 +344,7 @@ int upload_items(fdtd_batch *b) {
         std::vector<FusedItem> fi(n);
         std::vector<RowsArgs> ri[3] = {std::vector<RowsArgs>(n), std::vector<RowsArgs>(n), std::vector<RowsArgs>(n)};
         std::vector<LineDev> li(n);
+        std::vector<StepAll> ai(b->one ? n : 0);
         std::vector<DispDev> di(n);
         std::vector<SampleItem> si(n);
         for (int i = 0; i < n; i++) {
@@ -342,6 +356,12 @@ int upload_items(fdtd_batch *b) {
                 fi[i] = at_parity(s, par, [&] { return fused_full(s, b->ta[i], b->tb[i]); });
             }
             li[i] = at_parity(s, par, [&] { return make_line(s); });
+            if (b->one) {
+                ai[i] = at_parity(s, par, [&] { return make_step_all(s, li[i], one_tiles(rows_waves(s->g.NZ)), b->one_chunk); });
+                const long nb = step_all_blocks(ai[i]);
+                if (nb < 0 || nb >= (1L << kBatchLocalBits)) return berr(b, FDTD_ERR_UNSUPPORTED, "batch: grid too large for the block map");
+                if (par == 0) add_blocks(group(ls, Launch::All, one_waves(rows_waves(s->g.NZ)), 0, 0), i, nb);
+            }
             const int q = at_parity(s, par, [&] { return s->p; });
             di[i] = make_disp(s, 1 - q);
             SampleItem &S = si[i];
@@ -354,14 +374,14 @@ int upload_items(fdtd_batch *b) {
         }
         if (par == 0) {
             // field update: row-blocked launches, then the general kernel; TFSF fix-up; dispersive; samples
-            for (int i = 0; i < n; i++) {
+            for (int i = 0; i < n && !b->one; i++) {
                 if (!b->rowpath[i]) continue;
                 const int W = rows_waves(b->sims[i]->g.NZ);
                 add_blocks(group(ls, Launch::Rows, W, b->ta[i], 0), i, rows_blocks(ri[0][i]));
                 if (rows_blocks(ri[1][i])) add_blocks(group(ls, Launch::Rows, W, 2, 1), i, rows_blocks(ri[1][i]));
                 if (rows_blocks(ri[2][i])) add_blocks(group(ls, Launch::Rows, W, 2, 2), i, rows_blocks(ri[2][i]));
             }
-            for (int i = 0; i < n; i++) {
+            for (int i = 0; i < n && !b->one; i++) {
                 const int tj = b->rowpath[i] ? b->sims[i]->ctj : b->ta[i];
                 const long nb = b->rowpath[i] && !b->sims[i]->ncorner ? 0 : fi[i].pc.start[fi[i].pc.n];
                 if (nb) add_blocks(group(ls, Launch::Fused, tj, 0, 0), i, nb);
@@ -374,6 +394,7 @@ int upload_items(fdtd_batch *b) {
         BCHK(b, hipMemcpy(b->fused[par], fi.data(), n * sizeof(FusedItem), hipMemcpyHostToDevice));
         for (int v = 0; v < 3; v++) BCHK(b, hipMemcpy(b->rows[par][v], ri[v].data(), n * sizeof(RowsArgs), hipMemcpyHostToDevice));
         BCHK(b, hipMemcpy(b->line[par], li.data(), n * sizeof(LineDev), hipMemcpyHostToDevice));
+        if (b->one) BCHK(b, hipMemcpy(b->all[par], ai.data(), n * sizeof(StepAll), hipMemcpyHostToDevice));
         BCHK(b, hipMemcpy(b->disp[par], di.data(), n * sizeof(DispDev), hipMemcpyHostToDevice));
         BCHK(b, hipMemcpy(b->samp[par], si.data(), n * sizeof(SampleItem), hipMemcpyHostToDevice));
     }
@@ -468,6 +489,19 @@ int enqueue_step_early(fdtd_batch *b, int par, int off, int sidx) {
 // order as after it); the samples follow the join.
 int enqueue_step(fdtd_batch *b, int par, int off, int sidx) {
     const int n = (int)b->sims.size();
+    if (b->one) {
+        for (const Launch &l : b->launches) {
+            const int nb = (int)l.map.size();
+            if (l.type == Launch::All) BCHK(b, launch_step_batch(b->all[par], l.d, nb, l.a, b->dyn, off, b->stream));
+        }
+        for (const Launch &l : b->launches) {
+            const int nb = (int)l.map.size();
+            if (l.type == Launch::Tfsf) BCHK(b, launch_tfsf_fix_batch(b->fused[par], l.d, nb, b->stream));
+            if (l.type == Launch::Disp) BCHK(b, launch_disp_batch(b->disp[par], l.d, nb, b->stream));
+            if (l.type == Launch::Sample && sidx >= 0) BCHK(b, launch_sample_batch(b->samp[par], l.d, nb, b->dyn, sidx, b->stream));
+        }
+        return FDTD_OK;
+    }
     const bool fork = b->stream2 != nullptr;
     const bool three = fork && b->stream3 && b->stream4;
     if (fork && b->early && b->early_ok && b->ev_early) return enqueue_step_early(b, par, off, sidx);
@@ -625,6 +659,11 @@ int fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out)
     if (int rc = check_sims(b)) return fail(rc);
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(berr(b, FDTD_ERR_DEVICE, "hipStreamCreate failed"));
+    b->one = !(flags & FDTD_BATCH_GENERAL);
+    for (fdtd_sim *s : b->sims) b->one = b->one && s->use_rows && s->rows == 2;
+    for (const char *k : {"FDTD_CONCURRENT", "FDTD_SIDE_STREAMS", "FDTD_BATCH_EARLY", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_CTJ"})
+        if (std::getenv(k)) b->one = false;
+    if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) b->one = b->one && std::atoi(v) != 0;
     const char *conc = std::getenv("FDTD_CONCURRENT");
     if (!conc || std::atoi(conc) != 0) {
         if (hipStreamCreateWithFlags(&b->stream2, hipStreamNonBlocking) != hipSuccess ||
@@ -654,14 +693,29 @@ int fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out)
             if ((rc = balloc(b, &b->rows[par][v], n))) return fail(rc);
     }
     if ((rc = balloc(b, &b->dyn, 2))) return fail(rc);
+    if (b->one) {
+        // one chunk for the batch, by the rule of the single step over all its columns
+        // (block rows times planes; blocks of 12 waves leave one resident per CU)
+        if ((rc = balloc(b, &b->all[0], n)) || (rc = balloc(b, &b->all[1], n))) return fail(rc);
+        long columns = 0;
+        int NX = 1;
+        for (fdtd_sim *s : b->sims) NX = std::max(NX, s->g.NX);
+        for (fdtd_sim *s : b->sims) {
+            const int t = one_tiles(rows_waves(s->g.NZ));
+            columns += (long)((s->g.NY + 2 * t - 1) / (2 * t)) * s->g.NX;
+        }
+        // at most 8 planes: us per step of 12 rods with chunks 4, 8, 12, 16, 24: 1129, 1054, 1070,
+        // 1075, 1070 (of 4 rods 378, 351, 358, 358, 360)
+        b->one_chunk = march_chunk((columns + NX - 1) / NX, NX, 256, 8);
+    }
     b->rowpath.assign(n, 0);
     b->ta.assign(n, 8);
     b->tb.assign(n, 32);
     for (int i = 0; i < n; i++) {
         fdtd_sim *s = b->sims[i];
         b->rowpath[i] = s->use_rows && !(flags & FDTD_BATCH_GENERAL) ? 1 : 0;
-        if (b->rowpath[i]) { b->ta[i] = s->rows; b->tb[i] = s->cchunk; }
-        if (!(flags & FDTD_BATCH_NO_TUNE))
+        if (b->rowpath[i]) { b->ta[i] = s->rows; b->tb[i] = b->one ? b->one_chunk : s->cchunk; }
+        if (!b->one && !(flags & FDTD_BATCH_NO_TUNE))
             if ((rc = autotune(b, s, b->rowpath[i] != 0, &b->ta[i], &b->tb[i]))) return fail(rc);
         long nb[4] = {0, 0, 0, 0};
         if (b->rowpath[i]) {

@@ -267,6 +267,12 @@ struct StepAll {
     int start[kStepAllPieces + 1];
 };
 hipError_t launch_step_all(StepAll a, hipStream_t st);
+// Fills in start and the wave counts; the blocks of the launch (line and pieces) or -1.
+long step_all_blocks(StepAll &a);
+// Over many simulations (items prepared by step_all_blocks; nw waves per block,
+// at least waves * tiles of every item): dyn and step_off as launch_line_batch.
+hipError_t launch_step_batch(const StepAll *items, const unsigned *map, int nblocks, int nw, const int *dyn, int step_off,
+                             hipStream_t st);
 // Blocks of one piece (two rows per thread, r.tiles row tiles per block).
 long rows_pieces_blocks(const RowsArgs &r, const int box[4], int ichunk);
 

@@ -791,7 +791,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
     const int lane = threadIdx.x, wg = __builtin_amdgcn_readfirstlane((int)threadIdx.y), w = wg % W;
     const int t = w * 64 + lane;
     const int jt0 = jtb * T + wg / W;
-    const bool live = jt0 < njt;
+    const bool live = jt0 < njt && wg < W * T;   // a batch's blocks may hold more waves than this item's columns fill
     const int jt = live ? jt0 : njt - 1;
     const int k = seg * (64 * W - 2) - 1 + t;
     const int kc = min(k, NZ - 1);
@@ -2074,6 +2074,7 @@ __global__ void k_disp_sync(DispDev d, int from_field) {
 // The incident wave at the source plane over the first `steps` steps, for the
 // spectra that are divided by it: the line run again from rest in the LDS of
 // one block (e in [0, L), h in [L, 2L)), two barriers a step, then its DFT at
+// one block (e in [0, L), h in [L, 2L)), two barriers a step, then its DFT at
 // the monitors' samples.  Bound by the barriers (0.6 us a step); the host
 // took 3 us a step for the same recurrences (L = 1200).  The pulse of every
 // step is formed beforehand by a launch over the steps.
@@ -2146,15 +2147,13 @@ __global__ __launch_bounds__(1024) void k_line(LineDev l) { line_body(l, l.t, th
 // against 90, of 125 x 173 x 204 88 against 122.  Large grids are bound by
 // memory: at 281^3 the launch moves 1.56 GB (1.25 GB it cannot do without) in
 // 315 us, 4.9 TB/s, what a large copy reaches on this card.
-__global__ __launch_bounds__(64 * kRowsMaxWaves) void k_step_all(StepAll) {
-    // the arguments in place (their only copy; a by-value struct indexed by piece would be copied to scratch)
-    const StepAll &a = batch_item((const StepAll *)(const CONST_AS StepAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
+__device__ __forceinline__ void step_all_body(const StepAll &a, int t, int block, int nwaves) {
     __shared__ RowsLds<2, false> lds;
-    if (blockIdx.x == 0) {
-        line_body(a.line, a.line.t, threadIdx.y * 64 + threadIdx.x, 64 * a.r.waves * a.r.tiles);
+    if (block == 0) {
+        line_body(a.line, t, threadIdx.y * 64 + threadIdx.x, 64 * nwaves);
         return;
     }
-    const int b = (int)blockIdx.x - 1;
+    const int b = block - 1;
     int q = 0;
     while (q + 1 < a.n && b >= a.start[q + 1]) q++;
     const int ia = a.box[q][0], ib = a.box[q][1], ja = a.box[q][2], jb = a.box[q][3], ich = a.ich[q];
@@ -2165,6 +2164,26 @@ __global__ __launch_bounds__(64 * kRowsMaxWaves) void k_step_all(StepAll) {
         case 2: rows_piece<2, false, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
         default: rows_piece<2, true, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
     }
+}
+__global__ __launch_bounds__(64 * kRowsMaxWaves) void k_step_all(StepAll) {
+    // the arguments in place (their only copy; a by-value struct indexed by piece would be copied to scratch)
+    const StepAll &a = batch_item((const StepAll *)(const CONST_AS StepAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
+    step_all_body(a, a.line.t, (int)blockIdx.x, a.r.waves * a.r.tiles);
+}
+// The same over many simulations (map as the other batched kernels, block 0 of
+// each simulation its line).  Grids of 2, 3, 4 and 6 waves a column share the
+// launch in blocks of 12 waves (6, 4, 3 and 2 row tiles): one launch for the
+// whole batch leaves one tail a step, and the taller blocks read fewer halo
+// rows.  us per step of 4, 12 and 32 rods (17, 56 and 147 M cells): 351, 1054
+// and 2671, with a launch per variant and column height on two streams 413,
+// 1162 and 2910.  The launch is bound by memory (909 of the 1075 us a step at 12
+// rods in a trace).
+template <int MW>
+__global__ __launch_bounds__(64 * MW) void k_step_batch(const StepAll *items, const unsigned *map, const int *dyn, int step_off) {
+    const unsigned m = batch_map(map);
+    const CONST_AS int *d = (const CONST_AS int *)dyn;
+    step_all_body(batch_item(items, m >> kBatchLocalBits), d[0] + step_off, (int)(m & ((1u << kBatchLocalBits) - 1)),
+                  (int)blockDim.y);
 }
 
 // ----------------------------------------------------------------- DFT contraction
@@ -3191,6 +3210,15 @@ hipError_t launch_step_rows(RowsArgs ra, int R, int variant, hipStream_t st) {
     }
 }
 
+hipError_t launch_step_batch(const StepAll *items, const unsigned *map, int nblocks, int nw, const int *dyn, int step_off,
+                             hipStream_t st) {
+    if (nblocks <= 0) return hipSuccess;
+    if (nw < 1 || nw > kRowsMaxWaves) return hipErrorInvalidValue;
+    if (nw <= 12) hipLaunchKernelGGL((k_step_batch<12>), dim3(nblocks), dim3(64, nw), 0, st, items, map, dyn, step_off);
+    else hipLaunchKernelGGL((k_step_batch<16>), dim3(nblocks), dim3(64, nw), 0, st, items, map, dyn, step_off);
+    return hipGetLastError();
+}
+
 // Checks the pieces of a one-launch step and fills in the rest; returns the blocks of all pieces or -1.
 template <typename A>
 static long pieces_prepare(A &a, int max_waves) {
@@ -3212,6 +3240,11 @@ static long pieces_prepare(A &a, int max_waves) {
     if (total > 0x7fffff00) return -1;
     a.start[a.n] = (int)total;
     return total;
+}
+
+long step_all_blocks(StepAll &a) {
+    const long n = pieces_prepare(a, kRowsMaxWaves);
+    return n < 0 ? -1 : n + 1;
 }
 
 hipError_t launch_step_all(StepAll a, hipStream_t st) {

@@ -205,6 +205,10 @@ int upload(fdtd_sim *s, T **ptr, const std::vector<T> &v) {
     return FDTD_OK;
 }
 
+// One-launch step: the x chunk for `columns` blocks per chunk layer of NX planes
+// and `slots` resident blocks, and the arguments at the handle's parity.
+int march_chunk(long columns, int NX, long slots, int most);
+StepAll make_step_all(fdtd_sim *s, const LineDev &l, int tiles, int chunk);
 // Kernel arguments at the handle's current parity.
 StepDev make_step(fdtd_sim *s, bool fused);
 LineDev make_line(fdtd_sim *s);

@@ -324,7 +324,9 @@ int  fdtd_kernel_timing(fdtd_sim *sim, int enable, double *total_ms, long *launc
  * the launches of one DFT sampling period are captured in a HIP graph and
  * replayed.  The field update is fdtd_step's: the row-blocked kernel with the
  * TFSF fix-up where the simulation's grid allows it, else the general fused
- * kernel; the tile of each grid size's dominant launch is picked by the
+ * kernel.  Where every simulation has the row-blocked kernel, its pieces and
+ * the 1D lines of all of them are one launch, its x chunk chosen by the batch's
+ * cells.  Else the tile of each grid size's dominant launch is picked by the
  * autotuner (timed on the device at fdtd_batch_create, remembered per process
  * and, when the environment variable FDTD_TUNE_FILE names a file, across
  * processes).
@@ -336,7 +338,7 @@ int  fdtd_kernel_timing(fdtd_sim *sim, int enable, double *total_ms, long *launc
  */
 typedef struct fdtd_batch fdtd_batch;
 #define FDTD_BATCH_NO_GRAPH 1   /* launch every step directly instead of replaying a graph */
-#define FDTD_BATCH_NO_TUNE  2   /* the simulations' own tiles (those fdtd_step uses)       */
+#define FDTD_BATCH_NO_TUNE  2   /* no autotuner: the simulations' own tiles               */
 #define FDTD_BATCH_GENERAL  4   /* general fused kernel for every simulation               */
 int  fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out);
 /* Advances every simulation by nsteps full steps (as fdtd_step does). */

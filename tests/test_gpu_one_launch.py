@@ -81,3 +81,31 @@ def test_general_kernel_chunks_by_rule(n, monkeypatch):
     for c in range(6):
         scale = max(np.abs(f).max() for f in (out[1][:3] if c < 3 else out[1][3:]))
         assert np.abs(out[0][c] - out[1][c]).max() <= 1e-5 * scale, c
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_batch_of_every_column_height_equals_each_alone(graph):
+    """Grids of 2, 3, 4, 5, 6 and 8 waves a column in one batch: the first five
+    share blocks of 12 waves (6, 4, 3, 2 and 2 row tiles, two waves idle at 5),
+    the last has blocks of 8.  203 steps, so periods by graph and single steps."""
+    def sims():
+        out = []
+        for q, (nx, ny, nz) in enumerate(((24, 24, 24), (21, 27, 131), (22, 24, 200), (20, 23, 270), (25, 20, 330), (20, 21, 400))):
+            p = small_params(fdtd_amd, sphere=q % 2, radius=6e-9)
+            p.NCELLX, p.NCELLY, p.NCELLZ = nx, ny, nz
+            s = fdtd_amd.Simulation(p)
+            rng = np.random.default_rng(q)
+            for c in range(3):
+                s.set_field(c, (rng.standard_normal(s.shape) * 0.1).astype(np.float32))
+            out.append(s)
+        return out
+    a, b = sims(), sims()
+    batch = fdtd_amd.Batch(a, flags=0 if graph else fdtd_amd.BATCH_NO_GRAPH)
+    assert all(batch.tile(i)[:2] == (1, 2) for i in range(len(a)))
+    batch.run(203)
+    for s, t in zip(a, b):
+        t.step(203)
+        for c in range(6):
+            assert np.array_equal(s.get_field(c), t.get_field(c)), (s.shape, c)
+        for x, y in zip(s.get_line(), t.get_line()):
+            assert np.array_equal(x, y)
