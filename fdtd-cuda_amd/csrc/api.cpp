@@ -21,6 +21,8 @@
 using fdtd::Setup;
 using namespace fdtd_host;
 
+static int flush_records(fdtd_sim *s);
+
 namespace {
 thread_local std::string g_create_err = "no error";
 }
@@ -62,6 +64,8 @@ StepDev make_step(fdtd_sim *s, bool fused) {
     t.cH = (float)S.Che; t.cE = (float)S.Ceh;
     t.dscale = 1.0f;  // d_1D = dx (tfsf2.cu:19)
     t.m0 = S.m0;
+    t.line_lo = 1 - S.m0;
+    t.line_hi = S.L - 1 - S.m0;
     t.e_inc = s->line_e[s->le];
     t.h_inc = s->line_h;
     d.tfsf_on = fused ? 1 : 0;
@@ -92,6 +96,10 @@ LineDev make_line(fdtd_sim *s) {
     l.t = s->t;
     l.probe = s->E[s->p][0] + s->probe_cell;
     l.status = s->status_d;
+    for (int q = 0; q < 2; q++) {
+        l.rec_dst[q] = s->rec_dst[q];
+        for (int c = 0; c < 3; c++) l.rec_src[q][c] = s->E[s->p][c] + s->rec_p[q];
+    }
     return l;
 }
 
@@ -560,12 +568,13 @@ int plan_rows(fdtd_sim *s) {
     }
     s->use_rows = s->has_clean;
     // One launch for the whole update up to 12 M cells, unless a knob of the stream schedule
-    // asks for that (FDTD_ONE_LAUNCH=0: the schedule with its defaults); two rows per thread
+    // asks for that (FDTD_ONE_LAUNCH=0: the schedule with its defaults, 1: one launch whatever the size); two rows per thread
     // only.  Measured us per step, one launch against the streams: 22 and 91 at 0.05 M cells,
     // 35 and 90 at 0.6 M, 89 and 121 at 4.4 M, 374 and 369 at 22 M, 929 and 907 at 68 M
     // (there the post-update launch overlaps the next step's side pieces).
-    s->one_launch = s->rows == 2 && (long)s->g.NX * s->g.NY * s->g.NZ <= 12000000L;
-    if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = s->one_launch && std::atoi(v) != 0;
+    s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= 12000000L;
+    if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = std::atoi(v) != 0;
+    s->one_launch = s->one_launch && s->rows == 2;
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
                           "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
         if (std::getenv(k)) s->one_launch = false;
@@ -625,9 +634,9 @@ bool tfsf_in_clean(const fdtd_sim *s) {
 // velocity-state and density buffers (k_hydro_ce leaves v^{n+1} in h_vnew and
 // n~^{n+1} in h_nd, and reads neither the old velocity state nor h_ndp of the
 // component it updates at a neighbour after writing it).
-hipError_t launch_box(fdtd_sim *s, const DispDev &dd) {
+hipError_t launch_box(fdtd_sim *s, const DispDev &dd, const StepDev *with = nullptr, bool samp = false) {
     if (!s->S.hydro) return launch_dispersive(dd, s->stream);
-    const hipError_t e = launch_hydro(dd, s->stream);
+    const hipError_t e = launch_hydro(dd, with, samp, s->stream);
     if (e == hipSuccess)
         for (int c = 0; c < 3; c++) {
             std::swap(s->disp_st[c][2], s->h_vnew[c]);
@@ -805,12 +814,15 @@ int launch_rows_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Di
         s->early_ready = true;
     }
     const bool merge_disp = disp_early && tf_early && !s->S.hydro;
+    const bool merge_samp = tf_early && samp && d.sample_row && (s->nbox <= 0 || disp_early) && sample_in_clean(s);
+    const bool hydro_post = disp_early && tf_early && s->S.hydro;
     if (disp_early && !merge_disp) {
-        HIPCHK(s, launch_box(s, *dd));
+        HIPCHK(s, launch_box(s, *dd, hydro_post ? &d : nullptr, merge_samp));
         *disp_done = true;
     }
-    const bool merge_samp = tf_early && samp && d.sample_row && (s->nbox <= 0 || disp_early) && sample_in_clean(s);
-    if (tf_early) {
+    if (hydro_post) {
+        *samp_done = merge_samp;
+    } else if (tf_early) {
         if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, true, merge_disp ? dd : nullptr, merge_samp, s->stream));
         else HIPCHK(s, launch_tfsf_fix(d, s->stream));
         *disp_done = *disp_done || merge_disp;
@@ -845,9 +857,10 @@ int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Dis
     // the box and the sample ride with the TFSF fix-up where their cells are apart from it
     const bool merge_disp = dd && !s->S.hydro && disp_in_clean(s);
     const bool merge_samp = samp && d.sample_row && (s->nbox <= 0 || disp_in_clean(s)) && sample_in_clean(s);
-    if (merge_disp || merge_samp) HIPCHK(s, launch_post(d, true, merge_disp ? dd : nullptr, merge_samp, s->stream));
-    else HIPCHK(s, launch_tfsf_fix(d, s->stream));
-    *disp_done = merge_disp;
+    const bool hydro_post = dd && s->S.hydro && disp_in_clean(s);
+    if (hydro_post) HIPCHK(s, launch_box(s, *dd, &d, merge_samp));
+    else HIPCHK(s, launch_post(d, true, merge_disp ? dd : nullptr, merge_samp, s->stream));
+    *disp_done = merge_disp || hydro_post;
     *samp_done = merge_samp;
     return FDTD_OK;
 }
@@ -1327,6 +1340,7 @@ int fdtd_adjoint(fdtd_sim *s, int nsteps, int ckpt, const int r0[3], int nf, con
     if (W.probe) (void)hipFree(W.probe);
     if (W.traj) (void)hipFree(W.traj);
     s->probe = nullptr;
+    s->rec_dst[0] = s->rec_dst[1] = nullptr;
     s->sampling = true;
     for (int c = 0; c < 3; c++) s->traj_step[c] = s->traj_first[0][c] = s->traj_first[1][c] = nullptr;
     return rc;
@@ -1559,13 +1573,20 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
     s->probe_t0 = t0;
     // the recorded loops step one at a time (record() only moves host pointers),
     // keeping the early start of the side pieces across the steps of a loop
-    if (store) {
+    auto recorded_steps = [&](int len) -> int {
         s->early_ready = false;
-        for (int st = 0; st < nsteps; st++) {
+        s->defer_records = true;
+        int r = FDTD_OK;
+        for (int st = 0; st < len && !r; st++) {
             record(st);
-            if ((rc = step_steps(s, 1))) return rc;
+            r = step_steps(s, 1);
         }
+        s->defer_records = false;
         unrecord();
+        return r ? r : flush_records(s);
+    };
+    if (store) {
+        if ((rc = recorded_steps(nsteps))) return rc;
     } else {
         for (int seg = 0; seg < nseg; seg++) {
             const int len = std::min(ckpt, nsteps - seg * ckpt);
@@ -1575,12 +1596,7 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
             } else {
                 // the last segment records its box trajectory on the way, so the
                 // reverse sweep starts on it without a checkpoint or a recompute
-                s->early_ready = false;
-                for (int st = 0; st < len; st++) {
-                    record(st);
-                    if ((rc = step_steps(s, 1))) return rc;
-                }
-                unrecord();
+                if ((rc = recorded_steps(len))) return rc;
             }
         }
     }
@@ -1642,12 +1658,7 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
                 Checkpoint &ck = cks[seg];
                 s->t = ck.t; s->p = ck.p; s->pp = ck.pp; s->le = ck.le;
                 if ((rc = ckpt_copy(s, ck, false))) return rc;
-                s->early_ready = false;
-                for (int st = 0; st < len; st++) {
-                    record(st);
-                    if ((rc = step_steps(s, 1))) return rc;
-                }
-                unrecord();
+                if ((rc = recorded_steps(len))) return rc;
                 s->early_ready = false;
                 s->adj_early_ready = false;
             }
@@ -1802,8 +1813,23 @@ int fdtd_step(fdtd_sim *s, int nsteps) {
 
 // fdtd_step without clearing the early start: for loops of single steps that
 // launch nothing else between them (the adjoint's recorded steps).
+// Records (point monitor, objective probe) of a step are taken by the next
+// step's line launch; a launch of their own (5 us a step) only takes those of a
+// call's last step.
+static int flush_records(fdtd_sim *s) {
+    for (int q = 0; q < 2; q++) {
+        if (!s->rec_dst[q]) continue;
+        const float *E[3] = {s->E[s->p][0], s->E[s->p][1], s->E[s->p][2]};
+        float *dst = s->rec_dst[q];
+        s->rec_dst[q] = nullptr;
+        HIPCHK(s, launch_probe(E, s->rec_p[q], dst, s->stream));
+    }
+    return FDTD_OK;
+}
+
 int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
     if (int rc = check_finite(s)) return rc;
+    if (!s->defer_records) s->rec_dst[0] = s->rec_dst[1] = nullptr;   // left by a call that failed
     if (s->S.P.periodic_xy) {
         for (int n = 0; n < nsteps; n++)
             if (int rc = periodic_step(s)) return rc;
@@ -1851,13 +1877,16 @@ int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
         }
         if (step_timing) s->ev_used++;
         if (s->nbox && !disp_done) HIPCHK(s, launch_box(s, dd));
+        // this step's line took the records of the step before; those of this one wait for the
+        // next step's line, or for the end of the call
+        s->rec_dst[0] = s->rec_dst[1] = nullptr;
         if (s->probe) {
-            const float *E1[3] = {s->E[1 - q][0], s->E[1 - q][1], s->E[1 - q][2]};
-            HIPCHK(s, launch_probe(E1, s->probe_p, s->probe + 3 * (size_t)(s->t - s->probe_t0), s->stream));
+            s->rec_dst[0] = s->probe + 3 * (size_t)(s->t - s->probe_t0);
+            s->rec_p[0] = s->probe_p;
         }
         if (s->mon && s->t - s->mon_t0 < s->mon_cap) {
-            const float *E1[3] = {s->E[1 - q][0], s->E[1 - q][1], s->E[1 - q][2]};
-            HIPCHK(s, launch_probe(E1, s->mon_p, s->mon + 3 * (size_t)(s->t - s->mon_t0), s->stream));
+            s->rec_dst[1] = s->mon + 3 * (size_t)(s->t - s->mon_t0);
+            s->rec_p[1] = s->mon_p;
         }
         s->p ^= 1;
         s->pp ^= 1;
@@ -1876,7 +1905,7 @@ int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
         }
         s->t++;
     }
-    return FDTD_OK;
+    return s->defer_records ? FDTD_OK : flush_records(s);
 }
 
 int fdtd_set_point_monitor(fdtd_sim *s, const int r[3], int capacity) {

@@ -56,6 +56,7 @@ struct TfsfDev {
     float inv_d[3];          // 1/dx, 1/dy, 1/dz
     float dscale;            // dx / d_1D
     int m0;
+    int line_lo, line_hi;    // values of the line from m0 on that exist in both e_inc and h_inc (from m0 - 1)
     const double *e_inc;     // e_inc^n
     const double *h_inc;     // h_inc^{n+1/2}
 };
@@ -188,6 +189,9 @@ struct LineDev {
     // when it is NaN or Inf (either may be null)
     const float *probe;
     unsigned *status;
+    // records of the last step's E: three values each to rec_dst (null: none)
+    const float *rec_src[2][3];
+    float *rec_dst[2];
 };
 
 // ---------------------------------------------------------------------------
@@ -318,7 +322,9 @@ hipError_t launch_pack_field(const float *f, const Geom &g, float *dense, int to
 hipError_t launch_slice(const float *f, const Geom &g, int axis, int index, float *out, hipStream_t st);
 hipError_t launch_disp_sync_state(const DispDev &d, int from_field, hipStream_t st);
 // Hydrodynamic model: velocity update, then per component (x, y, z) continuity and E update.
-hipError_t launch_hydro(const DispDev &d, hipStream_t st);
+// With s: its TFSF fix-up and, with sample, the DFT sample (as launch_post) ride on the
+// first launch; only for cell sets apart from the box.
+hipError_t launch_hydro(const DispDev &d, const StepDev *s, bool sample, hipStream_t st);
 // NONLOCAL == 1: grad(div) of the Drude polarisation into d.gd (no-op when d.gd[0] is null).
 hipError_t launch_nonlocal_gd(const DispDev &d, hipStream_t st);
 

@@ -63,6 +63,11 @@ struct fdtd_sim {
     long mon_p = 0;
     int mon_t0 = 0, mon_cap = 0, mon_cap_alloc = 0;
     long probe_p = 0;
+    // records of the last step's E not yet taken (0 probe, 1 point monitor): set within a call of
+    // step_steps only, or between its calls while defer_records is on
+    float *rec_dst[2] = {};
+    long rec_p[2] = {0, 0};
+    bool defer_records = false;
     int probe_t0 = 0;               // step whose E^{n+1} lands in probe[0..2]
     float *traj_step[3] = {};       // dispersive kernel writes E^{n+1} here when set
     float *traj_first[2][3] = {};   // and E^{n-1}, E^n here for the first recorded step
