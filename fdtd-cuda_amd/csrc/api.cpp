@@ -1932,20 +1932,24 @@ int fdtd_point_spectrum(fdtd_sim *s, int nf, const double *freq, double *e2, dou
     if (!s || nf < 1 || !freq || (!e2 && !amp)) return FDTD_ERR_INVALID;
     if (!s->mon) return set_err(s, FDTD_ERR_INVALID, "no point monitor set");
     const int n = std::min(s->t - s->mon_t0, s->mon_cap);
-    std::vector<float> e((size_t)3 * std::max(n, 1));
     HIPCHK(s, hipStreamSynchronize(s->stream));
     if (int rc = check_finite(s)) return rc;
-    if (n > 0) HIPCHK(s, hipMemcpy(e.data(), s->mon, (size_t)3 * n * sizeof(float), hipMemcpyDeviceToHost));
-    const double dt = s->S.dt;
-    for (int f = 0; f < nf; f++) {
-        std::complex<double> g[3] = {0.0, 0.0, 0.0};
-        for (int q = 0; q < n; q++) {
-            const std::complex<double> w = std::exp(std::complex<double>(0, 2 * fdtd::kPI * freq[f] * (s->mon_t0 + q + 1.0) * dt));
-            for (int c = 0; c < 3; c++) g[c] += (double)e[(size_t)3 * q + c] * w;
+    // the frequencies and amplitudes pass through the staging buffer, as many at a time as it holds
+    const int most = (int)std::min<size_t>((size_t)s->g.NX * s->g.NY * s->g.NZ / 14, 1 << 20);
+    std::vector<double> g(6 * (size_t)std::min(nf, most));
+    double *fd = (double *)s->dense;
+    for (int f0 = 0; f0 < nf; f0 += most) {
+        const int m = std::min(most, nf - f0);
+        double *out = fd + m;
+        HIPCHK(s, hipMemcpyAsync(fd, freq + f0, m * sizeof(double), hipMemcpyHostToDevice, s->stream));
+        HIPCHK(s, launch_point_dft(s->mon, std::max(n, 0), s->mon_t0, m, fd, s->S.dt, out, s->stream));
+        HIPCHK(s, hipStreamSynchronize(s->stream));
+        HIPCHK(s, hipMemcpy(g.data(), out, 6 * (size_t)m * sizeof(double), hipMemcpyDeviceToHost));
+        for (int f = 0; f < m; f++) {
+            const double *v = &g[6 * (size_t)f];
+            if (e2) e2[f0 + f] = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]) + (v[4] * v[4] + v[5] * v[5]);
+            if (amp) std::memcpy(amp + 6 * ((size_t)f0 + f), v, 6 * sizeof(double));
         }
-        if (e2) e2[f] = std::norm(g[0]) + std::norm(g[1]) + std::norm(g[2]);
-        if (amp)
-            for (int c = 0; c < 3; c++) { amp[(f * 3 + c) * 2] = g[c].real(); amp[(f * 3 + c) * 2 + 1] = g[c].imag(); }
     }
     return FDTD_OK;
 }

@@ -294,6 +294,8 @@ hipError_t launch_tfsf_split(const StepDev &s, hipStream_t st);
 // TFSF terms added after a fused step run with tfsf_on = 0 (H faces, E faces, curl of dH).
 hipError_t launch_tfsf_fix(const StepDev &s, hipStream_t st);
 hipError_t launch_line(const LineDev &l, hipStream_t st);
+// DFT of n point-monitor records (three floats each, the first of step t0): 6 nf doubles to out.
+hipError_t launch_point_dft(const float *rec, int n, int t0, int nf, const double *freq, double dt, double *out, hipStream_t st);
 // DFT of e_inc[m0] over the first `steps` steps of the line (re then im, F
 // each, at *out in the scratch of line_dft_scratch doubles; -1: line too long).
 long line_dft_scratch(int L, int steps, int stride, int F);
