@@ -87,6 +87,8 @@ struct fdtd_sim {
     } adj;
     // misc
     float *dense = nullptr;         // NX*NY*NZ staging for field copies
+    char *pinned = nullptr;         // staging of field read-outs (two halves; from the first large one on)
+    size_t pinned_half = 0;
     size_t fsz = 0;                 // floats per padded field allocation
     long fbase = 0;                 // offset of element (0,0,0) in it
     size_t hsz[6] = {}, esz[6] = {};
@@ -228,6 +230,8 @@ bool disp_in_clean(const fdtd_sim *s);
 bool tfsf_off_clean_edges(const fdtd_sim *s);
 // nsteps steps keeping an early start from the step before (fdtd_step clears it first)
 int step_steps(fdtd_sim *s, int nsteps);
+// Device memory to the caller's, after the work queued on the solver stream.
+int copy_out(fdtd_sim *s, const void *dev, void *host, size_t bytes);
 // FDTD_ERR_NONFINITE (with a message) when a kernel has flagged a NaN or Inf.
 int check_finite(fdtd_sim *s);
 // DFT bookkeeping: a sampling step, the ring slot just written, the K-sample contraction.
