@@ -385,7 +385,7 @@ hipEvent_t next_event(fdtd_sim *s, int which) {
 // the launch takes as many rounds of resident blocks as its block count needs:
 // the chunk with the smallest rounds * (chunk + 2) is taken.  It goes from one
 // plane where every block is resident at once to 12 where many rounds run
-// (measured us per step, chunks 1, 2, 4, 8, 12, 16: 37^3 22, 26, 34, 47, -, 53;
+// (measured us per step with the march unrolled, chunks 1, 2, 4, 8, 12, 16: 37^3 22, 26, 34, 47, -, 53;
 // 85^3 37, 34, 39, 55, -, 67; 125 x 173 x 204 -, 102, 89, 92, -, -; 281^3 648,
 // 477, 400, 373, 370, 375).
 // columns: blocks per x chunk; slots: blocks resident at once.
@@ -571,8 +571,8 @@ int plan_rows(fdtd_sim *s) {
     s->use_rows = s->has_clean;
     // One launch for the whole update up to 12 M cells, unless a knob of the stream schedule
     // asks for that (FDTD_ONE_LAUNCH=0: the schedule with its defaults, 1: one launch whatever the size); two rows per thread
-    // only.  Measured us per step, one launch against the streams: 22 and 91 at 0.05 M cells,
-    // 35 and 90 at 0.6 M, 89 and 121 at 4.4 M, 374 and 369 at 22 M, 929 and 907 at 68 M
+    // only.  Measured us per step, one launch against the streams: 21 and 91 at 0.05 M cells,
+    // 33 and 90 at 0.6 M, 86 and 121 at 4.4 M, 351 and 348 at 22 M, 929 and 907 at 68 M
     // (there the post-update launch overlaps the next step's side pieces).
     s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= 12000000L;
     if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = std::atoi(v) != 0;
@@ -580,7 +580,8 @@ int plan_rows(fdtd_sim *s) {
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
                           "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
         if (std::getenv(k)) s->one_launch = false;
-    s->one_chunk = one_launch_chunk(s, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1, 4);
+    const int ot = s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1;
+    s->one_chunk = one_launch_chunk(s, ot, step_all_bound(ot * rows_waves(s->g.NZ)) / 4);
     return FDTD_OK;
 }
 

@@ -1273,7 +1273,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
         for (int r = 0; r <= R; r++) { h.h[0][r] = ldb(bHx, pl + ro[r]); h.h[1][r] = ldb(bHy, pl + ro[r]); h.h[2][r] = ldb(bHz, pl + ro[r]); }
     };
     ESet EA, EB, EC;
-    HSet H0, H1;
+    HSet HN;
     PSet P0, P1;   // P1 only for the prologue plane
     // prologue: H^{n+1/2} of plane i0-1 (not needed at i0 = 0: ey, ez are not
     // updated there), E^n of planes i0 and i0+1, H and psi of plane i0
@@ -1285,7 +1285,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
         float pxk[R + 1], pyk[R + 1], hx[R + 1], hy[R + 1], hz[R + 1];
         float vxy[R + 2], vzy[R + 2], vyx[R + 1], vzx[R + 1], pyx[R + 1], pzx[R + 1];
         load_e(i0 - 1, P);
-        load_h(i0 - 1, H1);
+        load_h(i0 - 1, HN);
         load_psi(i0 - 1, P1);
         if constexpr (AS && XG) {
             // psi_E along x of the prologue plane itself (load_psi brings plane i0's)
@@ -1312,7 +1312,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
             vxweights(i0 - 1, P.y, P.z, pyx, pzx, false, vyx, vzx);
             vxweights(i0, EA.y, EA.z, P1.eyx, P1.ezx, true, vyxC, vzxC);   // plane i0 is this chunk's: psi written
         }
-        hplane(i0 - 1, P.x, P.y, P.z, P.xj, P.zj, pxk, pyk, EA.y, EA.z, H1.h, P1, false, zx, zy, vxy, vzy, vyx, vzx,
+        hplane(i0 - 1, P.x, P.y, P.z, P.xj, P.zj, pxk, pyk, EA.y, EA.z, HN.h, P1, false, zx, zy, vxy, vzy, vyx, vzx,
                vyxC, vzxC, hx, hy, hz);
         if constexpr (AS && XG) {
             wxweights(i0 - 1, hy, hz, P1, false, hyP, hzP);
@@ -1323,12 +1323,12 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
     }
     e_publish(EA.x, EA.y, 0);
     load_e(i0 + 1, EB);
-    load_h(i0, H0);
+    load_h(i0, HN);
     lds_sync();
 
     // one x step: C = E of plane i, N = E of plane i+1, Fr <- E of plane i+2,
-    // Hc = H of plane i, Hn <- H of plane i+1, Pc <- psi of plane i
-    auto step = [&](int i, ESet &C, ESet &N, ESet &Fr, HSet &Hc, HSet &Hn, PSet &Pc) INLINE_LAMBDA {
+    // Hn: H of plane i, then <- H of plane i+1, Pc <- psi of plane i
+    auto step = [&](int i, ESet &C, ESet &N, ESet &Fr, HSet &Hn, PSet &Pc) INLINE_LAMBDA {
         const bool more = i + 1 < i1;
         const int buf = (i - i0) & 1;
         const unsigned pl = (unsigned)(i + 1) * sxy4;
@@ -1338,6 +1338,7 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
         // plane i, which is cached) so the wait counts after them are exact
         load_psi(i, Pc);
         load_e(more ? i + 2 : i, Fr);
+        const HSet Hc = Hn;
         load_h(more ? i + 1 : i, Hn);
         float hx[R + 1], hy[R + 1], hz[R + 1], exk[R + 1], eyk[R + 1], zx[R + 1], zy[R + 1];
         if constexpr (ADJ) {
@@ -1449,13 +1450,15 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
             for (int r = 0; r <= R; r++) { hyP[r] = hy[r]; hzP[r] = hz[r]; }
         }
     };
-    for (int i = i0;;) {
-        step(i, EA, EB, EC, H0, H1, P0); if (++i >= i1) break;
-        step(i, EB, EC, EA, H1, H0, P0); if (++i >= i1) break;
-        step(i, EC, EA, EB, H0, H1, P0); if (++i >= i1) break;
-        step(i, EA, EB, EC, H1, H0, P0); if (++i >= i1) break;
-        step(i, EB, EC, EA, H0, H1, P0); if (++i >= i1) break;
-        step(i, EC, EA, EB, H1, H0, P0); if (++i >= i1) break;
+    // One copy of the step; the E sets move on by register copies (22 values).  Six
+    // copies with the sets' roles turned need no copies, but made k_step_all 222 kB of code (now 67), several times
+    // the instruction cache, and chunks of a few planes run most of it once: 37^3 21.9 us per step
+    // against 20.7, 85^3 34.0 against 32.9, 125 x 173 x 204 87.6 against 85.6, 281^3 351 against 348.
+#pragma clang loop unroll(disable)
+    for (int i = i0; i < i1; i++) {
+        step(i, EA, EB, EC, HN, P0);
+        EA = EB;
+        EB = EC;
     }
 }
 
@@ -2274,9 +2277,9 @@ __global__ __launch_bounds__(1024) void k_line(LineDev l) { line_body(l, l.t, th
 // others the pieces of the grid (corner columns, x slabs, y slabs, clean box),
 // each piece with its own x chunk.  Small grids are bound by the march (2-3 us
 // per plane whatever the grid) and by the packets between launches: on one
-// stream, with chunks of 1 to 4 planes, the step of a 37^3 grid takes 22 us
-// against 91 us with the pieces on four streams in chunks of 16, of 85^3 34
-// against 90, of 125 x 173 x 204 88 against 122.  Large grids are bound by
+// stream, with chunks of 1 to 4 planes, the step of a 37^3 grid takes 21 us
+// against 91 us with the pieces on four streams in chunks of 16, of 85^3 33
+// against 90, of 125 x 173 x 204 86 against 122.  Large grids are bound by
 // memory: at 281^3 the launch moves 1.56 GB (1.25 GB it cannot do without) in
 // 315 us, 4.9 TB/s, what a large copy reaches on this card.
 __device__ __forceinline__ void step_all_body(const StepAll &a, int t, int block, int nwaves) {
@@ -2297,7 +2300,8 @@ __device__ __forceinline__ void step_all_body(const StepAll &a, int t, int block
         default: rows_piece<2, true, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
     }
 }
-__global__ __launch_bounds__(64 * kRowsMaxWaves) void k_step_all(StepAll) {
+template <int MW>
+__global__ __launch_bounds__(64 * MW) void k_step_all(StepAll) {
     // the arguments in place (their only copy; a by-value struct indexed by piece would be copied to scratch)
     const StepAll &a = batch_item((const StepAll *)(const CONST_AS StepAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
     step_all_body(a, a.line.t, (int)blockIdx.x, a.r.waves * a.r.tiles);
@@ -3377,7 +3381,9 @@ long step_all_blocks(StepAll &a) {
 hipError_t launch_step_all(StepAll a, hipStream_t st) {
     const long total = pieces_prepare(a, kRowsMaxWaves);
     if (total < 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_step_all, dim3((unsigned)(total + 1)), dim3(64, a.r.waves * a.r.tiles), 0, st, a);
+    const dim3 G((unsigned)(total + 1)), B(64, a.r.waves * a.r.tiles);
+    if (step_all_bound(B.y) == 12) hipLaunchKernelGGL(k_step_all<12>, G, B, 0, st, a);
+    else hipLaunchKernelGGL(k_step_all<16>, G, B, 0, st, a);
     return hipGetLastError();
 }
 
