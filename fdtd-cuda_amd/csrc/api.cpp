@@ -350,7 +350,7 @@ int contract(fdtd_sim *s) {
     } else {
         const int parts = s->S.P.dft_exact == 2 ? 3 : 2;
         HIPCHK(s, launch_twiddle_frag(s->Wf, s->slot_t.data(), s->K, s->slot, F, s->freq_d, s->S.dt, parts, s->stream));
-        HIPCHK(s, launch_dft_mfma(s->X, s->Wf, s->acc, s->mtot, s->fd.mE_pad, s->K, F, parts, s->stream));
+        HIPCHK(s, launch_dft_mfma(s->X, s->Wf, s->acc, s->mtot, s->fd.mE_pad, s->K, s->slot, F, parts, s->stream));
     }
     if (timed) {
         HIPCHK(s, hipEventRecord(next_event(s, 1), s->stream));

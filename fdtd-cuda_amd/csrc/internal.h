@@ -321,8 +321,8 @@ hipError_t launch_dft_contract(const float *X, const double *W, double *acc, lon
 // (2 * ceil(K/16) * ceil(2F/32) * parts * 64 * 16 bytes) and contraction.
 hipError_t launch_twiddle_frag(void *Wf, const int *t_slot_host, int K, int nvalid, int F, const double *freq,
                                double dt, int parts, hipStream_t st);
-hipError_t launch_dft_mfma(const float *X, const void *Wf, double *acc, long mtot, long mE_pad, int K, int F, int parts,
-                           hipStream_t st);
+hipError_t launch_dft_mfma(const float *X, const void *Wf, double *acc, long mtot, long mE_pad, int K, int nvalid, int F,
+                           int parts, hipStream_t st);
 hipError_t launch_flux_reduce(const double *acc, const FaceDev &fd, long mtot, long mE_pad, int F, double dA,
                               double *out, hipStream_t st);
 hipError_t launch_pack_field(const float *f, const Geom &g, float *dense, int to_dense, hipStream_t st);

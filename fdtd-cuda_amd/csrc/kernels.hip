@@ -2394,13 +2394,15 @@ __device__ inline float from_bf16(__bf16 b) {
 // Split of a value into P BF16 parts v ~ p0 + p1 + ... (each the rounded
 // remainder of the previous ones): two parts carry ~16 significant bits,
 // three ~24 (FP32).
-template <int P>
-__device__ inline void split_bf16(double v, __bf16 *out) {
-    double r = v;
+// The remainders of a float are floats (they keep its last place and have at
+// most 16 bits), so T = float gives the parts that T = double gives.
+template <int P, typename T>
+__device__ inline void split_bf16(T v, __bf16 *out) {
+    T r = v;
 #pragma unroll
     for (int q = 0; q < P; q++) {
         out[q] = to_bf16((float)r);
-        r -= (double)from_bf16(out[q]);
+        r -= (T)from_bf16(out[q]);
     }
 }
 
@@ -2445,9 +2447,20 @@ __global__ void k_twiddle_frag(bf16x8 *Wf, SlotTimes ts, int nks, int nmt, int n
 // m-tiles.  B operand: lane l holds column l % 32, slots 16 ks + 8 (l / 32)
 // + j.  C/D: lane l holds column l % 32, rows 8 i + 4 (l / 32) + j in
 // element 4 i + j.
+//
+// Bound by the accumulator's way through memory (16 bytes per row and column,
+// against 4 per slot and column of samples).  Only the used k-steps run
+// (slots past them hold zero twiddles), the samples of a k-step are loaded
+// while the one before is multiplied, and the accumulator of an m-tile is
+// loaded whole before any of it is stored (loads and stores in turn are a
+// chain of 16 memory latencies a tile, as the compiler must keep their order),
+// the first one before the products.  us per contraction, before and after, blocks
+// of 64 slots: 281^3 grid, 64 frequencies, every slot used 2218 and 1261 (5.5 GB at
+// 4.4 TB/s); 8 frequencies, 6 slots 695 and 187; 409^3, 24 frequencies, 16 slots 2651
+// and 978; 125 x 173 x 204, 32 frequencies, 24 slots, three parts 408 and 172.
 template <int P>
 __global__ __launch_bounds__(256) void k_dft_mfma(const float *X, const bf16x8 *Wf, double *acc, long mtot,
-                                                 long mE_pad, int nks, int nmt, int rows) {
+                                                 long mE_pad, int nks, int used, int nmt, int rows) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
     const long col0 = ((long)blockIdx.x * 4 + w) * 32;
     if (col0 >= mtot) return;
@@ -2456,19 +2469,32 @@ __global__ __launch_bounds__(256) void k_dft_mfma(const float *X, const bf16x8 *
     const int nm = min(4, nmt - 4 * mg);
     const long col = col0 + (l & 31);
     const bool cok = col < mtot;
+    const long cc = cok ? col : mtot - 1;
+    auto load_x = [&](int ks, float *x) INLINE_LAMBDA {
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = X[(long)(16 * ks + 8 * (l >> 5) + j) * mtot + cc];
+    };
+    auto row_of = [&](int q, int e) INLINE_LAMBDA { return 32 * (4 * mg + q) + 8 * (e >> 2) + 4 * (l >> 5) + (e & 3); };
+    auto load_acc = [&](int q, double *d) INLINE_LAMBDA {
+#pragma unroll
+        for (int e = 0; e < 16; e++) d[e] = __builtin_nontemporal_load(&acc[(long)min(row_of(q, e), rows - 1) * mtot + cc]);
+    };
     f32x16 c[4];
 #pragma unroll
     for (int q = 0; q < 4; q++)
 #pragma unroll
         for (int e = 0; e < 16; e++) c[q][e] = 0.f;
-    for (int ks = 0; ks < nks; ks++) {
+    float x[8], xn[8];
+    double d[16];
+    load_x(0, x);
+    load_acc(0, d);
+    for (int ks = 0; ks < used; ks++) {
+        load_x(min(ks + 1, used - 1), xn);
         bf16x8 b[P];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const int sidx = 16 * ks + 8 * (l >> 5) + j;
-            const float x = cok ? X[(long)sidx * mtot + col] : 0.f;
             __bf16 bs[P];
-            split_bf16<P>((double)x, bs);
+            split_bf16<P>(x[j], bs);
 #pragma unroll
             for (int q = 0; q < P; q++) b[q][j] = bs[q];
         }
@@ -2489,18 +2515,23 @@ __global__ __launch_bounds__(256) void k_dft_mfma(const float *X, const bf16x8 *
                 }
             }
         }
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = xn[j];
     }
-    if (!cok) return;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         if (q >= nm) continue;
+        double dn[16];
+        if (q + 1 < nm) load_acc(q + 1, dn);
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int e = 0; e < 16; e++) {
+            const int r = row_of(q, e);
+            if (cok && r < rows) __builtin_nontemporal_store(d[e] + (double)c[q][e], &acc[(long)r * mtot + col]);
+        }
+        if (q + 1 < nm) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = 32 * (4 * mg + q) + 8 * i + 4 * (l >> 5) + j;
-                if (r < rows) acc[(long)r * mtot + col] += (double)c[q][4 * i + j];
-            }
+            for (int e = 0; e < 16; e++) d[e] = dn[e];
+        }
     }
 }
 
@@ -3617,15 +3648,17 @@ hipError_t launch_twiddle_frag(void *Wf, const int *t_slot_host, int K, int nval
     return hipGetLastError();
 }
 
-hipError_t launch_dft_mfma(const float *X, const void *Wf, double *acc, long mtot, long mE_pad, int K, int F, int parts,
-                           hipStream_t st) {
-    if (parts != 2 && parts != 3) return hipErrorInvalidValue;
-    const int nks = (K + 15) / 16, nmt = (2 * F + 31) / 32;
+hipError_t launch_dft_mfma(const float *X, const void *Wf, double *acc, long mtot, long mE_pad, int K, int nvalid, int F,
+                           int parts, hipStream_t st) {
+    if ((parts != 2 && parts != 3) || nvalid < 1 || nvalid > K) return hipErrorInvalidValue;
+    const int nks = (K + 15) / 16, used = (nvalid + 15) / 16, nmt = (2 * F + 31) / 32;
     dim3 grid((unsigned)((mtot + 127) / 128), (nmt + 3) / 4), block(256);
     if (parts == 2)
-        hipLaunchKernelGGL(k_dft_mfma<2>, grid, block, 0, st, X, (const bf16x8 *)Wf, acc, mtot, mE_pad, nks, nmt, 2 * F);
+        hipLaunchKernelGGL(k_dft_mfma<2>, grid, block, 0, st, X, (const bf16x8 *)Wf, acc, mtot, mE_pad, nks, used, nmt,
+                           2 * F);
     else
-        hipLaunchKernelGGL(k_dft_mfma<3>, grid, block, 0, st, X, (const bf16x8 *)Wf, acc, mtot, mE_pad, nks, nmt, 2 * F);
+        hipLaunchKernelGGL(k_dft_mfma<3>, grid, block, 0, st, X, (const bf16x8 *)Wf, acc, mtot, mE_pad, nks, used, nmt,
+                           2 * F);
     return hipGetLastError();
 }
 
