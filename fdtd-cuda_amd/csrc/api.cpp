@@ -536,6 +536,8 @@ int plan_rows(fdtd_sim *s) {
     if (const char *v = std::getenv("FDTD_EARLY")) s->early = std::atoi(v) != 0;
     if (const char *v = std::getenv("FDTD_TILES")) s->tiles = std::min(3, std::max(1, std::atoi(v)));
     if (const char *v = std::getenv("FDTD_STILES")) s->stiles = std::atoi(v) == 2 ? 2 : 1;
+    s->one_tiles = s->tiles ? s->tiles : one_launch_tiles(s->g.NZ);
+    if (s->one_tiles * rows_waves(s->g.NZ) > kRowsMaxWaves) s->one_tiles = 1;
     if (!s->tiles) s->tiles = rows_tiles(s->g.NZ);
     // x chunk of the clean box: 16, or 32 for two-tile blocks when that still
     // leaves at least 512 blocks (two per CU; fewer prologue planes, measured
@@ -569,19 +571,20 @@ int plan_rows(fdtd_sim *s) {
             return set_err(s, FDTD_ERR_DEVICE, "side streams or events could not be created");
     }
     s->use_rows = s->has_clean;
-    // One launch for the whole update up to 12 M cells, unless a knob of the stream schedule
+    // One launch for the whole update up to 50 M cells, unless a knob of the stream schedule
     // asks for that (FDTD_ONE_LAUNCH=0: the schedule with its defaults, 1: one launch whatever the size); two rows per thread
     // only.  Measured us per step, one launch against the streams: 21 and 91 at 0.05 M cells,
-    // 33 and 90 at 0.6 M, 86 and 121 at 4.4 M, 351 and 348 at 22 M, 929 and 907 at 68 M
-    // (there the post-update launch overlaps the next step's side pieces).
-    s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= 12000000L;
+    // 33 and 90 at 0.6 M, 86 and 121 at 4.4 M, 213 and 237 at 13 M, 354 and 357 at 22 M, 442 and 459
+    // at 29 M, 577 and 590 at 41 M, 663 and 675 at 49 M, 916 and 917 at 68 M (there the post-update
+    // launch overlaps the next step's side pieces).  The transposed step, forward and back 40 steps in ms:
+    // 18.4 and 20.6 at 14 M cells, 26.3 and 28.9 at 21 M, 33.3 and 36.3 at 29 M, 50.6 and 52.2 at 47 M.
+    s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= 50000000L;
     if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = std::atoi(v) != 0;
     s->one_launch = s->one_launch && s->rows == 2;
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
                           "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
         if (std::getenv(k)) s->one_launch = false;
-    const int ot = s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1;
-    s->one_chunk = one_launch_chunk(s, ot, step_all_bound(ot * rows_waves(s->g.NZ)) / 4);
+    s->one_chunk = one_launch_chunk(s, s->one_tiles, step_all_bound(s->one_tiles * rows_waves(s->g.NZ)) / 4);
     return FDTD_OK;
 }
 
@@ -620,6 +623,12 @@ RowsArgs make_rows(fdtd_sim *s) {
 // waves, so a block holds at most 10; with 8-wave columns the 16-wave block
 // of two tiles measured slower than two 8-wave blocks per CU.
 int rows_tiles(int NZ) { return rows_waves(NZ) <= 5 ? 2 : 1; }
+// Row tiles of the steps in one launch: two also where a column is 6 waves.
+// Forward (us per step, 1 and 2 tiles) 341^3 570 and 564, 365^3 658 and 654; on
+// streams one tile stays better there, 584 and 602.  The transposed step has
+// three waves per SIMD, so a block of 6 waves would be alone on its compute
+// unit: 341^3 685 and 536.
+int one_launch_tiles(int NZ) { return rows_waves(NZ) <= 6 ? 2 : 1; }
 
 // Whether the TFSF fix may run right after the clean-box kernel, before the
 // side pieces finish: its cells (planes t0-1, t0, t1, t1+1 of each axis over
@@ -853,7 +862,7 @@ StepAll make_step_all(fdtd_sim *s, const LineDev &l, int tiles, int chunk) {
 // post-update launch.
 int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const DispDev *dd, bool samp, bool *disp_done,
                       bool *samp_done, hipEvent_t ev0, hipEvent_t ev1) {
-    const StepAll a = make_step_all(s, l, s->tiles * rows_waves(s->g.NZ) <= kRowsMaxWaves ? s->tiles : 1, s->one_chunk);
+    const StepAll a = make_step_all(s, l, s->one_tiles, s->one_chunk);
     if (ev0) HIPCHK(s, hipEventRecord(ev0, s->stream));
     HIPCHK(s, launch_step_all(a, s->stream));
     if (ev1) HIPCHK(s, hipEventRecord(ev1, s->stream));
@@ -1353,7 +1362,7 @@ int adj_alloc(fdtd_sim *s) {
             s->adj.rows_slabs = !(sl && std::string(sl) == "general");
             // every piece in one launch where fdtd_step runs that way too, unless a knob of the
             // transposed step's schedule or tiles is set
-            s->adj.one_launch = s->one_launch && rows_waves(NZ) * rows_tiles(NZ) <= kAdjAllMaxWaves;
+            s->adj.one_launch = s->one_launch && rows_waves(NZ) * one_launch_tiles(NZ) <= kAdjAllMaxWaves;
             for (const char *k : {"FDTD_ADJ_SLABS", "FDTD_ADJ_SCHUNK", "FDTD_ADJ_RCHUNK", "FDTD_ADJ_SCHED", "FDTD_ADJ_TILES",
                                   "FDTD_ADJ_ROWS", "FDTD_ADJ_CTJ", "FDTD_ADJ_CICH", "FDTD_ADJ_CORNER_ROWS", "FDTD_ADJ_CRCHUNK",
                                   "FDTD_ADJ_CCHUNK", "FDTD_ADJ_STILES", "FDTD_ADJ_FUSE_INJECT", "FDTD_ADJ_EARLY", "FDTD_ADJ_STJ"})
@@ -1487,7 +1496,7 @@ int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, cons
     if (s->adj.one_launch) {
         AdjAll a{};
         a.r = adj_rows_args(s, pa, pe, ph);
-        a.r.tiles = rows_tiles(s->g.NZ);
+        a.r.tiles = one_launch_tiles(s->g.NZ);
         a.ad = ad;
         add_pieces(s, a, one_launch_chunk(s, a.r.tiles, 3));
         HIPCHK(s, launch_adj_all(a, s->stream));

@@ -110,7 +110,7 @@ struct fdtd_sim {
     unsigned *aux_d = nullptr;      // table image of the row-blocked kernel
     std::vector<uint32_t> aux_img;  // host copy of it
     bool one_launch = false;        // field update of fdtd_step in one launch (k_step_all), not on streams
-    int one_chunk = 1;              // its x chunk
+    int one_chunk = 1, one_tiles = 1;   // its x chunk and row tiles
     bool concurrent = true;         // side slabs on a second stream beside the clean box (FDTD_CONCURRENT=0 to serialise)
     hipStream_t stream2 = nullptr;
     // ev_line: the 1D line's completion in a step; the transposed step reuses it
@@ -225,6 +225,7 @@ RowsArgs make_rows(fdtd_sim *s);
 // Cell-set tests of the two-stream schedule (the clean box and the TFSF,
 // dispersive and monitor cells; see api.cpp).
 int rows_tiles(int NZ);
+int one_launch_tiles(int NZ);
 bool tfsf_in_clean(const fdtd_sim *s);
 bool disp_in_clean(const fdtd_sim *s);
 bool tfsf_off_clean_edges(const fdtd_sim *s);
