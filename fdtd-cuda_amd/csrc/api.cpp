@@ -1469,7 +1469,8 @@ RowsArgs adj_rows_args(fdtd_sim *s, int pa, int pe, int ph) {
 // the dispersive cells, which reads the box state it writes).  next: the
 // injection of the following step, folded into this step's correction when
 // it is on (the caller turns it on only where the objective cell lies in the
-// clean box, which no side launch writes); *injected reports whether it was.
+// clean box, which no side launch writes), or into the general kernel where
+// that runs the whole grid; *injected reports whether it was.
 int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, const AdjInject &next, bool *injected) {
     AdjDev av{};
     const StepDev sd = make_step(s, false);
@@ -1489,6 +1490,8 @@ int adjoint_step(fdtd_sim *s, int pa, int pe, int ph, const AdjDispDev &ad, cons
     *injected = false;
     if (!s->adj.rows) {
         const int full[1][4] = {{0, s->g.NX, 0, s->g.NY}};
+        av.inj = next;
+        *injected = next.on != 0;
         HIPCHK(s, launch_adj_disp(ad, s->stream));
         HIPCHK(s, launch_adj_step(av, s->tj, s->ichunk ? s->ichunk : general_chunk(s, 62), full, 1, s->stream));
         return FDTD_OK;
@@ -1777,7 +1780,7 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
             ad.grad = s->adj.grad;
             ad.Ceh = (float)S.Ceh;
             ad.Cee = (float)S.Cee;
-            const AdjInject nx = fuse && t > t0 ? inject_at(t - 1) : AdjInject{};
+            const AdjInject nx = (fuse || !s->adj.rows) && t > t0 ? inject_at(t - 1) : AdjInject{};
             if ((rc = adjoint_step(s, pa, pe, ph, ad, nx, &injected))) return rc;
             pa ^= 1; pe ^= 1; ph ^= 1;
         }

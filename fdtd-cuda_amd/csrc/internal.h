@@ -133,6 +133,16 @@ struct DispDev {
     float nl_e, nl_p, nl_i2;        // d_NL eps0 / C_E, d_NL, 1/dx^2
 };
 
+// The objective's injection dJ/dE at one cell, added to the E adjoint by
+// k_adj_inject, or by the step before after its own update of that cell: in
+// its dispersive-cell correction, or in k_adj_step where that runs the grid.
+struct AdjInject {
+    long p0;                        // cell (field layout)
+    float a[3];
+    int on;
+    int inside;                     // p0 lies in the cells of the correction launch
+};
+
 // Adjoint step arguments.  The transposed step has the stencil shape of the
 // forward step: the adjoint of H^{n+1/2} gathers forward differences of the
 // E-side weights V, the adjoint of E^n gathers backward differences of the
@@ -150,16 +160,7 @@ struct AdjDev {
     const float *Qb[3], *Eb[3];
     // per box cell, Qb - Ceh Ehat and Eb - Cee Ehat (zero at cells that are not dispersive)
     const float *dq[3], *db[3];
-};
-
-// The objective's injection dJ/dE at one cell, added to the E adjoint by
-// k_adj_inject, or folded into the dispersive-cell correction of the step
-// before (after its own update of that cell).
-struct AdjInject {
-    long p0;                        // cell (field layout)
-    float a[3];
-    int on;
-    int inside;                     // p0 lies in the cells of the correction launch
+    AdjInject inj;                  // k_adj_step over the whole grid: of the following step
 };
 
 // Adjoint of the dispersive update on the box (run before k_adj_step).
