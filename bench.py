@@ -135,7 +135,9 @@ def main():
     ms_step = (wall * 1e3 - in_window * contraction_ms) / args.steps + contraction_ms / (K * stride)
     value = cells / (ms_step * 1e-3) / 1e6
     abytes = algorithmic_bytes(info, p)
-    kbytes = cbytes if cbytes else abytes
+    # one launch runs the whole grid (tile's last entry 0): no launch of the clean box alone
+    one = rows and info.tile[6] == 0
+    kbytes = cbytes if cbytes and not one else abytes
     k_avg_s = (k_ms / 1e3) / max(k_n, 1)
     achieved = kbytes / k_avg_s / 1e9
     u_avg_s = (u_ms / 1e3) / max(u_n, 1)
@@ -144,7 +146,7 @@ def main():
     # the same kernel with the side pieces on the main stream after it (one
     # stream), so its duration is not shared with them: reported beside the
     # roofline figure, which is the production two-stream schedule
-    serial = serial_kernel_ms(p, max(64, args.steps // 8)) if cbytes else None
+    serial = serial_kernel_ms(p, max(64, args.steps // 8)) if cbytes and not one else None
     if args.calibrate_copy:
         copy_calibration()
     # the 32-simulation sweep last: after its allocations and frees the device
@@ -186,13 +188,13 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "k_step_rows<clean>" if cbytes else ("k_step_rows" if rows else "k_fused_step"),
+            "kernel": "k_step_all" if one else "k_step_rows<clean>" if cbytes else ("k_step_rows" if rows else "k_fused_step"),
             "clean_box": list(info.clean),
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": traffic_per_launch(),
+            "traffic": traffic_per_launch("k_step_all" if one else "k_step_rows"),
             "bytes_per_launch": kbytes,
             "kernel_avg_ms": round(k_avg_s * 1e3, 5),
             "launches": k_n,
@@ -204,7 +206,7 @@ def main():
             # also holds the 1D line and, with schedule bits 1 and 2, the
             # dispersive box and the DFT sample (every fourth step), whose bytes
             # are not counted (the figure is a lower bound)
-            "kernels": ("k_line + k_step_rows + k_fused_step (corners) + "
+            "kernels": (("k_step_all (with the 1D line) + " if one else "k_line + k_step_rows + k_fused_step (corners) + ")
                         + ("k_post (TFSF fix-up" + (" + dispersive box" if info.schedule & 2 else "")
                            + (" + DFT sample" if info.schedule & 4 else "") + ")"
                            if info.schedule & 6 else "k_tfsf_fix")) if rows else "k_fused_step",
@@ -244,11 +246,11 @@ def serial_kernel_ms(p, steps):
     return ms / max(n, 1)
 
 
-def traffic_per_launch():
+def traffic_per_launch(kernel):
     """HBM bytes per launch of the dominant kernel from the committed PMC
     summary (FETCH_SIZE + WRITE_SIZE, scaled by the copy-kernel factor), or
     None when no such measurement is on file."""
-    path = os.path.join(ROOT, "profiles", "k_step_rows_dimer281_traffic.json")
+    path = os.path.join(ROOT, "profiles", kernel + "_dimer281_traffic.json")
     try:
         with open(path) as f:
             return json.load(f)["traffic_bytes_per_launch"]

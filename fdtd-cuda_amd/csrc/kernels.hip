@@ -1,14 +1,19 @@
 // HIP kernels of the FDTD hot path for gfx950 (MI355X).
 //
-// Fused fast path, one launch per time step:
-//   k_fused_step   H update + CPML psi_H + TFSF + E update + CPML psi_E +
-//                  DFT face sampling, marching along x through a (j,k) tile.
-//                  E and H are ping-ponged so every field is read once from
-//                  buffer A and written once to buffer B (48 B per vacuum cell).
-//   k_dispersive   Drude + 2 CP ADE on the dense box holding the metal; runs
-//                  after k_fused_step and overwrites E at dispersive cells.
-//   k_line         1D incident line (h_inc, e_inc, Mur, source) on device.
-//   k_dft_*        twiddle build, buffered DFT contraction, flux reduction.
+// A step: H update + CPML psi_H + E update + CPML psi_E in one pass, E and H
+// ping-ponged so every field is read once from buffer A and written once to
+// buffer B (48 B per vacuum cell), then what adds to it.
+//   k_step_all     the whole grid and the 1D line in one launch (up to 50 M
+//                  cells); k_step_rows the same pieces on streams; k_step_batch
+//                  over many simulations; k_adj_all the transposed step.
+//   k_fused_step   the same update on the general kernel, with TFSF and face
+//                  sampling, for grids that the row-blocked one does not take.
+//   k_post         TFSF, Drude + 2 CP ADE on the dense box holding the metal,
+//                  face samples.
+//   k_line         1D incident line (h_inc, e_inc, Mur, source) where it is
+//                  not block 0 of k_step_all.
+//   k_dft_*        twiddle build, buffered DFT contraction; k_flux, k_point_dft,
+//                  k_line_replay the sums of the read-outs.
 // Split path (reference call structure): k_split_h, k_tfsf_split, k_split_e,
 // k_dft_sample_split, sharing the per-cell device functions below.
 //
@@ -1252,10 +1257,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
 
     // Register sets: E^n of one plane (rows 0..R, and ex, ez of row R+1) and
     // H^{n-1/2} of one plane.  Step i uses E of planes i and i+1 and H of
-    // plane i, and loads E of plane i+2 and H of plane i+1 for later steps;
-    // the x march is unrolled six times over three E sets and two H sets so no
-    // set is copied while its loads are in flight.  psi of plane i is loaded at
-    // the top of step i (one set).
+    // plane i, and loads E of plane i+2 and H of plane i+1 for later steps.
+    // psi of plane i is loaded at the top of step i (one set).
     struct ESet { float x[R + 1], y[R + 1], z[R + 1], xj, zj; };
     struct HSet { float h[3][R + 1]; };
     float hyP[R + 1], hzP[R + 1];                         // H^{n+1/2} of plane i-1 (adjoint x slabs: Wyx, Wzx)
