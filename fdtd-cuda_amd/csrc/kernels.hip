@@ -2320,10 +2320,10 @@ __global__ __launch_bounds__(64 * MW) void k_step_all(StepAll) {
 // each simulation its line).  Grids of 2, 3, 4 and 6 waves a column share the
 // launch in blocks of 12 waves (6, 4, 3 and 2 row tiles): one launch for the
 // whole batch leaves one tail a step, and the taller blocks read fewer halo
-// rows.  us per step of 4, 12 and 32 rods (17, 56 and 147 M cells): 351, 1054
-// and 2671, with a launch per variant and column height on two streams 413,
-// 1162 and 2910.  The launch is bound by memory (909 of the 1075 us a step at 12
-// rods in a trace).
+// rows.  us per step of 4, 12 and 32 rods (17, 56 and 147 M cells): 343, 973
+// and 2556 (351, 1054 and 2671 with the march unrolled, on a slower card), with a
+// launch per variant and column height on two streams 413, 1162 and 2910.  The
+// launch is bound by memory (889 of the 960 us a step at 12 rods in a trace).
 template <int MW>
 __global__ __launch_bounds__(64 * MW) void k_step_batch(const StepAll *items, const unsigned *map, const int *dyn, int step_off) {
     const unsigned m = batch_map(map);
@@ -3123,9 +3123,9 @@ __global__ void k_adj_disp(AdjDispDev A) { adj_disp_body(A, (long)blockIdx.x * b
 // nd blocks run the transposed dispersive update (it reads the input level, and
 // no piece reads what it writes), the others the pieces.  The dispersive-cell
 // correction follows in a launch of its own.  120 steps forward and back on an
-// 81^3 grid take 10.0 ms with both directions in one launch each, 24.7 ms with
-// their pieces on four streams (121^3 14.9 and 26.0, 221^3 46.2 and 48.9); this
-// launch takes 32 us on the 81^3 grid, bound by the march.
+// 81^3 grid take 9.4 ms with both directions in one launch each, 24.7 ms with
+// their pieces on four streams (121^3 14.2 and 26.0, 221^3 43.4 and 48.9); this
+// launch takes 32 us on the 81^3 grid, bound by the march, 369 on 281^3, by memory.
 __global__ __launch_bounds__(64 * 12) void k_adj_all(AdjAll) {
     const AdjAll &a = batch_item((const AdjAll *)(const CONST_AS AdjAll *)__builtin_amdgcn_kernarg_segment_ptr(), 0);
     __shared__ RowsLds<2, true> lds;
