@@ -1876,11 +1876,21 @@ int fdtd_dft_accumulate(fdtd_sim *s) {
     return rc;
 }
 
+// Whether every monitor plane of a periodic run lies off the dispersive box.  A
+// layer starts behind the source plane and ends before the transmission plane,
+// but with a negative sca_offset the reflection plane lies behind the source
+// plane as well, and a layer may contain it.
+static bool planes_off_box(const fdtd_sim *s) {
+    for (int q : {4, 5})
+        if (s->fd.plane[q] >= s->box_lo[2] && s->fd.plane[q] < s->box_lo[2] + s->box_n[2]) return false;
+    return true;
+}
+
 // One periodic step (Periodic_XY): H with the source plane and the line, E
 // with the source plane, dispersive box and monitors; the reference's order
 // (main.cu:2724-2934) with its corrections folded into the updates.  Fields
-// update in place.  The layer's cells lie strictly between the two monitor
-// planes, so the sample shares the box's launch.
+// update in place.  The sample shares the box's launch where it reads no cell
+// that the box writes, and follows it otherwise.
 static int periodic_step(fdtd_sim *s) {
     const LineDev l = make_line(s);
     StepDev d = inplace_step(s, true);
@@ -1889,9 +1899,11 @@ static int periodic_step(fdtd_sim *s) {
     s->le ^= 1;
     const bool samp = sampling_step(s);
     if (samp) d.sample_row = s->X + (size_t)s->slot * s->mtot;
+    const bool together = samp && (!s->nbox || planes_off_box(s));
     DispDev dd{};
     if (s->nbox) dd = make_disp(s, s->p);
-    HIPCHK(s, launch_post(d, false, s->nbox ? &dd : nullptr, samp, s->stream));
+    HIPCHK(s, launch_post(d, false, s->nbox ? &dd : nullptr, together, s->stream));
+    if (samp && !together) HIPCHK(s, launch_dft_sample_split(d, s->stream));
     if (int rc = record_monitor(s)) return rc;
     const int rc = samp ? after_sample(s) : FDTD_OK;
     s->t++;

@@ -1,0 +1,61 @@
+"""The host code alone, on a machine without a GPU: the library runs in a child
+process over a stand-in for the HIP runtime (hip_stub.cpp), and the tests look
+at the kernels that a call launches and at the handle's own state."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PACKAGE = os.path.join(os.path.dirname(HERE), "fdtd-cuda_amd")
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("stub") / "hip_stub.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-o", so,
+                    os.path.join(HERE, "hip_stub.cpp")], check=True)
+    return so
+
+
+def run(stub, tmp_path, code, env=()):
+    """Launches of the code after its last mark() as (kernel, grid, block), and what it printed."""
+    log = tmp_path / "launches"
+    log.write_text("")
+    head = (f"import sys, ctypes; sys.path[:0] = [{PACKAGE!r}, {HERE!r}]\n"
+            "import fdtd_amd as G\nfrom conftest import small_params\n"
+            f"stub = ctypes.CDLL({stub!r})\nmark = lambda: open({str(log)!r}, 'w').close()\n")
+    kept = {k: v for k, v in os.environ.items() if not k.startswith("FDTD_")}
+    r = subprocess.run([sys.executable, "-c", head + code], capture_output=True, text=True, timeout=300,
+                       env={**kept, "LD_PRELOAD": stub, "HIP_STUB_LOG": str(log), **dict(env)})
+    assert r.returncode == 0, r.stderr
+    launches = [line.split("\t") for line in log.read_text().splitlines()]
+    return [(k, *(tuple(int(x) for x in v.split()) for v in (g, b))) for k, g, b in launches], r.stdout
+
+
+PERIODIC = """
+p = small_params(G, sphere=0)
+p.periodic_xy, p.NcpmlX, p.NcpmlY, p.NcpmlZ = 1, 0, 0, 8
+p.NCELLX, p.NCELLY, p.NCELLZ = 6, 5, 80
+p.tfsf_inset, p.sca_offset, p.dft_stride = 10, {offset}, 1
+s = G.Simulation(p)
+k0 = s.info.tfsf[2] + {at}
+s.add_layer(k0, k0 + {thick})
+mark()
+s.step(1)
+"""
+
+
+@pytest.mark.parametrize("offset,at,thick,apart", [(5, 1, 4, True), (-3, 1, 5, False), (-3, 3, 1, False), (-3, 2, 1, False),
+                                                   (-3, 4, 2, False), (-3, 5, 4, True), (-8, 1, 4, True)])
+def test_periodic_sample_follows_a_layer_on_its_plane(stub, tmp_path, offset, at, thick, apart):
+    """The reflection plane is tfsf - offset: on or beside the layer's box, the
+    sample is a launch after the box's; apart from it, they share one."""
+    launches, _ = run(stub, tmp_path, PERIODIC.format(offset=offset, at=at, thick=thick))
+    names = [k for k, _, _ in launches]
+    tail = ["k_post"] if apart else ["k_post", "k_dft_sample_split"]
+    assert names == ["k_per_h", "k_per_e"] + tail
+    cells = 6 * 5
+    blocks = -(-cells * (thick + 2) // 256) + (-(-4 * cells // 256) if apart else 0)
+    assert launches[2][1] == (blocks, 1, 1)
