@@ -1918,8 +1918,6 @@ int fdtd_step(fdtd_sim *s, int nsteps) {
     return fdtd_host::step_steps(s, nsteps);
 }
 
-// fdtd_step without clearing the early start: for loops of single steps that
-// launch nothing else between them (the adjoint's recorded steps).
 // Records (point monitor, objective probe) of a step are taken by the next
 // step's line launch; a launch of their own (5 us a step) only takes those of a
 // call's last step.
@@ -1934,9 +1932,8 @@ static int flush_records(fdtd_sim *s) {
     return FDTD_OK;
 }
 
-int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
+static int run_steps(fdtd_sim *s, int nsteps) {
     if (int rc = check_finite(s)) return rc;
-    if (!s->defer_records) s->rec_dst[0] = s->rec_dst[1] = nullptr;   // left by a call that failed
     if (s->S.P.periodic_xy) {
         for (int n = 0; n < nsteps; n++)
             if (int rc = periodic_step(s)) return rc;
@@ -2013,6 +2010,21 @@ int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
         s->t++;
     }
     return s->defer_records ? FDTD_OK : flush_records(s);
+}
+
+// fdtd_step without clearing the early start: for loops of single steps that
+// launch nothing else between them (the adjoint's recorded steps).
+int fdtd_host::step_steps(fdtd_sim *s, int nsteps) {
+    const int rc = run_steps(s, nsteps);
+    if (rc) {
+        // the records of the steps before the one that failed, now: their buffer may be
+        // freed by the next call, and a later launch would write to it
+        const std::string why = s->err;
+        (void)flush_records(s);
+        s->rec_dst[0] = s->rec_dst[1] = nullptr;
+        s->err = why;
+    }
+    return rc;
 }
 
 int fdtd_set_point_monitor(fdtd_sim *s, const int r[3], int capacity) {

@@ -25,7 +25,8 @@ def run(stub, tmp_path, code, env=()):
     log.write_text("")
     head = (f"import sys, ctypes; sys.path[:0] = [{PACKAGE!r}, {HERE!r}]\n"
             "import fdtd_amd as G\nfrom conftest import small_params\n"
-            f"stub = ctypes.CDLL({stub!r})\nmark = lambda: open({str(log)!r}, 'w').close()\n")
+            f"stub = ctypes.CDLL({stub!r})\nmark = lambda: open({str(log)!r}, 'w').close()\n"
+            f"launched = lambda kernel: open({str(log)!r}).read().count(kernel)\n")
     kept = {k: v for k, v in os.environ.items() if not k.startswith("FDTD_")}
     r = subprocess.run([sys.executable, "-c", head + code], capture_output=True, text=True, timeout=300,
                        env={**kept, "LD_PRELOAD": stub, "HIP_STUB_LOG": str(log), **dict(env)})
@@ -59,3 +60,29 @@ def test_periodic_sample_follows_a_layer_on_its_plane(stub, tmp_path, offset, at
     cells = 6 * 5
     blocks = -(-cells * (thick + 2) // 256) + (-(-4 * cells // 256) if apart else 0)
     assert launches[2][1] == (blocks, 1, 1)
+
+
+@pytest.mark.parametrize("env", [{}, {"FDTD_ONE_LAUNCH": "0"}, {"FDTD_PATH": "general"}])
+def test_a_failed_step_leaves_no_record_behind(stub, tmp_path, env):
+    """Whichever launch of three steps fails, the handle holds no pointer into
+    the point monitor's buffer afterwards, and the records of the steps before
+    are taken."""
+    launches, out = run(stub, tmp_path, """
+for n in range(1, 40):
+    s = G.Simulation(small_params(G))
+    s.set_point_monitor((5, 6, 7), 10)
+    mark()
+    stub.stub_fail_launch(n)
+    try:
+        s.step(3)
+    except G.FDTDError as e:
+        assert 'stub error' in str(e)
+        print(n, stub.stub_pending_records(s.h), launched('k_probe'))
+    else:
+        break
+    s.close()
+""", env)
+    rows = [tuple(map(int, line.split())) for line in out.splitlines()]
+    assert len(rows) >= 7
+    assert all(pending == 0 for _, pending, _ in rows), rows
+    assert rows[0][2] == 0 and rows[-2][2] == 1, rows   # the last launch of all is the record's own
