@@ -578,7 +578,7 @@ int plan_rows(fdtd_sim *s) {
     // at 29 M, 577 and 590 at 41 M, 663 and 675 at 49 M, 916 and 917 at 68 M (there the post-update
     // launch overlaps the next step's side pieces).  The transposed step, forward and back 40 steps in ms:
     // 18.4 and 20.6 at 14 M cells, 26.3 and 28.9 at 21 M, 33.3 and 36.3 at 29 M, 50.6 and 52.2 at 47 M.
-    s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= 50000000L;
+    s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= kOneLaunchCells;
     if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = std::atoi(v) != 0;
     s->one_launch = s->one_launch && s->rows == 2;
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",

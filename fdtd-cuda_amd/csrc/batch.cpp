@@ -330,9 +330,12 @@ void add_blocks(Launch &l, int sim, long n) {
 }
 
 // Waves per block of the one-launch step for W waves a column: 12 where the
-// columns of several row tiles fill that (and for 5 waves, two tiles in 12), else
-// one column; and its row tiles.
-int one_waves(int W) { return W <= 6 ? 12 : W; }
+// columns of several row tiles fill that, three columns of 5 waves, else one
+// column; and its row tiles.  Columns of 5 waves in blocks of 12, 10 and 15 (12
+// and 10 leave every compute unit two of its waves short), us per step: 4 grids of
+// 221 x 221 x 270 844, 807 and 794, 3 of 261^3 867, 830 and 809, 4 of 61 x 61 x
+// 260 130, 124 and 128.
+int one_waves(int W) { return W == 5 ? 15 : (W <= 6 ? 12 : W); }
 int one_tiles(int W) { return one_waves(W) / W; }
 
 // Uploads every per-simulation argument for both parities and rebuilds the
@@ -659,11 +662,16 @@ int fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out)
     if (int rc = check_sims(b)) return fail(rc);
     if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(berr(b, FDTD_ERR_DEVICE, "hipStreamCreate failed"));
-    b->one = !(flags & FDTD_BATCH_GENERAL);
-    for (fdtd_sim *s : b->sims) b->one = b->one && s->use_rows && s->rows == 2;
+    // One launch by fdtd_step's rule, for every simulation.  us per step, one launch against the
+    // launches per variant: 6 of 61 x 61 x 390 236 and 277, 4 of 181^3 414 and 476, 4 of 301^3
+    // 1533 and 1516, 3 of 365^3 1908 and 1918, 2 of 240 x 240 x 800 (46 M cells) 1324 and 1260,
+    // 2 of 390^3 (59 M) 1597 and 1584, 2 of 301 x 301 x 800 (72 M) 2006 and 1921.
+    const char *one = std::getenv("FDTD_ONE_LAUNCH");
+    b->one = !(flags & FDTD_BATCH_GENERAL) && (!one || std::atoi(one) != 0);
+    for (fdtd_sim *s : b->sims)
+        b->one = b->one && s->use_rows && s->rows == 2 && (one || (long)s->g.NX * s->g.NY * s->g.NZ <= kOneLaunchCells);
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_SIDE_STREAMS", "FDTD_BATCH_EARLY", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_CTJ"})
         if (std::getenv(k)) b->one = false;
-    if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) b->one = b->one && std::atoi(v) != 0;
     const char *conc = std::getenv("FDTD_CONCURRENT");
     if (!conc || std::atoi(conc) != 0) {
         if (hipStreamCreateWithFlags(&b->stream2, hipStreamNonBlocking) != hipSuccess ||

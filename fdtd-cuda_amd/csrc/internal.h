@@ -275,8 +275,9 @@ hipError_t launch_step_all(StepAll a, hipStream_t st);
 // The block bound of the instance that a block of so many waves runs.  Bound to 12 waves the kernel has 136
 // registers and three waves per SIMD; bound to 16 it has 128, four waves and 28 bytes per thread in scratch
 // memory.  The first, unless its blocks need two waves of every SIMD (or four), where it holds half as
-// many (or none): us per step, 12 against 16, in blocks of 2 waves (37^3) 20.7 and 21.3, of 4 (85^3) 32.6
-// and 33.5, of 10 (281^3) 367 and 373; of 8 (125 x 173 x 204) 92 and 89.
+// many (or none): us per step, 12 against 16, in blocks of 4 waves (37^3) 20.7 and 21.3, (85^3) 32.6
+// and 33.5, of 10 (281^3) 367 and 373; of 8 (125 x 173 x 204) 92 and 89.  A batch the same, in blocks of 8
+// waves: 6 grids of 141 x 141 x 400 851 and 763, 2 of 390^3 1767 and 1597.
 inline int step_all_bound(int waves) { return (waves + 3) / 4 % 2 ? 12 : 16; }
 // Fills in start and the wave counts; the blocks of the launch (line and pieces) or -1.
 long step_all_blocks(StepAll &a);

@@ -212,6 +212,8 @@ int upload(fdtd_sim *s, T **ptr, const std::vector<T> &v) {
     return FDTD_OK;
 }
 
+// Cells of the largest grid whose field update is one launch (measured: plan_rows).
+constexpr long kOneLaunchCells = 50000000;
 // One-launch step: the x chunk for `columns` blocks per chunk layer of NX planes
 // and `slots` resident blocks, and the arguments at the handle's parity.
 int march_chunk(long columns, int NX, long slots, int most);

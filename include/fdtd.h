@@ -324,9 +324,9 @@ int  fdtd_kernel_timing(fdtd_sim *sim, int enable, double *total_ms, long *launc
  * the launches of one DFT sampling period are captured in a HIP graph and
  * replayed.  The field update is fdtd_step's: the row-blocked kernel with the
  * TFSF fix-up where the simulation's grid allows it, else the general fused
- * kernel.  Where every simulation has the row-blocked kernel, its pieces and
- * the 1D lines of all of them are one launch, its x chunk chosen by the batch's
- * cells.  Else the tile of each grid size's dominant launch is picked by the
+ * kernel.  Where every simulation has the row-blocked kernel and at most 50 M
+ * cells, its pieces and the 1D lines of all of them are one launch per column
+ * height, its x chunk chosen by the batch's cells.  Else the tile of each grid size's dominant launch is picked by the
  * autotuner (timed on the device at fdtd_batch_create, remembered per process
  * and, when the environment variable FDTD_TUNE_FILE names a file, across
  * processes).

@@ -86,3 +86,41 @@ for n in range(1, 40):
     assert len(rows) >= 7
     assert all(pending == 0 for _, pending, _ in rows), rows
     assert rows[0][2] == 0 and rows[-2][2] == 1, rows   # the last launch of all is the record's own
+
+
+@pytest.mark.parametrize("nz,kernel,waves", [(24, "k_step_batch<12>", 12), (200, "k_step_batch<12>", 12), (270, "k_step_batch<16>", 15),
+                                             (330, "k_step_batch<12>", 12), (400, "k_step_batch<16>", 8),
+                                             (600, "k_step_batch<12>", 12), (800, "k_step_batch<16>", 16)])
+def test_batch_blocks_fill_a_compute_unit(stub, tmp_path, nz, kernel, waves):
+    """Blocks of the batched one-launch step by column height: 5 waves a column
+    in blocks of 15, and the instance by the waves that fit a compute unit."""
+    launches, _ = run(stub, tmp_path, f"""
+p = small_params(G, sphere=0)
+p.NCELLZ = {nz}
+s = [G.Simulation(p) for _ in range(2)]
+b = G.Batch(s, flags=G.BATCH_NO_GRAPH)
+mark()
+b.run(1)
+""")
+    assert launches[0][0] == kernel and launches[0][2] == (64, waves, 1), launches
+
+
+@pytest.mark.parametrize("n,one", [((350, 364), True), ((354, 364), False)])
+def test_batch_leaves_one_launch_where_fdtd_step_does(stub, tmp_path, n, one):
+    """One launch for a batch only up to the 50 M cells a simulation that fdtd_step's rule has."""
+    launches, out = run(stub, tmp_path, f"""
+sims = []
+for nx, nz in ((24, 24), {n}):
+    p = small_params(G, sphere=0, nfreq=1)
+    p.NCELLX = p.NCELLY = nx
+    p.NCELLZ = nz
+    sims.append(G.Simulation(p))
+print(sims[1].info.NX * sims[1].info.NY * sims[1].info.NZ, sims[1].get_info().tile[6])
+b = G.Batch(sims, flags=G.BATCH_NO_GRAPH | G.BATCH_NO_TUNE)
+mark()
+b.run(1)
+""")
+    cells, streams = map(int, out.split())
+    assert (cells <= 50_000_000) == one and (streams == 0) == one
+    assert any(k.startswith("k_step_batch") for k, _, _ in launches) == one, launches
+    assert any(k.startswith("k_rows_batch") for k, _, _ in launches) != one
