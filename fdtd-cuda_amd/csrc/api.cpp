@@ -1733,7 +1733,9 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
         return v;
     };
     // the injection of step t-1 rides on the dispersive-cell correction of step t
-    // where the objective cell lies in the clean box (written there by the clean box alone)
+    // where the objective cell lies in the clean box (written there by the clean box alone),
+    // or on the general transposed kernel where that runs the whole grid
+    const bool fuse_general = !s->adj.rows && s->adj_fuse_inject;
     const bool fuse = s->adj.rows && s->nbox > 0 && s->adj_fuse_inject && r0[0] >= s->cbox[0] &&
                       r0[0] < s->cbox[1] && r0[1] >= s->cbox[2] && r0[1] < s->cbox[3];
     // the next step's slabs may start before this step's correction is added
@@ -1780,7 +1782,7 @@ int adjoint_run(fdtd_sim *s, AdjScratch &W, int nsteps, int ckpt, const int r0[3
             ad.grad = s->adj.grad;
             ad.Ceh = (float)S.Ceh;
             ad.Cee = (float)S.Cee;
-            const AdjInject nx = (fuse || !s->adj.rows) && t > t0 ? inject_at(t - 1) : AdjInject{};
+            const AdjInject nx = (fuse || fuse_general) && t > t0 ? inject_at(t - 1) : AdjInject{};
             if ((rc = adjoint_step(s, pa, pe, ph, ad, nx, &injected))) return rc;
             pa ^= 1; pe ^= 1; ph ^= 1;
         }

@@ -124,3 +124,23 @@ b.run(1)
     assert (cells <= 50_000_000) == one and (streams == 0) == one
     assert any(k.startswith("k_step_batch") for k, _, _ in launches) == one, launches
     assert any(k.startswith("k_rows_batch") for k, _, _ in launches) != one
+
+
+@pytest.mark.parametrize("path", ["general", "rows"])
+@pytest.mark.parametrize("fuse,own", [(None, 1), ("1", 1), ("0", 9)])
+def test_injection_has_its_own_launch_where_the_switch_says(stub, tmp_path, path, fuse, own):
+    """FDTD_ADJ_FUSE_INJECT=0 gives every injection of a reverse sweep a launch
+    of its own on either transposed kernel; else only the first one has."""
+    env = {"FDTD_ADJ_PATH": "general"} if path == "general" else {}
+    if fuse:
+        env["FDTD_ADJ_FUSE_INJECT"] = fuse
+    launches, _ = run(stub, tmp_path, """
+import numpy as np
+s = G.Simulation(small_params(G, n=22, ncpml=5, sphere=0))
+s.set_design((14, 15, 16), np.full((4, 3, 2), 0.5, np.float32))
+mark()
+s.adjoint(9, (17, 17, 14), [4e14], checkpoint=4)
+""", env)
+    names = [k for k, _, _ in launches]
+    assert names.count("k_adj_inject") == own
+    assert any(k.startswith("k_adj_step") for k in names) == (path == "general")
