@@ -1154,7 +1154,7 @@ int fdtd_get_info(const fdtd_sim *s, fdtd_grid_info *g) {
         if (s->one_launch) {
             g->tile[1] = s->one_chunk;
             g->tile[2] = std::min(s->one_chunk, 8);
-            g->tile[4] = g->tile[3];
+            g->tile[3] = g->tile[4] = s->one_tiles;
             g->tile[5] = 0;
         }
     } else {

@@ -120,7 +120,7 @@ typedef struct fdtd_grid_info {
     int    clean[4];           /* x [clean0, clean1) by y [clean2, clean3), all z: cells run by the
                                   CPML-free variant of the row-blocked kernel; -1 when none       */
     int    schedule;           /* what the cells of this grid allow fdtd_step's stream schedule
-                                  (the field update in one launch where tile[6] is 0 does not need it):
+                                  (the field update in one launch where tile[5] is 0 does not need it):
                                   bit 0 the TFSF fix-up, bit 1 the
                                   dispersive box, bit 2 the DFT sample follow the clean box without
                                   waiting for the side pieces; bit 3 the next step's y slabs and
@@ -129,9 +129,9 @@ typedef struct fdtd_grid_info {
     int    tile[7];            /* tiles fdtd_step uses (no reference counterpart): row-blocked kernel
                                   rows per thread, clean-box x chunk, side-slab x chunk, row tiles
                                   per block on the clean box and on the side slabs, tile rows of the
-                                  corner columns (0: row-blocked as well), streams of the side pieces
-                                  beside the clean box (0: none, every piece in one launch; 1: one,
-                                  3: x slabs, y slabs, corners on their own)                       */
+                                  corner columns (0: row-blocked as well, and every piece in one
+                                  launch), streams of the side pieces beside the clean box (0: none;
+                                  1: one, 3: x slabs, y slabs, corners on their own)               */
 } fdtd_grid_info;
 
 typedef struct fdtd_sim fdtd_sim;
@@ -311,7 +311,7 @@ int  fdtd_add_layer(fdtd_sim *sim, int k0, int k1);
  * reset (HIP events on the solver stream; no reference counterpart).  Returns
  * the time and count recorded so far, then resets and sets the mode: 0 off,
  * 1 all field-update kernels of a step, 2 the clean-box launch of the
- * row-blocked kernel alone, or the launch of all pieces where tile[6] is 0 (the
+ * row-blocked kernel alone, or the launch of all pieces where tile[5] is 0 (the
  * dominant one; same as 1 when there is none),
  * 3 the K-sample DFT contractions (twiddles and contraction kernel). */
 int  fdtd_kernel_timing(fdtd_sim *sim, int enable, double *total_ms, long *launches);

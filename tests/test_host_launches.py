@@ -144,3 +144,27 @@ s.adjoint(9, (17, 17, 14), [4e14], checkpoint=4)
     names = [k for k, _, _ in launches]
     assert names.count("k_adj_inject") == own
     assert any(k.startswith("k_adj_step") for k in names) == (path == "general")
+
+
+@pytest.mark.parametrize("nz", [24, 200, 270, 331, 420, 600])
+@pytest.mark.parametrize("env,one", [({}, True), ({"FDTD_TILES": "1"}, True), ({"FDTD_CONCURRENT": "0"}, False),
+                                     ({"FDTD_ONE_LAUNCH": "0"}, False)])
+def test_info_names_the_launch_that_runs(stub, tmp_path, nz, env, one):
+    """fdtd_grid_info.tile: the row tiles of the launch, and tile[5] 0 exactly
+    where every piece is in one launch (tile[6] is 0 on one stream as well)."""
+    launches, out = run(stub, tmp_path, f"""
+p = small_params(G, sphere=0)
+p.NCELLZ = {nz}
+s = G.Simulation(p)
+print(*s.get_info().tile, s.info.NZ)
+mark()
+s.step(1)
+""", env)
+    *tile, nz = map(int, out.split())
+    assert (tile[5] == 0) == one and (tile[6] == 0) == (one or "FDTD_CONCURRENT" in env)
+    columns = next(w for w in (2, 3, 4, 5, 6, 8, 12, 16) if 64 * w - 2 >= nz + 1)
+    kernel = "k_step_all" if one else "k_step_rows"
+    blocks = [b[1] for k, _, b in launches if k.startswith(kernel)]
+    assert columns * tile[3] in blocks and columns * tile[4] in blocks, (tile, launches)
+    if one:
+        assert len(blocks) == 1
