@@ -436,6 +436,14 @@ void add_pieces(const fdtd_sim *s, A &a, int chunk) {
     add(0, chunk, &s->cbox, 1);
 }
 
+// Floats of the largest psi array.
+size_t psi_largest(const fdtd_sim *s) {
+    return std::max(*std::max_element(s->hsz, s->hsz + 6), *std::max_element(s->esz, s->esz + 6));
+}
+// Whether n floats can be reached by 32-bit byte offsets, the last word left for the lanes whose access is dropped.
+bool in_window(size_t n) { return (double)n * 4.0 < 4294967292.0; }
+bool psi_in_one_window(const fdtd_sim *s) { return in_window(s->npsi); }
+
 // The row-blocked kernel (k_step_rows) runs the whole grid with TFSF left
 // out; k_tfsf_fix then adds it, which needs the TFSF cells and their
 // neighbours free of CPML and with 1/(kappa d) at its interior value.  The
@@ -453,8 +461,8 @@ int plan_rows(fdtd_sim *s) {
     if (const char *v = std::getenv("FDTD_CCHUNK")) s->cchunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_SCHUNK")) s->schunk = std::max(1, std::atoi(v));
     if (const char *v = std::getenv("FDTD_XCD")) s->xcd = std::atoi(v) != 0;
-    // 32-bit byte offsets, the last word left for the lanes whose access is dropped
-    if ((double)s->fsz * 4.0 >= 4294967292.0 || (double)s->npsi * 4.0 >= 4294967292.0) return FDTD_OK;
+    // 32-bit byte offsets into each array
+    if (!in_window(s->fsz) || !in_window(psi_largest(s))) return FDTD_OK;
     std::vector<uint32_t> img(kRowsAuxWords, 0u);
     auto put = [&](int q, float v) { std::memcpy(&img[q], &v, 4); };
     for (int a = 0; a < 3; a++) {
@@ -580,7 +588,7 @@ int plan_rows(fdtd_sim *s) {
     // 18.4 and 20.6 at 14 M cells, 26.3 and 28.9 at 21 M, 33.3 and 36.3 at 29 M, 50.6 and 52.2 at 47 M.
     s->one_launch = (long)s->g.NX * s->g.NY * s->g.NZ <= kOneLaunchCells;
     if (const char *v = std::getenv("FDTD_ONE_LAUNCH")) s->one_launch = std::atoi(v) != 0;
-    s->one_launch = s->one_launch && s->rows == 2;
+    s->one_launch = s->one_launch && s->rows == 2 && psi_in_one_window(s);
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_EARLY", "FDTD_SIDE_STREAMS", "FDTD_CHAIN_JOIN", "FDTD_POST_AFTER_JOIN",
                           "FDTD_EARLY_SIDE", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_STILES", "FDTD_CTJ"})
         if (std::getenv(k)) s->one_launch = false;
@@ -599,11 +607,11 @@ RowsArgs make_rows(fdtd_sim *s) {
     }
     r.fbytes = (unsigned)(s->fsz * 4);
     r.psi = (const char *)s->psi;
-    r.psi_bytes = (unsigned)(s->npsi * 4);
+    r.psi_bytes = (unsigned)(psi_largest(s) * 4);
     for (int a = 0; a < 6; a++) {
-        r.hin[a] = (unsigned)((s->psiH[s->pp][a] - s->psi) * 4);
-        r.hout[a] = (unsigned)((s->psiH[1 - s->pp][a] - s->psi) * 4);
-        r.eio[a] = (unsigned)((s->psiE[a] - s->psi) * 4);
+        r.hin[a] = (unsigned)((s->psiH[s->pp][a] - s->psi) * 4 / kPsiUnit);
+        r.hout[a] = (unsigned)((s->psiH[1 - s->pp][a] - s->psi) * 4 / kPsiUnit);
+        r.eio[a] = (unsigned)((s->psiE[a] - s->psi) * 4 / kPsiUnit);
     }
     r.aux = s->aux_d;
     r.Chh = (float)S.Chh; r.Che = (float)S.Che; r.Cee = (float)S.Cee; r.Ceh = (float)S.Ceh;
@@ -852,6 +860,8 @@ int launch_rows_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Di
 StepAll make_step_all(fdtd_sim *s, const LineDev &l, int tiles, int chunk) {
     StepAll a{};
     a.r = make_rows(s);
+    a.r.psi_bytes = (unsigned)(s->npsi * 4);
+    for (int x = 0; x < 6; x++) { a.r.hin[x] *= kPsiUnit; a.r.hout[x] *= kPsiUnit; a.r.eio[x] *= kPsiUnit; }
     a.line = l;
     a.r.tiles = tiles;
     add_pieces(s, a, chunk);
@@ -1025,8 +1035,8 @@ int fdtd_create(const fdtd_params *p, fdtd_sim **out) {
     const size_t hsz[6] = {hz_, hy_, hz_, hx_, hx_, hy_};
     const size_t esz[6] = {ez_, ey_, ez_, ex_, ey_, ex_};
     for (int a = 0; a < 6; a++) { s->hsz[a] = hsz[a]; s->esz[a] = esz[a]; }
-    // one allocation, so the row-blocked kernel reaches every array from one base
-    auto pad64 = [](size_t n) { return (n + 63) / 64 * 64; };
+    // one allocation, so the one-launch step reaches every array from one base
+    auto pad64 = [](size_t n) { return (n + 63) / 64 * 64; };   // kPsiUnit
     size_t npsi = 0;
     for (int a = 0; a < 6; a++) npsi += 2 * pad64(hsz[a]) + pad64(esz[a]);
     if ((rc = dalloc(s, &s->psi, npsi))) return fail(rc);

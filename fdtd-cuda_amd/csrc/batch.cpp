@@ -669,7 +669,7 @@ int fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out)
     const char *one = std::getenv("FDTD_ONE_LAUNCH");
     b->one = !(flags & FDTD_BATCH_GENERAL) && (!one || std::atoi(one) != 0);
     for (fdtd_sim *s : b->sims)
-        b->one = b->one && s->use_rows && s->rows == 2 && (one || (long)s->g.NX * s->g.NY * s->g.NZ <= kOneLaunchCells);
+        b->one = b->one && s->use_rows && s->rows == 2 && psi_in_one_window(s) && (one || (long)s->g.NX * s->g.NY * s->g.NZ <= kOneLaunchCells);
     for (const char *k : {"FDTD_CONCURRENT", "FDTD_SIDE_STREAMS", "FDTD_BATCH_EARLY", "FDTD_CCHUNK", "FDTD_SCHUNK", "FDTD_CTJ"})
         if (std::getenv(k)) b->one = false;
     const char *conc = std::getenv("FDTD_CONCURRENT");

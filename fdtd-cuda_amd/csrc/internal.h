@@ -216,12 +216,15 @@ struct Pieces {
 // 1/(kappa d) = ik0[e][axis] (e: 0 E, 1 H), pass every domain test, and
 // have an H-clean plane or row just below the box.  nseg and start are
 // filled in by the launcher.
+constexpr int kPsiUnit = 256;           // bytes
 struct RowsArgs {
     const char *Ein[3], *Hin[3];
     char *Eout[3], *Hout[3];
     unsigned fbytes;                    // bytes of a field allocation
-    // forward psi: one allocation, byte offsets of the six psi_H arrays read
-    // and written by this step and of the psi_E arrays (updated in place)
+    // forward psi: one allocation, the six psi_H arrays read and written by
+    // this step and the psi_E arrays (updated in place) at multiples of
+    // kPsiUnit.  One-launch kernels: byte offsets, psi_bytes of all arrays
+    // together; the launches per variant: in units, psi_bytes of the largest
     const char *psi;
     unsigned psi_bytes, hin[6], hout[6], eio[6];
     const unsigned *aux;

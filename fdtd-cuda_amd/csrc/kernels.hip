@@ -787,7 +787,7 @@ struct RowsLds {
 };
 
 // Block L of the box x in [ia, ib), y in [ja, jbox): row-tile groups fastest, then z segments, then x chunks.
-template <int R, bool XG, bool YG, bool ADJ, bool ZS>
+template <int R, bool XG, bool YG, bool ADJ, bool ZS, bool WIN>
 __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, int ja, int jbox, int ichunk, int L,
                                            RowsLds<R, ADJ> &lds) {
     constexpr bool AS = ADJ && (XG || YG);   // adjoint on a side slab or corner column
@@ -857,7 +857,14 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
 #pragma unroll
     for (int r = 1; r <= R; r++) so[r] = kown && jb + r < jbox ? ro[r] : kOob;
     // psi accesses of the forward step: lane part of the offset (the plane, row and layer are scalar)
+    // through one window over all arrays, or one per array where those together pass 4 GB
     const rsrc_t rp = make_rsrc(ra.psi, ra.psi_bytes);
+    auto own = [&](unsigned at) INLINE_LAMBDA { return make_rsrc(ra.psi + (unsigned long)at * kPsiUnit, ra.psi_bytes); };
+    auto pld = [&](unsigned at, unsigned v, unsigned o) INLINE_LAMBDA { return WIN ? bld(rp, v, at + o) : bld(own(at), v, o); };
+    auto pst = [&](unsigned at, unsigned v, unsigned o, float x) INLINE_LAMBDA {
+        if constexpr (WIN) bst<false>(rp, v, at + o, x);
+        else bst<false>(own(at), v, o, x);
+    };
     const unsigned vzh = lzh >= 0 ? (unsigned)lzh * 4u : kOob, vze = lze >= 0 ? (unsigned)lze * 4u : kOob;
     const unsigned vzhs = kown ? vzh : kOob, vzes = kown ? vze : kOob;
     const unsigned vk = (unsigned)kq * 4u, vkA = kown && kA ? vk : kOob, vkC = kown && kC ? vk : kOob;
@@ -970,28 +977,28 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
 #pragma unroll
             for (int r = 0; r <= R; r++) {
                 const unsigned o = ((unsigned)(ip * NY + jq(r)) * (unsigned)Lzh) * 4u;
-                P.hxz[r] = bld(rp, vzh, ra.hin[0] + o);
-                P.hyz[r] = bld(rp, vzh, ra.hin[2] + o);
+                P.hxz[r] = pld(ra.hin[0], vzh, o);
+                P.hyz[r] = pld(ra.hin[2], vzh, o);
             }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
                 const unsigned o = ((unsigned)(ip * NY + jq(r)) * (unsigned)Lze) * 4u;
-                P.exz[r - 1] = bld(rp, vze, ra.eio[0] + o);
-                P.eyz[r - 1] = bld(rp, vze, ra.eio[2] + o);
+                P.exz[r - 1] = pld(ra.eio[0], vze, o);
+                P.eyz[r - 1] = pld(ra.eio[2], vze, o);
             }
         }
         if (YG) {
 #pragma unroll
             for (int r = 0; r <= R; r++) {
                 const unsigned o = ((unsigned)(ip * Lyh + max(lyh(r), 0)) * (unsigned)NZ) * 4u;
-                P.hxy[r] = bld(rp, vk, ra.hin[1] + o);
-                P.hzy[r] = bld(rp, vk, ra.hin[5] + o);
+                P.hxy[r] = pld(ra.hin[1], vk, o);
+                P.hzy[r] = pld(ra.hin[5], vk, o);
             }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
                 const unsigned o = ((unsigned)(ip * Lye + max(lye(r), 0)) * (unsigned)NZ) * 4u;
-                P.exy[r - 1] = bld(rp, vk, ra.eio[1] + o);
-                P.ezy[r - 1] = bld(rp, vk, ra.eio[4] + o);
+                P.exy[r - 1] = pld(ra.eio[1], vk, o);
+                P.ezy[r - 1] = pld(ra.eio[4], vk, o);
             }
         }
         if (XG) {
@@ -999,14 +1006,14 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
 #pragma unroll
             for (int r = 0; r <= R; r++) {
                 const unsigned o = ((unsigned)(lh * NY + jq(r)) * (unsigned)NZ) * 4u;
-                P.hyx[r] = bld(rp, vk, ra.hin[3] + o);
-                P.hzx[r] = bld(rp, vk, ra.hin[4] + o);
+                P.hyx[r] = pld(ra.hin[3], vk, o);
+                P.hzx[r] = pld(ra.hin[4], vk, o);
             }
 #pragma unroll
             for (int r = 1; r <= R; r++) {
                 const unsigned o = ((unsigned)(le * NY + jq(r)) * (unsigned)NZ) * 4u;
-                P.eyx[r - 1] = bld(rp, vk, ra.eio[3] + o);
-                P.ezx[r - 1] = bld(rp, vk, ra.eio[5] + o);
+                P.eyx[r - 1] = pld(ra.eio[3], vk, o);
+                P.ezx[r - 1] = pld(ra.eio[5], vk, o);
             }
         }
     };
@@ -1211,8 +1218,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 }
                 if (wr && r > 0) {
                     const unsigned v = u && srow ? vzhs : kOob;
-                    bst<false>(rp, v, ra.hout[0] + o, a);
-                    bst<false>(rp, v, ra.hout[2] + o, b);
+                    pst(ra.hout[0], v, o, a);
+                    pst(ra.hout[2], v, o, b);
                 }
             }
             const int ly = lyh(r);
@@ -1227,8 +1234,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 if (u && kA) vx -= Che * a;
                 if (wr && r > 0) {
                     const unsigned v = u && srow ? vkA : kOob;
-                    bst<false>(rp, v, ra.hout[1] + o, a);
-                    bst<false>(rp, v, ra.hout[5] + o, pyz);
+                    pst(ra.hout[1], v, o, a);
+                    pst(ra.hout[5], v, o, pyz);
                 }
             }
             if constexpr (!ADJ && XG) {
@@ -1244,8 +1251,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 }
                 if (wr && r > 0) {
                     const unsigned v = u && srow ? vkA : kOob;
-                    bst<false>(rp, v, ra.hout[3] + o, a);
-                    bst<false>(rp, v, ra.hout[4] + o, b);
+                    pst(ra.hout[3], v, o, a);
+                    pst(ra.hout[4], v, o, b);
                 }
             }
             if (!ADJ && YG && iA && ly >= 0 && kA) vz += Che * pyz;
@@ -1415,8 +1422,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 const bool ua = iA && jC(r), ub = iC && jA(r);
                 if (ua && lze >= 0) vx -= Ceh * a;
                 if (ub && lze >= 0) vy += Ceh * b;
-                bst<false>(rp, ua && srow ? vzes : kOob, ra.eio[0] + o, a);
-                bst<false>(rp, ub && srow ? vzes : kOob, ra.eio[2] + o, b);
+                pst(ra.eio[0], ua && srow ? vzes : kOob, o, a);
+                pst(ra.eio[2], ub && srow ? vzes : kOob, o, b);
             }
             const int ly = lye(r);
             if constexpr (!ADJ && YG) {
@@ -1427,8 +1434,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 const bool ua = iA && ly >= 0, ub = iC && ly >= 0;
                 if (ua && kC) vx += Ceh * a;
                 if (ub && kA) vz -= Ceh * b;
-                bst<false>(rp, ua && srow ? vkC : kOob, ra.eio[1] + o, a);
-                bst<false>(rp, ub && srow ? vkA : kOob, ra.eio[4] + o, b);
+                pst(ra.eio[1], ua && srow ? vkC : kOob, o, a);
+                pst(ra.eio[4], ub && srow ? vkA : kOob, o, b);
             }
             if constexpr (!ADJ && XG) {
                 const int lc = max(lx, 0);
@@ -1438,8 +1445,8 @@ __device__ __forceinline__ void rows_block(const RowsArgs &ra, int ia, int ib, i
                 const bool ua = lx >= 0 && jA(r), ub = lx >= 0 && jC(r);
                 if (ua && kC) vy -= Ceh * a;
                 if (ub && kA) vz += Ceh * b;
-                bst<false>(rp, ua && srow ? vkC : kOob, ra.eio[3] + o, a);
-                bst<false>(rp, ub && srow ? vkA : kOob, ra.eio[5] + o, b);
+                pst(ra.eio[3], ua && srow ? vkC : kOob, o, a);
+                pst(ra.eio[5], ub && srow ? vkA : kOob, o, b);
             }
             bst<true>(sEx, so[r], pl, ux ? vx : C.x[r]);
             bst<true>(sEy, so[r], pl, uy ? vy : C.y[r]);
@@ -1478,11 +1485,14 @@ __device__ __forceinline__ bool rows_zwave(const RowsArgs &ra, int ja, int jbox,
 // Waves without z-slab lanes run a march without the z-CPML loads and stores
 // (20 of some 60 memory instructions per plane); both marches hold the same
 // barriers.
-template <int R, bool XG, bool YG, bool ADJ>
+// WIN: the forward psi arrays through one window of 4 GB, not one per array.  The one-launch kernels, which
+// hold four variants of the march, spill 411 scalar registers so and 789 with a window per array; the
+// launches per variant (two rows per thread) at most 184 and 260, and only grids of theirs hold 4 GB of psi.
+template <int R, bool XG, bool YG, bool ADJ, bool WIN>
 __device__ __forceinline__ void rows_piece(const RowsArgs &ra, int ia, int ib, int ja, int jbox, int ichunk, int L,
                                            RowsLds<R, ADJ> &lds) {
-    if (ADJ || rows_zwave<R>(ra, ja, jbox, L)) rows_block<R, XG, YG, ADJ, true>(ra, ia, ib, ja, jbox, ichunk, L, lds);
-    else rows_block<R, XG, YG, ADJ, false>(ra, ia, ib, ja, jbox, ichunk, L, lds);
+    if (ADJ || rows_zwave<R>(ra, ja, jbox, L)) rows_block<R, XG, YG, ADJ, true, WIN>(ra, ia, ib, ja, jbox, ichunk, L, lds);
+    else rows_block<R, XG, YG, ADJ, false, WIN>(ra, ia, ib, ja, jbox, ichunk, L, lds);
 }
 
 // A block of a launch over the pieces of one variant (ra.box, ra.start).
@@ -1491,7 +1501,7 @@ __device__ __forceinline__ void rows_body(const RowsArgs &ra, int L) {
     __shared__ RowsLds<R, ADJ> lds;
     int pc = 0;
     while (pc + 1 < ra.npiece && L >= ra.start[pc + 1]) pc++;
-    rows_piece<R, XG, YG, ADJ>(ra, ra.box[pc][0], ra.box[pc][1], ra.box[pc][2], ra.box[pc][3], ra.ichunk,
+    rows_piece<R, XG, YG, ADJ, false>(ra, ra.box[pc][0], ra.box[pc][1], ra.box[pc][2], ra.box[pc][3], ra.ichunk,
                                      L - ra.start[pc], lds);
 }
 
@@ -2304,10 +2314,10 @@ __device__ __forceinline__ void step_all_body(const StepAll &a, int t, int block
     const int ia = a.box[q][0], ib = a.box[q][1], ja = a.box[q][2], jb = a.box[q][3], ich = a.ich[q];
     const int L = a.r.xcd ? xcd_order(b - a.start[q], a.start[q + 1] - a.start[q]) : b - a.start[q];
     switch (a.kind[q]) {
-        case 0: rows_piece<2, false, false, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        case 1: rows_piece<2, true, false, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        case 2: rows_piece<2, false, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        default: rows_piece<2, true, true, false>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 0: rows_piece<2, false, false, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 1: rows_piece<2, true, false, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 2: rows_piece<2, false, true, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        default: rows_piece<2, true, true, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
     }
 }
 template <int MW>
@@ -3138,10 +3148,10 @@ __global__ __launch_bounds__(64 * 12) void k_adj_all(AdjAll) {
     while (q + 1 < a.n && b >= a.start[q + 1]) q++;
     const int ia = a.box[q][0], ib = a.box[q][1], ja = a.box[q][2], jb = a.box[q][3], ich = a.ich[q], L = b - a.start[q];
     switch (a.kind[q]) {
-        case 0: rows_piece<2, false, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        case 1: rows_piece<2, true, false, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        case 2: rows_piece<2, false, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
-        default: rows_piece<2, true, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 0: rows_piece<2, false, false, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 1: rows_piece<2, true, false, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        case 2: rows_piece<2, false, true, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
+        default: rows_piece<2, true, true, true, true>(a.r, ia, ib, ja, jb, ich, L, lds); break;
     }
 }
 

@@ -218,6 +218,8 @@ constexpr long kOneLaunchCells = 50000000;
 // and `slots` resident blocks, and the arguments at the handle's parity.
 int march_chunk(long columns, int NX, long slots, int most);
 StepAll make_step_all(fdtd_sim *s, const LineDev &l, int tiles, int chunk);
+// Whether the one-launch step's 32-bit offsets reach every psi array.
+bool psi_in_one_window(const fdtd_sim *s);
 // Kernel arguments at the handle's current parity.
 StepDev make_step(fdtd_sim *s, bool fused);
 LineDev make_line(fdtd_sim *s);

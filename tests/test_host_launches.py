@@ -168,3 +168,21 @@ s.step(1)
     assert columns * tile[3] in blocks and columns * tile[4] in blocks, (tile, launches)
     if one:
         assert len(blocks) == 1
+
+
+@pytest.mark.parametrize("env", [{}, {"FDTD_ONE_LAUNCH": "1"}])
+def test_more_than_4_gb_of_psi_keep_the_row_blocked_kernel(stub, tmp_path, env):
+    """31 CPML layers of a flat grid: each array within 4 GB, all together not."""
+    launches, out = run(stub, tmp_path, """
+p = small_params(G, sphere=0, nfreq=1, ncpml=31)
+p.NCELLX = p.NCELLY = 1577
+s = G.Simulation(p)
+print(s.info.NX, s.info.NZ, s.info.fused_path, s.get_info().tile[5])
+mark()
+s.step(1)
+""", env)
+    n, nz, path, corners = map(int, out.split())
+    assert 4 * (n + 2) * (n + 2) * (nz + 11) < 1 << 32
+    assert 4 * (4 * 62 + 2 * 64) * (n * n + 2 * n * nz) > 1 << 32
+    assert path == 1 and corners > 0
+    assert any(k.startswith("k_step_rows") for k, _, _ in launches)
