@@ -892,7 +892,9 @@ int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Dis
 // thread, which also takes the page faults of a fresh buffer (8.5 ms for a field
 // of 281^3, 10 GB/s; the link does 56).  Here the two halves of a pinned buffer
 // of the handle take turns: the device fills one while up to eight threads move
-// the other's bytes on.  Below 1 MB the threads cost more than they save.
+// the other's bytes on.  Below 1 MB the threads cost more than they save.  The
+// threads poll for the first half, so the caller lets earlier work end first and
+// leaves on the stream only what fills dev.
 int copy_out(fdtd_sim *s, const void *dev, void *host, size_t bytes) {
     constexpr size_t kMin = 1u << 20, kHalf = 8u << 20;
     if (bytes < kMin) {
@@ -2094,6 +2096,7 @@ int fdtd_sync(fdtd_sim *s) {
 int fdtd_get_field(fdtd_sim *s, int comp, float *out) {
     if (!s || !out || comp < 0 || comp > 5) return FDTD_ERR_INVALID;
     const float *f = comp < 3 ? s->E[s->p][comp] : s->H[s->p][comp - 3];
+    HIPCHK(s, hipStreamSynchronize(s->stream));
     HIPCHK(s, launch_pack_field(f, s->g, s->dense, 1, s->stream));
     return copy_out(s, s->dense, out, (size_t)s->g.NX * s->g.NY * s->g.NZ * sizeof(float));
 }

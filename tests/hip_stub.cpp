@@ -4,15 +4,19 @@
 // memory is host memory, kernels do not run, and every launch appends
 //   kernel name (demangled, no arguments) <tab> grid x y z <tab> block x y z
 // to the file HIP_STUB_LOG.  After stub_fail_launch(n) the n-th launch from
-// then on returns an error once.
+// then on returns an error once; after stub_queue(ms) the next synchronisation
+// of a stream takes so long.
 #include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 
+#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <string>
+#include <thread>
+#include <utility>
 
 #include "../fdtd-cuda_amd/csrc/sim.h"
 
@@ -27,6 +31,7 @@ size_t g_shmem;
 hipStream_t g_stream;
 hipError_t g_last = hipSuccess;
 long g_fail = -1;
+int g_queued_ms = 0;
 char g_handle[8];
 template <typename T>
 hipError_t handle(T *out) {
@@ -43,6 +48,7 @@ hipError_t alloc(T *out, size_t n) {
 extern "C" {
 
 void stub_fail_launch(long n) { g_fail = n; }
+void stub_queue(int ms) { g_queued_ms = ms; }
 // Records of a point monitor or objective probe that the handle still holds for a later launch.
 int stub_pending_records(const fdtd_sim *s) { return (s->rec_dst[0] != nullptr) + (s->rec_dst[1] != nullptr); }
 
@@ -99,7 +105,10 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipSt
 hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }   // no kernel runs: memory is as allocated
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle(s); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+    std::this_thread::sleep_for(std::chrono::milliseconds(std::exchange(g_queued_ms, 0)));
+    return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) { return handle(g); }

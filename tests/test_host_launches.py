@@ -186,3 +186,24 @@ s.step(1)
     assert 4 * (4 * 62 + 2 * 64) * (n * n + 2 * n * nz) > 1 << 32
     assert path == 1 and corners > 0
     assert any(k.startswith("k_step_rows") for k, _, _ in launches)
+
+
+@pytest.mark.parametrize("read", ["s.get_field(2)", "s.checkpoint()"])
+def test_a_read_out_behind_queued_steps_does_not_keep_the_cores_busy(stub, tmp_path, read):
+    """The threads that move a field to the caller poll for its bytes, so they
+    start once the work queued before has ended (0.4 s of it here)."""
+    _, out = run(stub, tmp_path, f"""
+import time
+s = G.Simulation(small_params(G, n=120, nfreq=1, sphere=0))
+{read}
+s.step(1)
+idle = time.process_time()
+{read}
+idle = time.process_time() - idle
+stub.stub_queue(400)
+queued = time.process_time()
+{read}
+print(idle, time.process_time() - queued)
+""")
+    idle, queued = map(float, out.split())
+    assert queued - idle < 0.2, (idle, queued)
