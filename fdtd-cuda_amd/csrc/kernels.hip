@@ -2199,7 +2199,6 @@ __global__ void k_disp_sync(DispDev d, int from_field) {
 // The incident wave at the source plane over the first `steps` steps, for the
 // spectra that are divided by it: the line run again from rest in the LDS of
 // one block (e in [0, L), h in [L, 2L)), two barriers a step, then its DFT at
-// one block (e in [0, L), h in [L, 2L)), two barriers a step, then its DFT at
 // the monitors' samples.  Bound by the barriers (0.6 us a step); the host
 // took 3 us a step for the same recurrences (L = 1200).  The pulse of every
 // step is formed beforehand by a launch over the steps.
@@ -2231,7 +2230,9 @@ __global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int 
         }
         if (tid < 2) {
             const double en = ei - l.ce * (h[in] - h[in - 1]);
-            e[end] = mur + l.mur_coef * (en - eo);
+            double v = mur + l.mur_coef * (en - eo);
+            if (end == l.src) v += p;
+            e[end] = v;
             mur = en;
         }
         __syncthreads();
