@@ -4,8 +4,8 @@
 // batched step is that loop body for every simulation at once.
 //
 // Per step every kernel runs ONCE for all simulations that use it.  Where all
-// of them have the row path, the lines and the whole field update are one
-// launch (k_step_batch).  Else: the 1D
+// of them have the row path and at most 50 M cells, the lines and the whole
+// field update are one launch per block height (k_step_batch).  Else: the 1D
 // lines (one block each); the field update of fdtd_step's fast path (the
 // row-blocked kernel on clean boxes and side slabs, one launch per variant,
 // block height and rows per thread; the general kernel on corner columns, or

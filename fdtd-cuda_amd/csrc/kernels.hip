@@ -2167,7 +2167,7 @@ __global__ __launch_bounds__(256) void k_hydro_v_ce0(DispDev d, int nd, StepDev 
 
 // Continuity + E update of component c = 1 (y) or 2 (z).  Every load stands before
 // the first store, so a cell is one memory latency after its mask, not two (a
-// launch on a 119^3 grid is that latency; the hydrodynamic step there 62.5 -> 60.3
+// launch on a 121^3 grid is that latency; the hydrodynamic step there 62.5 -> 60.3
 // us with the component fixed at compile time and 32-bit cell divisions).
 template <int c>
 __global__ void k_hydro_ce(DispDev d) {
