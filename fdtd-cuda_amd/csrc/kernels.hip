@@ -1687,15 +1687,52 @@ __global__ void k_per_tfsf(StepDev s) {
     s.Eout[1][pe] += tfsf_term_ct<true, 1, 2>(s.tf, LineGlobal{s.tf}, i, j, k0);
 }
 
+// The 64-lane rows of the TFSF planes: per normal axis a, `planes` planes of
+// [t0 - 1, t1 + past] along the other two, b0 row by row and b1 (fastest in
+// memory) in pieces of 64.  Every axis has its own extents: counted by the longest
+// one, rows are idle for the most part on flat and long boxes, and a block of the
+// fix-up loads the line before it knows (us per step: 3000 x 100 x 100 cells 969
+// and 644, 2500 x 45 x 45 393 and 171, 300 x 300 x 1000 1128 and 1087; cubes the same).
+__host__ __device__ inline int tfsf_axis_rows(const TfsfDev &t, int a, int planes, int past, int *nbx) {
+    const int b0 = a == 0 ? 1 : 0, b1 = a == 2 ? 1 : 2;
+    *nbx = (t.t1[b1] - t.t0[b1] + 2 + past + 63) / 64;
+    return planes * (t.t1[b0] - t.t0[b0] + 2 + past) * *nbx;
+}
+inline long tfsf_nblocks(const TfsfDev &t, int planes, int past) {   // four rows a block
+    long n = 0;
+    for (int a = 0, nbx; a < 3; a++) n += tfsf_axis_rows(t, a, planes, past, &nbx);
+    return (n + 3) / 4;
+}
+struct TfsfRow { int a, q, by, bx; };   // axis, plane, row along b0, piece along b1
+__device__ __forceinline__ bool tfsf_row(const TfsfDev &t, int L, int planes, int past, TfsfRow &r) {
+    L = __builtin_amdgcn_readfirstlane(L);   // uniform across a wave
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        int nbx;
+        const int n = tfsf_axis_rows(t, a, planes, past, &nbx);
+        if (L < n) {
+            const int u = n / (planes * nbx);
+            r.a = a;
+            r.bx = L % nbx;
+            r.by = L / nbx % u;
+            r.q = L / (nbx * u);
+            return true;
+        }
+        L -= n;
+    }
+    return false;
+}
+
 // CORRECT_X/Y/Z in place: per normal axis the planes t0-1, t0 and t1 over
 // [t0-1, t1] of the other two, a cell on planes of several axes taken by the
 // lowest one.  Only the planes' cells are visited (the box they bound has
 // some 20 times as many; a 97^3 grid 13.4 -> 5.5 us).
-__global__ __launch_bounds__(256) void k_tfsf_split(StepDev s, int nbx, int span) {
+__global__ __launch_bounds__(256) void k_tfsf_split(StepDev s) {
     const TfsfDev &t = s.tf;
-    const int L = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (L >= nbx * span * 9) return;
-    const int u0 = (L / nbx) % span, v0 = L % nbx * 64 + lane, pq = L / (nbx * span), a = pq / 3, q = pq % 3;
+    const int lane = threadIdx.x & 63;
+    TfsfRow r;
+    if (!tfsf_row(t, (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), 3, 0, r)) return;
+    const int u0 = r.by, v0 = r.bx * 64 + lane, a = r.a, q = r.q;
     const int b0 = a == 0 ? 1 : 0, b1 = a == 2 ? 1 : 2;   // other axes, b1 fastest in memory
     const int u = pick3(b0, t.t0[0], t.t0[1], t.t0[2]) - 1 + u0, v = pick3(b1, t.t0[0], t.t0[1], t.t0[2]) - 1 + v0;
     if (u > pick3(b0, t.t1[0], t.t1[1], t.t1[2]) || v > pick3(b1, t.t1[0], t.t1[1], t.t1[2])) return;
@@ -1727,9 +1764,8 @@ __global__ __launch_bounds__(256) void k_tfsf_split(StepDev s, int nbx, int span
 // along the other axes; a cell lying on planes of several axes is taken by
 // the lowest one.  Requires the region free of CPML and inside every domain.
 template <class S>
-__device__ __forceinline__ void tfsf_fix_body(const StepDev &s, const S &src, int bx, int by, int bz, int lane) {
+__device__ __forceinline__ void tfsf_fix_body(const StepDev &s, const S &src, int bx, int by, int a, int q, int lane) {
     const TfsfDev &t = s.tf;
-    const int a = bz >> 2, q = bz & 3;
     const int b0 = a == 0 ? 1 : 0, b1 = a == 2 ? 1 : 2;   // other axes, b1 fastest in memory
     const int u = pick3(b0, t.t0[0], t.t0[1], t.t0[2]) - 1 + by;
     const int v = pick3(b1, t.t0[0], t.t0[1], t.t0[2]) - 1 + bx * 64 + lane;
@@ -1764,15 +1800,14 @@ __device__ __forceinline__ void tfsf_fix_body(const StepDev &s, const S &src, in
 }
 
 
-// Four 64-lane rows of the fix-up's planes, rows L to L + 3 of nbx * span * 12
-// (the launches' geometry: tfsf_fix_rows).  The line's values that the box
+// Four 64-lane rows of the fix-up's planes (four planes per axis).  The line's values that the box
 // reaches are brought to LDS once per block where they fit: a row evaluates
 // up to eight of its terms one after the other, each two loads away from the
 // line otherwise (with the hydrodynamic box of a 121^3 grid in one launch 11.4
 // -> 9.7 us).  On large grids the z planes bound it: every value there is a
 // cache line of its own (281^3: 23 us alone either way).
 constexpr int kFixLine = 1024;
-__device__ __forceinline__ void tfsf_fix_block(const StepDev &s, int b, int nbx, int span) {
+__device__ __forceinline__ void tfsf_fix_block(const StepDev &s, int b) {
     __shared__ float line[2 * kFixLine];
     const TfsfDev &t = s.tf;
     float lo = 0.f, hi = 0.f;
@@ -1794,22 +1829,14 @@ __device__ __forceinline__ void tfsf_fix_block(const StepDev &s, int b, int nbx,
         }
         __syncthreads();
     }
-    const int L = b * 4 + (int)(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (L >= nbx * span * 12) return;
-    const int bx = L % nbx, by = (L / nbx) % span, bz = L / (nbx * span);
-    if (fits) tfsf_fix_body(s, LineLds{line, l0, n}, bx, by, bz, lane);
-    else tfsf_fix_body(s, LineGlobal{t}, bx, by, bz, lane);
+    const int lane = threadIdx.x & 63;
+    TfsfRow r;
+    if (!tfsf_row(t, b * 4 + (int)(threadIdx.x >> 6), 4, 1, r)) return;
+    if (fits) tfsf_fix_body(s, LineLds{line, l0, n}, r.bx, r.by, r.a, r.q, lane);
+    else tfsf_fix_body(s, LineGlobal{t}, r.bx, r.by, r.a, r.q, lane);
 }
-__host__ __device__ inline void tfsf_fix_shape(const TfsfDev &t, int *nbx, int *span) {
-    *span = 0;
-    for (int a = 0; a < 3; a++) {
-        const int n = t.t1[a] - t.t0[a] + 3;
-        if (n > *span) *span = n;
-    }
-    *nbx = (*span + 63) / 64;
-}
-inline long tfsf_fix_nblocks(int nbx, int span) { return ((long)nbx * span * 12 + 3) / 4; }
-__global__ __launch_bounds__(256) void k_tfsf_fix(StepDev s, int nbx, int span) { tfsf_fix_block(s, (int)blockIdx.x, nbx, span); }
+inline long tfsf_fix_nblocks(const TfsfDev &t) { return tfsf_nblocks(t, 4, 1); }
+__global__ __launch_bounds__(256) void k_tfsf_fix(StepDev s) { tfsf_fix_block(s, (int)blockIdx.x); }
 
 // One thread per sample column of the E half (H taken at the same cell).
 __device__ __forceinline__ void sample_body(const Geom &g, const FaceDev &f, const float *const *E, const float *const *H,
@@ -1974,7 +2001,7 @@ __global__ void k_nonlocal_gd(DispDev d) {
 // blocks [0, nd) run the dispersive box, 256 cells each, the next nt the
 // fix-up, one 64-lane row of its planes per wave, the last ns the sample of
 // the new fields (s.Eout, s.Hout) into s.sample_row, 256 columns each.
-__global__ __launch_bounds__(256) void k_post(StepDev s, DispDev d, int nd, int nbx, int span, int nt, int ns) {
+__global__ __launch_bounds__(256) void k_post(StepDev s, DispDev d, int nd, int nt, int ns) {
     int b = (int)blockIdx.x;
     if (b < nd) {
         disp_body(d, (long)b * 256 + threadIdx.x);
@@ -1982,7 +2009,7 @@ __global__ __launch_bounds__(256) void k_post(StepDev s, DispDev d, int nd, int 
     }
     b -= nd;
     if (b < nt) {
-        tfsf_fix_block(s, b, nbx, span);
+        tfsf_fix_block(s, b);
         return;
     }
     b -= nt;
@@ -2145,11 +2172,11 @@ __device__ __forceinline__ void hydro_ce_cell(const DispDev &d, long idx, int bi
 // which no launch of the step writes.  Blocks past the box's nd run the TFSF
 // fix-up (nt) and the sample (ns), as in k_post, where their cells are apart
 // from the box (a step of 121^3: 71 -> 64 us, a launch of 8 us less).
-__global__ __launch_bounds__(256) void k_hydro_v_ce0(DispDev d, int nd, StepDev s, int nbx, int span, int nt, int ns) {
+__global__ __launch_bounds__(256) void k_hydro_v_ce0(DispDev d, int nd, StepDev s, int nt, int ns) {
     int b = (int)blockIdx.x - nd;
     if (b >= 0) {
         if (b < nt) {
-            tfsf_fix_block(s, b, nbx, span);
+            tfsf_fix_block(s, b);
             return;
         }
         b -= nt;
@@ -3215,9 +3242,7 @@ __global__ __launch_bounds__(64 * MW) __attribute__((amdgpu_waves_per_eu(R == 2 
 __global__ __launch_bounds__(256) void k_tfsf_fix_batch(const FusedItem *items, const unsigned *map) {
     const unsigned m = batch_map(map);
     const FusedItem &it = batch_item(items, m >> kBatchLocalBits);
-    int nbx, span;
-    tfsf_fix_shape(it.s.tf, &nbx, &span);
-    tfsf_fix_block(it.s, (int)(m & ((1u << kBatchLocalBits) - 1)), nbx, span);
+    tfsf_fix_block(it.s, (int)(m & ((1u << kBatchLocalBits) - 1)));
 }
 
 __global__ __launch_bounds__(1024) void k_line_batch(const LineDev *items, const int *dyn, int step_off) {
@@ -3311,9 +3336,7 @@ hipError_t launch_tfsf_fix_batch(const FusedItem *items, const unsigned *map, in
 }
 
 long tfsf_fix_blocks(const StepDev &s) {
-    int nbx, span;
-    tfsf_fix_shape(s.tf, &nbx, &span);
-    return tfsf_fix_nblocks(nbx, span);
+    return tfsf_fix_nblocks(s.tf);
 }
 
 hipError_t launch_line_batch(const LineDev *items, int n, const int *dyn, int step_off, hipStream_t st) {
@@ -3560,32 +3583,24 @@ hipError_t launch_split_e(const StepDev &s, hipStream_t st) {
 }
 
 hipError_t launch_tfsf_split(const StepDev &s, hipStream_t st) {
-    const TfsfDev &t = s.tf;
-    int span = 0;
-    for (int a = 0; a < 3; a++) span = max(span, t.t1[a] - t.t0[a] + 2);
-    const int nbx = (span + 63) / 64;
-    hipLaunchKernelGGL(k_tfsf_split, dim3((unsigned)(((long)nbx * span * 9 + 3) / 4)), dim3(256), 0, st, s, nbx, span);
+    hipLaunchKernelGGL(k_tfsf_split, dim3((unsigned)tfsf_nblocks(s.tf, 3, 0)), dim3(256), 0, st, s);
     return hipGetLastError();
 }
 
 hipError_t launch_tfsf_fix(const StepDev &s, hipStream_t st) {
-    int nbx, span;
-    tfsf_fix_shape(s.tf, &nbx, &span);
-    hipLaunchKernelGGL(k_tfsf_fix, dim3((unsigned)tfsf_fix_nblocks(nbx, span)), dim3(256), 0, st, s, nbx, span);
+    hipLaunchKernelGGL(k_tfsf_fix, dim3((unsigned)tfsf_fix_nblocks(s.tf)), dim3(256), 0, st, s);
     return hipGetLastError();
 }
 
 hipError_t launch_post(const StepDev &s, bool tfsf, const DispDev *d, bool sample, hipStream_t st) {
     static_assert(sizeof(StepDev) + sizeof(DispDev) + 32 <= 4096, "kernel arguments");
-    int nbx, span;
-    tfsf_fix_shape(s.tf, &nbx, &span);
     const long nb = d ? (long)d->n[0] * d->n[1] * d->n[2] : 0;
-    const long nd = (nb + 255) / 256, nt = tfsf ? tfsf_fix_nblocks(nbx, span) : 0, ns = sample ? (s.fd.mE + 255) / 256 : 0;
+    const long nd = (nb + 255) / 256, nt = tfsf ? tfsf_fix_nblocks(s.tf) : 0, ns = sample ? (s.fd.mE + 255) / 256 : 0;
     if (nd + nt + ns > 0x7fffffff) return hipErrorInvalidValue;
     if (nd + nt + ns == 0) return hipSuccess;
     const DispDev none{};
-    hipLaunchKernelGGL(k_post, dim3((unsigned)(nd + nt + ns)), dim3(256), 0, st, s, d ? *d : none, (int)nd, nbx, span,
-                       (int)nt, (int)ns);
+    hipLaunchKernelGGL(k_post, dim3((unsigned)(nd + nt + ns)), dim3(256), 0, st, s, d ? *d : none, (int)nd, (int)nt,
+                       (int)ns);
     return hipGetLastError();
 }
 
@@ -3606,15 +3621,13 @@ hipError_t launch_hydro(const DispDev &d, const StepDev *s, bool sample, hipStre
     if (nb <= 0) return hipSuccess;
     const dim3 grid((unsigned)((nb + 255) / 256)), block(256);
     const StepDev none{};
-    int nbx = 0, span = 0;
     long nt = 0, ns = 0;
     if (s) {
-        tfsf_fix_shape(s->tf, &nbx, &span);
-        nt = tfsf_fix_nblocks(nbx, span);
+        nt = tfsf_fix_nblocks(s->tf);
         ns = sample ? (s->fd.mE + 255) / 256 : 0;
     }
     if ((long)grid.x + nt + ns > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_hydro_v_ce0, dim3((unsigned)(grid.x + nt + ns)), block, 0, st, d, (int)grid.x, s ? *s : none, nbx, span,
+    hipLaunchKernelGGL(k_hydro_v_ce0, dim3((unsigned)(grid.x + nt + ns)), block, 0, st, d, (int)grid.x, s ? *s : none,
                        (int)nt, (int)ns);
     hipLaunchKernelGGL(k_hydro_ce<1>, grid, block, 0, st, d);
     hipLaunchKernelGGL(k_hydro_ce<2>, grid, block, 0, st, d);

@@ -207,3 +207,29 @@ print(idle, time.process_time() - queued)
 """)
     idle, queued = map(float, out.split())
     assert queued - idle < 0.2, (idle, queued)
+
+
+@pytest.mark.parametrize("shape", [(24, 24, 24), (300, 22, 24), (22, 300, 24), (24, 22, 300), (140, 150, 20)])
+def test_tfsf_launches_hold_the_rows_of_the_planes(stub, tmp_path, shape):
+    """Four planes of t0 - 1 .. t1 + 1 per axis after the update (three of t0 - 1 ..
+    t1 between separate calls), in rows of 64 cells along the faster axis and
+    four rows a block, each axis by its own extents."""
+    launches, out = run(stub, tmp_path, f"""
+p = small_params(G, sphere=0)
+p.NCELLX, p.NCELLY, p.NCELLZ = {shape}
+s = G.Simulation(p)
+print(s.info.NX, s.info.NY, s.info.NZ, *s.info.tfsf)
+mark()
+s.step(2)
+s.tfsf()
+""")
+    size, t0 = [int(x) for x in out.split()[:3]], [int(x) for x in out.split()[3:6]]
+    t1 = [n - t for n, t in zip(size, t0)]
+
+    def blocks(planes, past):
+        n = [b - a + 2 + past for a, b in zip(t0, t1)]
+        rows = sum(planes * n[0 if a else 1] * -(-n[1 if a == 2 else 2] // 64) for a in range(3))
+        return -(-rows // 4)
+    posts = [g for k, g, _ in launches if k == "k_post"]
+    assert posts[1] == (blocks(4, 1), 1, 1)      # the second step takes no sample
+    assert [g for k, g, _ in launches if k == "k_tfsf_split"] == [(blocks(3, 0), 1, 1)]
