@@ -892,16 +892,11 @@ int launch_one_update(fdtd_sim *s, const StepDev &d, const LineDev &l, const Dis
 // thread, which also takes the page faults of a fresh buffer (8.5 ms for a field
 // of 281^3, 10 GB/s; the link does 56).  Here the two halves of a pinned buffer
 // of the handle take turns: the device fills one while up to eight threads move
-// the other's bytes on.  Below 1 MB the threads cost more than they save.  The
-// threads poll for the first half, so the caller lets earlier work end first and
-// leaves on the stream only what fills dev.
+// the other's bytes on.  Below kThreadedCopy the threads cost more than they save
+// (the caller copies by itself).  The threads poll for the first half, so the caller
+// lets earlier work end first and leaves on the stream only what fills dev.
 int copy_out(fdtd_sim *s, const void *dev, void *host, size_t bytes) {
-    constexpr size_t kMin = 1u << 20, kHalf = 8u << 20;
-    if (bytes < kMin) {
-        HIPCHK(s, hipStreamSynchronize(s->stream));
-        HIPCHK(s, hipMemcpy(host, dev, bytes, hipMemcpyDeviceToHost));
-        return FDTD_OK;
-    }
+    constexpr size_t kMin = kThreadedCopy, kHalf = 8u << 20;
     const size_t half = std::min(kHalf, (bytes / 2 + 4095) / 4096 * 4096);
     if (s->pinned_half < half) {
         if (s->pinned) (void)hipHostFree(s->pinned);
@@ -2096,9 +2091,13 @@ int fdtd_sync(fdtd_sim *s) {
 int fdtd_get_field(fdtd_sim *s, int comp, float *out) {
     if (!s || !out || comp < 0 || comp > 5) return FDTD_ERR_INVALID;
     const float *f = comp < 3 ? s->E[s->p][comp] : s->H[s->p][comp - 3];
-    HIPCHK(s, hipStreamSynchronize(s->stream));
+    const size_t bytes = (size_t)s->g.NX * s->g.NY * s->g.NZ * sizeof(float);
+    if (bytes >= kThreadedCopy) HIPCHK(s, hipStreamSynchronize(s->stream));
     HIPCHK(s, launch_pack_field(f, s->g, s->dense, 1, s->stream));
-    return copy_out(s, s->dense, out, (size_t)s->g.NX * s->g.NY * s->g.NZ * sizeof(float));
+    if (bytes >= kThreadedCopy) return copy_out(s, s->dense, out, bytes);
+    HIPCHK(s, hipStreamSynchronize(s->stream));
+    HIPCHK(s, hipMemcpy(out, s->dense, bytes, hipMemcpyDeviceToHost));
+    return FDTD_OK;
 }
 
 int fdtd_get_slice(fdtd_sim *s, int comp, int axis, int index, float *out) {

@@ -141,8 +141,10 @@ int fdtd_checkpoint_save(fdtd_sim *s, void *buf, size_t bytes) {
         std::memcpy(o, &n, sizeof(n));
         o += sizeof(n);
         for (auto &p : sec) {
-            if (p.n && p.dev) {
+            if (p.n >= kThreadedCopy && p.dev) {
                 if (int rc = copy_out(s, p.p, o, p.n)) return rc;
+            } else if (p.n && p.dev) {
+                HIPCHK(s, hipMemcpy(o, p.p, p.n, hipMemcpyDeviceToHost));
             } else if (p.n) {
                 std::memcpy(o, p.p, p.n);
             }

@@ -235,7 +235,9 @@ bool disp_in_clean(const fdtd_sim *s);
 bool tfsf_off_clean_edges(const fdtd_sim *s);
 // nsteps steps keeping an early start from the step before (fdtd_step clears it first)
 int step_steps(fdtd_sim *s, int nsteps);
-// Device memory to the caller's, after the work queued on the solver stream.
+// Device memory to the caller's through threads, after the work queued on the solver
+// stream; for blocks of at least kThreadedCopy bytes.
+constexpr size_t kThreadedCopy = 1u << 20;
 int copy_out(fdtd_sim *s, const void *dev, void *host, size_t bytes);
 // FDTD_ERR_NONFINITE (with a message) when a kernel has flagged a NaN or Inf.
 int check_finite(fdtd_sim *s);

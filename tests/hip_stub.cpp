@@ -31,7 +31,7 @@ size_t g_shmem;
 hipStream_t g_stream;
 hipError_t g_last = hipSuccess;
 long g_fail = -1;
-int g_queued_ms = 0;
+int g_queued_ms = 0, g_waits = 0;
 char g_handle[8];
 template <typename T>
 hipError_t handle(T *out) {
@@ -49,6 +49,7 @@ extern "C" {
 
 void stub_fail_launch(long n) { g_fail = n; }
 void stub_queue(int ms) { g_queued_ms = ms; }
+int stub_waits(void) { return g_waits; }   // stream synchronisations so far
 // Records of a point monitor or objective probe that the handle still holds for a later launch.
 int stub_pending_records(const fdtd_sim *s) { return (s->rec_dst[0] != nullptr) + (s->rec_dst[1] != nullptr); }
 
@@ -106,6 +107,7 @@ hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess;
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return handle(s); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) {
+    g_waits++;
     std::this_thread::sleep_for(std::chrono::milliseconds(std::exchange(g_queued_ms, 0)));
     return hipSuccess;
 }

@@ -233,3 +233,17 @@ s.tfsf()
     posts = [g for k, g, _ in launches if k == "k_post"]
     assert posts[1] == (blocks(4, 1), 1, 1)      # the second step takes no sample
     assert [g for k, g, _ in launches if k == "k_tfsf_split"] == [(blocks(3, 0), 1, 1)]
+
+
+def test_small_read_outs_wait_once(stub, tmp_path):
+    """Blocks below the size that threads move: one wait for a field, one for a
+    whole checkpoint of small arrays, not one each."""
+    _, out = run(stub, tmp_path, """
+s = G.Simulation(small_params(G, nfreq=1, sphere=0))
+s.set_point_monitor((5, 6, 7), 10)
+for f in (lambda: s.get_field(0), lambda: s.checkpoint()):
+    n = stub.stub_waits()
+    f()
+    print(stub.stub_waits() - n)
+""")
+    assert [int(x) for x in out.split()] == [1, 1]
