@@ -2275,7 +2275,8 @@ int fdtd_reflectance(fdtd_sim *s, double *R, double *T, double *ref_r, double *r
     if (int rc = fdtd_flux(s, nullptr, nullptr, nullptr, raw.data())) return rc;
     // the incident wave at the source plane, sampled like the monitors: the same
     // FP64 line run again for the steps so far, on the device in the staging
-    // buffer where the line fits one block's LDS and the steps the buffer
+    // buffer where the line is long enough to gain by it and fits one block's LDS,
+    // and the steps the buffer
     std::vector<std::complex<double>> inc(F, 0.0);
     const long need = line_dft_scratch(S.L, s->t, S.P.dft_stride, F);
     if (S.P.StaticField == 1 || s->t == 0) {

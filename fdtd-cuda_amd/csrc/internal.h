@@ -308,7 +308,7 @@ hipError_t launch_line(const LineDev &l, hipStream_t st);
 // DFT of n point-monitor records (three floats each, the first of step t0): 6 nf doubles to out.
 hipError_t launch_point_dft(const float *rec, int n, int t0, int nf, const double *freq, double dt, double *out, hipStream_t st);
 // DFT of e_inc[m0] over the first `steps` steps of the line (re then im, F
-// each, at *out in the scratch of line_dft_scratch doubles; -1: line too long).
+// each, at *out in the scratch of line_dft_scratch doubles; -1: the line's length is left to the host).
 long line_dft_scratch(int L, int steps, int stride, int F);
 hipError_t launch_line_dft(const LineDev &l, int m0, int steps, int stride, int F, const double *freq, double dt,
                            double *scratch, double **out, hipStream_t st);

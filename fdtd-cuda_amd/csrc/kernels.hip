@@ -2233,7 +2233,10 @@ __global__ __launch_bounds__(256) void k_line_pulses(LineDev l, int steps, doubl
     const int t = (int)(blockIdx.x * 256 + threadIdx.x);
     if (t < steps) pulse[t] = line_pulse(l, t);
 }
-constexpr int kReplayMaxLine = 4096;     // 64 KB of LDS
+// Shorter lines stay on the host: a step takes at least 0.55 us here, some 0.46 ns a
+// cell there (6000 steps, here and there: L = 522 3.3 and 1.6 ms, 1722 4.6 and 4.8,
+// 3522 6.7 and 9.9).
+constexpr int kReplayMinLine = 1600, kReplayMaxLine = 4096;   // 64 KB of LDS
 __global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int stride, int m0, const double *pulse, double *hist) {
     extern __shared__ double lds[];
     const int L = l.L, tid = threadIdx.x, nt = blockDim.x;
@@ -3720,7 +3723,7 @@ hipError_t launch_slice(const float *f, const Geom &g, int axis, int index, floa
 }
 
 long line_dft_scratch(int L, int steps, int stride, int F) {
-    if (L > kReplayMaxLine || L < 4) return -1;
+    if (L > kReplayMaxLine || L < kReplayMinLine) return -1;
     return (long)steps + (steps + stride - 1) / stride + 2L * F;
 }
 

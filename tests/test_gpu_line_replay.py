@@ -2,9 +2,10 @@
 1D line off its usual cell: beside the source plane, next to either end and on
 the last cell.  R and the reference's column share the flux through the
 reflection plane, so their quotient is the incident power over the source's: the
-line alone (run again on the device: the steps fit the staging buffer of this
-grid), FP64 recurrences of 900 steps on both sides (some 1e-13 of each
-other per rounding; 1e-9 of the oracle's value allowed)."""
+line alone, FP64 recurrences of up to 3900 steps on both sides (some 1e-13 of each
+other per rounding; 1e-9 of the oracle's value allowed).  The line has 6 NCELLZ
+cells: 240 are replayed on the host, 1602 (the shortest) and 1800 on the device,
+whose staging buffer the steps fit here."""
 import numpy as np
 import pytest
 
@@ -15,13 +16,14 @@ from conftest import small_params
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("nz,steps", [(40, 900), (267, 3600), (300, 3900)])
 @pytest.mark.parametrize("src", ["m0 - 1", "1", "2", "L - 3", "L - 2", "L - 1"])
-def test_incident_power_with_the_source_anywhere_on_the_line(src):
+def test_incident_power_with_the_source_anywhere_on_the_line(src, nz, steps):
     def params(mod):
         p = small_params(mod, sphere=0, nfreq=4)
         p.periodic_xy, p.NcpmlX, p.NcpmlY, p.NcpmlZ = 1, 0, 0, 8
-        p.NCELLX, p.NCELLY, p.NCELLZ = 12, 9, 40
-        p.tfsf_inset, p.Tend, p.inc_phi = 10, 900, 90.0
+        p.NCELLX, p.NCELLY, p.NCELLZ = 12, 9, nz
+        p.tfsf_inset, p.Tend, p.inc_phi = 10, steps, 90.0
         line = 6 * p.NCELLZ
         p.source_offset = line // 2 - eval(src, {"L": line, "m0": line // 2})
         return p
@@ -30,7 +32,7 @@ def test_incident_power_with_the_source_anywhere_on_the_line(src):
     power = []
     for x in (s, o):
         x.add_layer(k0, k0 + 3)
-        x.step(900)
+        x.step(steps)
         r = x.reflectance()
         power.append(r["ref_r"] / r["R"])
     print(src, *power, flush=True)
