@@ -61,7 +61,7 @@ struct fdtd_batch {
     // every simulation's whole field update in one launch per step (k_step_batch),
     // on one stream, with x chunk one_chunk; else the launches per variant below
     bool one = false;
-    int one_chunk = 1;
+    int one_chunk = 1, two_waves = 12;      // two_waves: waves per block of columns of 2
     DispDev *disp[2] = {};
     SampleItem *samp[2] = {};
     int *dyn = nullptr;                     // {t of the next step, ring row of the next sample}
@@ -335,8 +335,30 @@ void add_blocks(Launch &l, int sim, long n) {
 // and 10 leave every compute unit two of its waves short), us per step: 4 grids of
 // 221 x 221 x 270 844, 807 and 794, 3 of 261^3 867, 830 and 809, 4 of 61 x 61 x
 // 260 130, 124 and 128.
-int one_waves(int W) { return W == 5 ? 15 : (W <= 6 ? 12 : W); }
-int one_tiles(int W) { return one_waves(W) / W; }
+// two: of columns of 2 waves, 12 or 4 (short_columns).
+int one_waves(int W, int two) { return W == 2 ? two : (W == 5 ? 15 : (W <= 6 ? 12 : W)); }
+int one_tiles(int W, int two) { return one_waves(W, two) / W; }
+
+// Columns of 2 waves in blocks of 4 (three a compute unit) where they are most of a
+// batch: the pieces of a small grid fill a block of six row tiles badly.  In blocks
+// of 12 they share a launch with the other heights, which a batch that does not
+// fill the device, or is mostly of those, needs more.  us per step, 12 against 4 and
+// the launches per variant: 64 grids of 45^3 364, 258 and 260, 16 of 45^3 114, 90 and
+// 114, 64 of 61^3 555, 451 and 508, 32 of 85^3 557, 505 and 587; with 8 of 45 x 45 x
+// 150 among 64 of 45^3 436, 364 and 395; two of 45^3 and one of 45 x 45 x 150 46 and 75.
+int short_columns(const std::vector<fdtd_sim *> &sims, bool *only) {
+    long two = 0, all = 0, blocks = 0;
+    for (fdtd_sim *s : sims) {
+        const int W = rows_waves(s->g.NZ);
+        const long w = (long)s->g.NX * ((s->g.NY + 1) / 2) * W;
+        all += w;
+        if (W != 2) continue;
+        two += w;
+        blocks += (long)((s->g.NY + 3) / 4) * ((s->g.NX + 7) / 8);
+    }
+    *only = two == all;
+    return *only || (2 * two > all && blocks >= 3 * 256) ? 4 : 12;
+}
 
 // Uploads every per-simulation argument for both parities and rebuilds the
 // launch list; a changed list invalidates the captured graph.
@@ -360,10 +382,10 @@ int upload_items(fdtd_batch *b) {
             }
             li[i] = at_parity(s, par, [&] { return make_line(s); });
             if (b->one) {
-                ai[i] = at_parity(s, par, [&] { return make_step_all(s, li[i], one_tiles(rows_waves(s->g.NZ)), b->one_chunk); });
+                ai[i] = at_parity(s, par, [&] { return make_step_all(s, li[i], one_tiles(rows_waves(s->g.NZ), b->two_waves), b->one_chunk); });
                 const long nb = step_all_blocks(ai[i]);
                 if (nb < 0 || nb >= (1L << kBatchLocalBits)) return berr(b, FDTD_ERR_UNSUPPORTED, "batch: grid too large for the block map");
-                if (par == 0) add_blocks(group(ls, Launch::All, one_waves(rows_waves(s->g.NZ)), 0, 0), i, nb);
+                if (par == 0) add_blocks(group(ls, Launch::All, one_waves(rows_waves(s->g.NZ), b->two_waves), 0, 0), i, nb);
             }
             const int q = at_parity(s, par, [&] { return s->p; });
             di[i] = make_disp(s, 1 - q);
@@ -703,18 +725,20 @@ int fdtd_batch_create(fdtd_sim *const *sims, int n, int flags, fdtd_batch **out)
     if ((rc = balloc(b, &b->dyn, 2))) return fail(rc);
     if (b->one) {
         // one chunk for the batch, by the rule of the single step over all its columns
-        // (block rows times planes; blocks of 12 waves leave one resident per CU)
+        // (block rows times planes; one block of 12 waves resident per CU, or three of 4)
         if ((rc = balloc(b, &b->all[0], n)) || (rc = balloc(b, &b->all[1], n))) return fail(rc);
         long columns = 0;
         int NX = 1;
+        bool only = false;
+        b->two_waves = short_columns(b->sims, &only);
         for (fdtd_sim *s : b->sims) NX = std::max(NX, s->g.NX);
         for (fdtd_sim *s : b->sims) {
-            const int t = one_tiles(rows_waves(s->g.NZ));
+            const int t = one_tiles(rows_waves(s->g.NZ), b->two_waves);
             columns += (long)((s->g.NY + 2 * t - 1) / (2 * t)) * s->g.NX;
         }
         // at most 8 planes: us per step of 12 rods with chunks 4, 8, 12, 16, 24: 1129, 1054, 1070,
         // 1075, 1070 (of 4 rods 378, 351, 358, 358, 360)
-        b->one_chunk = march_chunk((columns + NX - 1) / NX, NX, 256, 8);
+        b->one_chunk = march_chunk((columns + NX - 1) / NX, NX, only ? 3 * 256 : 256, 8);
     }
     b->rowpath.assign(n, 0);
     b->ta.assign(n, 8);

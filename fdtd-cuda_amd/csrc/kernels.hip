@@ -2361,7 +2361,8 @@ __global__ __launch_bounds__(64 * MW) void k_step_all(StepAll) {
 // each simulation its line).  Grids of 2, 3, 4 and 6 waves a column share the
 // launch in blocks of 12 waves (6, 4, 3 and 2 row tiles): one launch for the
 // whole batch leaves one tail a step, and the taller blocks read fewer halo
-// rows.  Other columns have a launch of their own (5 waves: three tiles).  us per step of 4, 12 and 32 rods (17, 56 and 147 M cells): 343, 973
+// rows.  Other columns have a launch of their own (5 waves: three tiles), and those of
+// 2 in blocks of 4 where they are most of a batch.  us per step of 4, 12 and 32 rods (17, 56 and 147 M cells): 343, 973
 // and 2556 (351, 1054 and 2671 with the march unrolled, on a slower card), with a
 // launch per variant and column height on two streams 413, 1162 and 2910.  The
 // launch is bound by memory (889 of the 960 us a step at 12 rods in a trace).

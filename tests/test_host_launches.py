@@ -88,12 +88,13 @@ for n in range(1, 40):
     assert rows[0][2] == 0 and rows[-2][2] == 1, rows   # the last launch of all is the record's own
 
 
-@pytest.mark.parametrize("nz,kernel,waves", [(24, "k_step_batch<12>", 12), (200, "k_step_batch<12>", 12), (270, "k_step_batch<16>", 15),
+@pytest.mark.parametrize("nz,kernel,waves", [(24, "k_step_batch<12>", 4), (200, "k_step_batch<12>", 12), (270, "k_step_batch<16>", 15),
                                              (330, "k_step_batch<12>", 12), (400, "k_step_batch<16>", 8),
                                              (600, "k_step_batch<12>", 12), (800, "k_step_batch<16>", 16)])
 def test_batch_blocks_fill_a_compute_unit(stub, tmp_path, nz, kernel, waves):
     """Blocks of the batched one-launch step by column height: 5 waves a column
-    in blocks of 15, and the instance by the waves that fit a compute unit."""
+    in blocks of 15, 2 (alone in their batch) in blocks of 4, and the instance by
+    the waves that fit a compute unit."""
     launches, _ = run(stub, tmp_path, f"""
 p = small_params(G, sphere=0)
 p.NCELLZ = {nz}
@@ -262,3 +263,22 @@ mark()
 s.reflectance()
 """)
     assert any(k == "k_line_replay" for k, _, _ in launches) == device
+
+
+@pytest.mark.parametrize("sizes,waves", [([(1, 24), (1, 150)], [12]), ([(1, 24), (1, 300)], [12, 15]), ([(48, 24), (1, 150)], [4, 12]),
+                                         ([(48, 24), (34, 150)], [12]), ([(3, 24)], [4]), ([(2, 24), (2, 101)], [4])])
+def test_batch_of_short_columns_takes_small_blocks(stub, tmp_path, sizes, waves):
+    """Columns of 2 waves in blocks of 4 where they are the whole batch, or most of
+    one that fills the device; else in the blocks of 12 of the other heights."""
+    launches, _ = run(stub, tmp_path, f"""
+s = []
+for n, nz in {sizes}:
+    for _ in range(n):
+        p = small_params(G, sphere=0, nfreq=1)
+        p.NCELLZ = nz
+        s.append(G.Simulation(p))
+b = G.Batch(s, flags=G.BATCH_NO_GRAPH)
+mark()
+b.run(1)
+""")
+    assert sorted(b[1] for k, _, b in launches if k.startswith("k_step_batch")) == waves, launches
