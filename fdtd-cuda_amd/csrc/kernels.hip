@@ -2233,10 +2233,11 @@ __global__ __launch_bounds__(256) void k_line_pulses(LineDev l, int steps, doubl
     const int t = (int)(blockIdx.x * 256 + threadIdx.x);
     if (t < steps) pulse[t] = line_pulse(l, t);
 }
-// Shorter lines stay on the host: a step takes at least 0.55 us here, some 0.46 ns a
-// cell there (6000 steps, here and there: L = 522 3.3 and 1.6 ms, 1722 4.6 and 4.8,
-// 3522 6.7 and 9.9).
-constexpr int kReplayMinLine = 1600, kReplayMaxLine = 4096;   // 64 KB of LDS
+// Shorter lines stay on the host: a step takes at least 0.55 us here, 0.4 to 0.6 ns a
+// cell there by the host's load (3000 steps, here and there: L = 522 1.71 and 0.93 ms,
+// 882 1.80 and 1.37 to 1.69, 1200 1.95 and 1.79 on one machine, 9 % more on another,
+// 1722 2.35 and 2.36).
+constexpr int kReplayMinLine = 800, kReplayMaxLine = 4096;   // 64 KB of LDS
 __global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int stride, int m0, const double *pulse, double *hist) {
     extern __shared__ double lds[];
     const int L = l.L, tid = threadIdx.x, nt = blockDim.x;

@@ -93,7 +93,9 @@ double source_pulse(const Setup &s, int t) {
     return s.P.MAX_AMP * std::exp(-(double)b2 / 2.0) * std::sin(2 * kPI * s.f0 * t * s.dt);
 }
 
-std::vector<std::complex<double>> line_dft(const Setup &s, int steps) {
+// O3 for the vector instructions (the same bits; 6000 steps of 522 cells 2.9 -> 1.6 ms).
+// Not for the whole file: the set-up of a 125 x 173 x 204 grid takes 12 % longer with it.
+__attribute__((optimize("O3"))) std::vector<std::complex<double>> line_dft(const Setup &s, int steps) {
     // the 1D line of k_line (UPDATE_h_inc, UPDATE_e_inc, Mur ends, additive
     // source: main.cu:2280-2337, 2831-2859) in FP64, and the DFT of e_inc[m0]
     // after every sampling step t (t % dft_stride == 0) with phase (t+1) dt
