@@ -2238,6 +2238,8 @@ __global__ __launch_bounds__(256) void k_line_pulses(LineDev l, int steps, doubl
 // 882 1.80 and 1.37 to 1.69, 1200 1.95 and 1.79 on one machine, 9 % more on another,
 // 1722 2.35 and 2.36).
 constexpr int kReplayMinLine = 800, kReplayMaxLine = 4096;   // 64 KB of LDS
+// END: the source stands on the last cell (a test in the loop is 2 % of a step).
+template <bool END>
 __global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int stride, int m0, const double *pulse, double *hist) {
     extern __shared__ double lds[];
     const int L = l.L, tid = threadIdx.x, nt = blockDim.x;
@@ -2262,7 +2264,7 @@ __global__ __launch_bounds__(1024) void k_line_replay(LineDev l, int steps, int 
         if (tid < 2) {
             const double en = ei - l.ce * (h[in] - h[in - 1]);
             double v = mur + l.mur_coef * (en - eo);
-            if (end == l.src) v += p;
+            if (END && tid == 1) v += p;
             e[end] = v;
             mur = en;
         }
@@ -3736,7 +3738,8 @@ hipError_t launch_line_dft(const LineDev &l, int m0, int steps, int stride, int 
     double *pulse = scratch, *hist = pulse + steps, *o = hist + n;
     const int nt = min(1024, ((l.L + 1) / 2 + 63) / 64 * 64);
     hipLaunchKernelGGL(k_line_pulses, dim3((steps + 255) / 256), dim3(256), 0, st, l, steps, pulse);
-    hipLaunchKernelGGL(k_line_replay, dim3(1), dim3(nt), 2 * l.L * sizeof(double), st, l, steps, stride, m0, pulse, hist);
+    const auto replay = l.src == l.L - 1 ? k_line_replay<true> : k_line_replay<false>;
+    hipLaunchKernelGGL(replay, dim3(1), dim3(nt), 2 * l.L * sizeof(double), st, l, steps, stride, m0, pulse, hist);
     hipLaunchKernelGGL(k_line_dft, dim3(F), dim3(256), 0, st, hist, n, stride, freq, dt, F, o);
     *out = o;
     return hipGetLastError();
